@@ -22,8 +22,9 @@
 //   adj_gather  one thread per control point (k1, k2, k3, c): sums the
 //               partial windows of the few workgroups whose windows hold
 //               (k1, k2, k3).
-// General path (any Nin, any degree, any sample order): adj_csr, one thread
-// per control point, walking each dimension's transposed band list.
+// General path (any Nin, any degree, any sample order): adj_csr, a thread,
+// wave or workgroup per control point, walking each dimension's transposed
+// band list.
 #include "sg_plan_host.hpp"
 
 namespace sg {
@@ -368,53 +369,102 @@ struct AdjCsrArgs {
   int accumulate;
 };
 
-template <typename T>
-__global__ __launch_bounds__(256) void adj_csr(AdjCsrArgs<T> a) {
-  const long long idx = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= a.ncp * a.nout) return;
-  const int c = static_cast<int>(idx / a.ncp);
-  long long r = idx - static_cast<long long>(c) * a.ncp;
-  int lo[SG_MAX_NIN], hi[SG_MAX_NIN], e[SG_MAX_NIN];
-  bool empty = false;
-#pragma unroll
-  for (int d = 0; d < SG_MAX_NIN; ++d) {
-    if (d < a.nin) {
-      const int k = static_cast<int>(r % a.n[d]);
-      r /= a.n[d];
-      lo[d] = a.ptr[d][k];
-      hi[d] = a.ptr[d][k + 1];
-      e[d] = lo[d];
-      empty |= lo[d] >= hi[d];
-    }
-  }
+// The general adjoint: G threads per control point (and channel) walk the
+// product of its per-dimension band lists, thread t the entries t, t + G, ...
+// in the lists' mixed-radix order, and add their sums in a fixed tree, so
+// every result is the same sum in the same order on every run.  Each entry
+// is two dependent loads (the list, then the table and ebar), so a lone
+// thread per control point waits through its whole list: G spreads it over
+// a wave or a workgroup (see csr_threads for the choice).  NIN1: curves, the
+// list of dimension 1 alone, kCsrBatch entries in flight per thread.
+constexpr int kCsrBatch = 4;
+constexpr int kCsrBlock = 1024;  // the widest G: one workgroup per control point
+
+template <typename T, int G, bool NIN1>
+__global__ __launch_bounds__(G > 256 ? G : 256) void adj_csr(AdjCsrArgs<T> a) {
+  constexpr int B = G > 256 ? G : 256;
+  const long long idx = (static_cast<long long>(blockIdx.x) * B + threadIdx.x) / G;
+  const int sub = static_cast<int>(threadIdx.x % G);
+  const bool live = idx < a.ncp * a.nout;
   T sum = T(0);
-  if (!empty) {
+  if (live) {
+    const int c = static_cast<int>(idx / a.ncp);
+    long long r = idx - static_cast<long long>(c) * a.ncp;
     const T* E = a.E + a.nsamp * c;
-    while (true) {
-      T prod = T(1);
-      long long lin = 0;
+    if constexpr (NIN1) {
+      const int e1 = a.ptr[0][r + 1];
+      const int32_t* js = a.js[0];
+      for (int e0 = a.ptr[0][r] + sub; e0 < e1; e0 += kCsrBatch * G) {
+        int at[kCsrBatch];
+        T b[kCsrBatch], v[kCsrBatch];
 #pragma unroll
-      for (int d = 0; d < SG_MAX_NIN; ++d)
-        if (d < a.nin) {
-          const int js = a.js[d][e[d]];
-          prod *= a.tab[d][js];
-          lin += static_cast<long long>(js / a.w[d]) * a.sst[d];
+        for (int u = 0; u < kCsrBatch; ++u) at[u] = js[min(e0 + u * G, e1 - 1)];
+#pragma unroll
+        for (int u = 0; u < kCsrBatch; ++u) {
+          b[u] = a.tab[0][at[u]];
+          v[u] = E[at[u] / a.w[0]];
         }
-      sum += prod * E[lin];
-      bool carry = true;
+#pragma unroll
+        for (int u = 0; u < kCsrBatch; ++u)
+          if (e0 + u * G < e1) sum += b[u] * v[u];
+      }
+    } else {
+      // digits of the thread's next entry and of the step G in the radices
+      // len_d; entries left for this thread
+      int lo[SG_MAX_NIN], len[SG_MAX_NIN], e[SG_MAX_NIN], st[SG_MAX_NIN];
+      long long total = 1, qt = sub, qg = G;
 #pragma unroll
       for (int d = 0; d < SG_MAX_NIN; ++d) {
-        if (carry && d < a.nin) {
-          if (++e[d] < hi[d])
-            carry = false;
-          else
-            e[d] = lo[d];
+        if (d < a.nin) {
+          const int k = static_cast<int>(r % a.n[d]);
+          r /= a.n[d];
+          lo[d] = a.ptr[d][k];
+          len[d] = a.ptr[d][k + 1] - lo[d];
+          total *= len[d];
+          if (len[d] > 0) {
+            e[d] = static_cast<int>(qt % len[d]);
+            st[d] = static_cast<int>(qg % len[d]);
+            qt /= len[d];
+            qg /= len[d];
+          }
         }
       }
-      if (carry) break;
+      for (long long left = total > sub ? (total - 1 - sub) / G + 1 : 0; left > 0; --left) {
+        T prod = T(1);
+        long long lin = 0;
+#pragma unroll
+        for (int d = 0; d < SG_MAX_NIN; ++d)
+          if (d < a.nin) {
+            const int js = a.js[d][lo[d] + e[d]];
+            prod *= a.tab[d][js];
+            lin += static_cast<long long>(js / a.w[d]) * a.sst[d];
+          }
+        sum += prod * E[lin];
+        int carry = 0;
+#pragma unroll
+        for (int d = 0; d < SG_MAX_NIN; ++d) {
+          if (d < a.nin) {
+            e[d] += st[d] + carry;
+            carry = e[d] >= len[d] ? 1 : 0;
+            e[d] -= carry ? len[d] : 0;
+          }
+        }
+      }
     }
   }
-  a.out[idx] = a.accumulate ? a.out[idx] + sum : sum;
+  if constexpr (G > 1) {
+#pragma unroll
+    for (int m = (G < kLanes ? G : kLanes) / 2; m >= 1; m /= 2) sum += __shfl_xor(sum, m);
+  }
+  if constexpr (G > kLanes) {  // one control point per workgroup
+    __shared__ T part[G / kLanes];
+    if (threadIdx.x % kLanes == 0) part[threadIdx.x / kLanes] = sum;
+    __syncthreads();
+    sum = part[0];
+#pragma unroll
+    for (int w = 1; w < G / kLanes; ++w) sum += part[w];
+  }
+  if (live && sub == 0) a.out[idx] = a.accumulate ? a.out[idx] + sum : sum;
 }
 
 template <typename T>
@@ -549,6 +599,20 @@ hipError_t gather(const Plan& pl, const Tiling& tl, const T* part, T* Pbar, int 
   return hipGetLastError();
 }
 
+// Threads per control point of adj_csr, from the mean entries of a list and
+// the outputs (control points times channels).  Short lists keep one thread
+// (20 000 control points x 3 of 40 entries: 15 us, a wave each 20 us).  A
+// wave otherwise (1 600 outputs of 150 entries: 31 -> 14 us; 131 072 of 410:
+// 562 -> 320 us), and a workgroup where the lists are long, sooner when the
+// outputs alone leave CUs empty (20 outputs of 8 000: a thread 1 167 us, a
+// wave 25 us, a workgroup 16 us; 1 296 of 1 296: 6 065 / 91 / 33 us; but
+// 3 200 of 1 600: 1 320 / 30 / 54 us).
+int csr_threads(long long outputs, double entries) {
+  if (entries <= 48.0) return 1;
+  if (entries > 64.0 * kLanes || (entries > 16.0 * kLanes && outputs <= 2048)) return kCsrBlock;
+  return kLanes;
+}
+
 template <typename T>
 hipError_t adjoint_csr(const Plan& pl, const int32_t* orders, const T* E,
                        T* Pbar, int accumulate, hipStream_t s) {
@@ -572,8 +636,20 @@ hipError_t adjoint_csr(const Plan& pl, const int32_t* orders, const T* E,
     a.nsamp *= dd.m;
   }
   const long long total = a.ncp * pl.nout;
-  hipLaunchKernelGGL(adj_csr<T>, dim3(static_cast<unsigned>((total + 255) / 256)),
-                     dim3(256), 0, s, a);
+  // mean list entries per control point, before the threads are chosen
+  const double entries = [&] {
+    double len = 1.0;
+    for (const DimDev& dd : pl.dims) len *= static_cast<double>(dd.m) * (dd.p + 1) / dd.n;
+    return len;
+  }();
+  const int g = csr_threads(total, entries);
+  const int block = std::max(g, 256);
+  const bool one = pl.nin == 1;
+  void (*k)(AdjCsrArgs<T>) = g == kCsrBlock ? (one ? adj_csr<T, kCsrBlock, true> : adj_csr<T, kCsrBlock, false>)
+                             : g == kLanes  ? (one ? adj_csr<T, kLanes, true> : adj_csr<T, kLanes, false>)
+                                            : (one ? adj_csr<T, 1, true> : adj_csr<T, 1, false>);
+  hipLaunchKernelGGL(k, dim3(static_cast<unsigned>((total * g + block - 1) / block)), dim3(block),
+                     0, s, a);
   return hipGetLastError();
 }
 
