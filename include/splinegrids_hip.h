@@ -173,7 +173,8 @@ int sg_evaluate_rational_fields(sg_plan* plan, int32_t n_fields,
  * w(x))]_k.  No counterpart in the reference, whose evaluate_adjoint! rejects
  * NURBS (src/adjoint.jl:57; sg_evaluate_adjoint keeps that behaviour).
  * accumulate as in sg_evaluate_adjoint.  workspace: device memory of
- * sg_rational_adjoint_workspace_bytes bytes; the call allocates nothing. */
+ * sg_rational_adjoint_workspace_bytes bytes (NULL where that is 0); the call
+ * allocates nothing. */
 int sg_rational_adjoint_workspace_bytes(const sg_plan* plan, int32_t dtype, int64_t* bytes);
 int sg_evaluate_rational_adjoint(sg_plan* plan, const void* weights, const void* eval,
                                  void* control_points, void* workspace,

@@ -19,9 +19,11 @@
 //     C  the (k1, k2) slab is added, weighted by B3[j3, a], into a ring of
 //        p3+1 k3-slabs in LDS; a k3 that leaves the band of the next j3 is
 //        final for this workgroup and is written to its partial window.
-//   adj_gather  one thread per control point (k1, k2, k3, c): sums the
+//   adj_gather  one or four lanes per control point (k1, k2, k3, c): sums the
 //               partial windows of the few workgroups whose windows hold
 //               (k1, k2, k3).
+// It takes the grids whose bands do not fit the matrix-core adjoint's windows
+// (sg_adjoint_mma.hip), whose partial windows go through the same gather.
 // General path (any Nin, any degree, any sample order): adj_csr, a thread,
 // wave or workgroup per control point, walking each dimension's transposed
 // band list.
@@ -290,68 +292,80 @@ template <typename T>
 struct AdjGatherArgs {
   const T* part;
   T* out;
-  // per dimension d and control point k: the windows that hold k, as
-  // offsets [ptr[k], ptr[k+1]) whose sum over the dimensions (plus the
-  // channel's) is the element offset in part
-  const int32_t* ptr1;
-  const long long* off1;
-  const int32_t* ptr2;
-  const long long* off2;
-  const int32_t* ptr3;
-  const long long* off3;
-  int n1, n2, nout;
+  const T* W;  // NURBS adjoint: weight of each control point (or null)
+  const long long* lists[3];  // gather_table of each dimension
+  int n1, n2, n3;
+  int blocks;  // workgroups per (k3, channel) plane of control points
+  int fast;    // no point is held by 2^20 windows or more
   int accumulate;
-  int fast;  // udiv_fast is exact for every window number of this plan
   long long ncp, chan;
 };
 
-// Lanes per control point in adj_gather: lane `sub` of a group sums the
-// windows sub, sub + kGatherLanes, ... (kBatch loads in flight), then the
-// group adds its partial sums with a fixed butterfly, so every result is
-// the same sum in the same order on every run.
-constexpr int kGatherLanes = 4;
+// LANES lanes per control point: lane `sub` sums the windows sub, sub +
+// LANES, ... (kGatherBatch loads in flight), then the group adds its partial
+// sums with a fixed butterfly, so every result is the same sum in the same
+// order on every run.  A workgroup lies in one (k3, channel) plane.
+//
+// Bound: latency -- a table row per dimension, then the windows.  One lane
+// per control point where the points alone fill the chip (64 x 64 x 32 points
+// x 3: 18 us with four lanes, 10 with one) or have few windows; four lanes
+// below kGatherFill points (20^3 x 3 points of up to 75 windows: 14 us with
+// one lane, 7 with four; 40 x 40 x 20 x 3: 6.3 and 6.7 us).
+constexpr int kGatherBatch = 4;
+constexpr long long kGatherFill = 1 << 16;
 
-template <typename T>
+template <typename T, int LANES>
 __global__ __launch_bounds__(256) void adj_gather(AdjGatherArgs<T> a) {
-  const long long gidx = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  const long long idx = gidx / kGatherLanes;
-  const int sub = static_cast<int>(gidx % kGatherLanes);
-  const bool live = idx < a.ncp * a.nout;
-  const long long cidx = live ? idx : 0;  // dead lanes join the butterfly
-  const int c = static_cast<int>(cidx / a.ncp);
-  long long r = cidx - static_cast<long long>(c) * a.ncp;
-  const int k1 = static_cast<int>(r % a.n1);
-  r /= a.n1;
-  const int k2 = static_cast<int>(r % a.n2);
-  const int k3 = static_cast<int>(r / a.n2);
-  const int e1a = a.ptr1[k1], n1e = a.ptr1[k1 + 1] - e1a;
-  const int e2a = a.ptr2[k2], n2e = a.ptr2[k2 + 1] - e2a;
-  const int e3a = a.ptr3[k3], n3e = a.ptr3[k3 + 1] - e3a;
-  // the n1e * n2e * n3e windows that hold (k1, k2, k3), dimension 1 fastest:
-  // window f is (i1, i2, i3) with f = i1 + n1e (i2 + n2e i3), split with
-  // udiv_fast where the plan's counts keep it exact (a.fast, uniform)
-  const int n12 = n1e * n2e;
-  const unsigned r1 = udiv_rcp(static_cast<unsigned>(n1e)), r12 = udiv_rcp(static_cast<unsigned>(n12));
-  const long long base = static_cast<long long>(c) * a.chan;
-  constexpr int kBatch = 4;
-  const int total = live ? n12 * n3e : 0;
+  const int plane = static_cast<int>(blockIdx.x) / a.blocks;
+  const int c = plane / a.n3, k3 = plane - c * a.n3;
+  const int t = (static_cast<int>(blockIdx.x) - plane * a.blocks) * 256 + static_cast<int>(threadIdx.x);
+  const int n12 = a.n1 * a.n2, sub = t % LANES;
+  const bool live = t / LANES < n12;
+  const int k12 = min(t / LANES, n12 - 1);  // dead lanes join the butterfly
+  const int k2 = k12 / a.n1, k1 = k12 - k2 * a.n1;
+  // each dimension's windows that hold the point: their number, and their
+  // parts of the element offset in `part` (which add up with the channel's)
+  const auto list = [&](int d, int k, int& count) {
+    const long long* row = a.lists[d] + static_cast<long long>(k) * kGatherRow;
+    count = static_cast<int>(row[0]);
+    return count <= kGatherRow - 2 ? row + 2 : a.lists[d] + row[1];
+  };
+  int c1, c2, c3;
+  const long long* l1 = list(0, k1, c1);
+  const long long* l2 = list(1, k2, c2);
+  const long long* l3 = list(2, k3, c3);
+  // window f = i1 + c1 (i2 + c2 i3)
+  const int total = c1 * c2 * c3;
+  // f / c for f < 2^20: (f + 1/2) / c is at least 1 / (2 c) from an integer,
+  // and its rounding error below f / c 2^-22
+  const float r1 = __builtin_amdgcn_rcpf(static_cast<float>(c1));
+  const float r2 = __builtin_amdgcn_rcpf(static_cast<float>(c2));
+  const auto quotient = [&](int n, int by, float rcp) {
+    return a.fast ? static_cast<int>((static_cast<float>(n) + 0.5f) * rcp) : n / by;
+  };
+  const T* part = a.part + static_cast<long long>(c) * a.chan;
   T sum = T(0);
-  for (int f0 = sub; f0 < total; f0 += kBatch * kGatherLanes) {
-    T v[kBatch];
+  for (int f0 = sub; f0 < total; f0 += kGatherBatch * LANES) {
+    T v[kGatherBatch];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int f = min(f0 + u * kGatherLanes, total - 1);
-      const int i3 = a.fast ? udiv_fast(f, n12, r12) : f / n12, f12 = f - i3 * n12;
-      const int i2 = a.fast ? udiv_fast(f12, n1e, r1) : f12 / n1e, i1 = f12 - i2 * n1e;
-      v[u] = a.part[base + a.off1[e1a + i1] + a.off2[e2a + i2] + a.off3[e3a + i3]];
+    for (int u = 0; u < kGatherBatch; ++u) {
+      const int f = min(f0 + u * LANES, total - 1);
+      const int f1 = quotient(f, c1, r1), i1 = f - f1 * c1;
+      const int i3 = quotient(f1, c2, r2), i2 = f1 - i3 * c2;
+      v[u] = part[l1[i1] + l2[i2] + l3[i3]];
     }
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u)
-      if (f0 + u * kGatherLanes < total) sum += v[u];
+    for (int u = 0; u < kGatherBatch; ++u)
+      if (f0 + u * LANES < total) sum += v[u];
   }
 #pragma unroll
-  for (int m = kGatherLanes / 2; m >= 1; m /= 2) sum += __shfl_xor(sum, m, kGatherLanes);
-  if (live && sub == 0) a.out[idx] = a.accumulate ? a.out[idx] + sum : sum;
+  for (int m = LANES / 2; m >= 1; m /= 2) sum += __shfl_xor(sum, m);
+  if (live && sub == 0) {
+    const long long k = k12 + static_cast<long long>(n12) * k3;
+    if (a.W) sum *= a.W[k];
+    T* dst = a.out + static_cast<long long>(c) * a.ncp + k;
+    *dst = a.accumulate ? *dst + sum : sum;
+  }
 }
 
 template <typename T>
@@ -575,27 +589,26 @@ hipError_t adjoint_stream(const Plan& pl, const int32_t* orders, const T* E,
 
 template <typename T>
 hipError_t gather(const Plan& pl, const Tiling& tl, const T* part, T* Pbar, int accumulate,
-                  hipStream_t s) {
+                  hipStream_t s, const T* W) {
   AdjGatherArgs<T> g{};
   g.part = part;
   g.out = Pbar;
-  g.ptr1 = tl.gptr[0];
-  g.off1 = tl.goff[0];
-  g.ptr2 = tl.gptr[1];
-  g.off2 = tl.goff[1];
-  g.ptr3 = tl.gptr[2];
-  g.off3 = tl.goff[2];
+  g.W = W;
+  for (int d = 0; d < 3; ++d) g.lists[d] = tl.glist[d];
   g.n1 = pl.dims[0].n;
   g.n2 = pl.dims[1].n;
-  g.nout = pl.nout;
+  g.n3 = pl.nin == 3 ? pl.dims[2].n : 1;
   g.chan = tl.gchan;
-  g.fast = tl.gfast;
   g.accumulate = accumulate;
-  g.ncp = 1;
-  for (int d = 0; d < pl.nin; ++d) g.ncp *= pl.dims[d].n;
-  const long long total = g.ncp * pl.nout * kGatherLanes;
-  hipLaunchKernelGGL(adj_gather<T>, dim3(static_cast<unsigned>((total + 255) / 256)),
-                     dim3(256), 0, s, g);
+  g.fast = tl.gwindows < (1 << 20);
+  const long long n12 = static_cast<long long>(g.n1) * g.n2;
+  g.ncp = n12 * g.n3;
+  const long long planes = static_cast<long long>(g.n3) * pl.nout;
+  const bool wide = tl.gwindows > kGatherBatch && g.ncp * pl.nout <= kGatherFill;
+  const int lanes = wide ? 4 : 1;
+  g.blocks = static_cast<int>((n12 * lanes + 255) / 256);
+  hipLaunchKernelGGL((wide ? adj_gather<T, 4> : adj_gather<T, 1>),
+                     dim3(static_cast<unsigned>(planes * g.blocks)), dim3(256), 0, s, g);
   return hipGetLastError();
 }
 
@@ -656,12 +669,12 @@ hipError_t adjoint_csr(const Plan& pl, const int32_t* orders, const T* E,
 }  // namespace
 
 hipError_t launch_adjoint_gather(const Plan& pl, const Tiling& tl, const void* part, void* Pbar,
-                                 int dtype, int accumulate, hipStream_t s) {
+                                 int dtype, int accumulate, hipStream_t s, const void* W) {
   if (dtype == SG_F32)
     return gather<float>(pl, tl, static_cast<const float*>(part), static_cast<float*>(Pbar),
-                         accumulate, s);
+                         accumulate, s, static_cast<const float*>(W));
   return gather<double>(pl, tl, static_cast<const double*>(part), static_cast<double*>(Pbar),
-                        accumulate, s);
+                        accumulate, s, static_cast<const double*>(W));
 }
 
 size_t adjoint_work_bytes(const Plan& pl) {
@@ -680,13 +693,14 @@ hipError_t launch_adjoint(const Plan& pl, const int32_t* orders,
     nsamp *= d.m;
   }
   if (ncp == 0) return hipSuccess;
+  if (pl.adjm.n_tiles1 > 0 && nsamp > 0 && adjoint_mma_shape_ok(pl, dtype))
+    return launch_adjoint_mma(pl, SG_TIER_NATIVE, orders, ebar, nullptr, Pbar, dtype, accumulate,
+                              s);
   const bool stream = pl.stream_ok && pl.adj.n_tiles1 > 0 && nsamp > 0 &&
                       (dtype == SG_F32 ? max_nc<float>(pl) : max_nc<double>(pl)) > 0;
   if (dtype == SG_F32) {
     auto e = static_cast<const float*>(ebar);
     auto o = static_cast<float*>(Pbar);
-    if (pl.adjm.n_tiles1 > 0 && nsamp > 0)
-      return launch_adjoint_mma(pl, SG_TIER_NATIVE, orders, e, o, accumulate, s);
     return stream ? adjoint_stream<float>(pl, orders, e, o, accumulate, s)
                   : adjoint_csr<float>(pl, orders, e, o, accumulate, s);
   }

@@ -1,469 +1,615 @@
-// sg_adjoint_mma.hip -- evaluate_adjoint!(grid) for FP32 arrays on matrix
-// cores: Pbar = M^T ebar without atomics (src/adjoint.jl:1-40, :52-83).
+// sg_adjoint_mma.hip -- evaluate_adjoint!(grid) on matrix cores, FP32 and
+// FP64: Pbar = M^T ebar without atomics (src/adjoint.jl:1-40, :52-83), and
+// the adjoint of a NURBS grid's evaluate! in its control points.
 //
 // The two innermost contractions of the adjoint are small matrix products.
-// For a tile of 64 samples j1 whose bands cover at most 16 control points k1
-// (from lo1), 16 rows j2 (a row block) and one sample j3:
+// For a tile of 16 NQ samples j1 whose bands cover at most 16 control points
+// k1 (from lo1), 16 rows j2 and one sample j3:
 //
-//   T1[j2][k1] = sum_j1 ebar[j1, j2, j3] * B1[j1, k1]     (16 x 64) (64 x 16)
+//   T1[j2][k1] = sum_j1 ebar[j1, j2, j3] * B1[j1, k1]     (16 x 16 NQ) (16 NQ x 16)
 //   T2[k2][k1] = sum_j2 B2[j2, k2] * T1[j2][k1]           (16 x 16) (16 x 16)
 //
-// Both run on v_mfma_f32_16x16x4f32 (FP32 products, FP32 sums).  With
-// lane l = 16 g + i, that instruction takes A[i][g] and B[g][i] from lane l
-// and leaves D[4 g + r][i] in register r.  So:
-//   GEMM1, K-step s (16 steps):  A = ebar[j1_0 + j1_of(g, s), row i]
-//                                B = B1[j1_0 + j1_of(g, s)][lo1 + i]
-//     (j1_of(g, s) = 16 (s / 4) + 4 g + s % 4: lane l reads four 16-byte
-//     pieces of its row, and the four lanes of a row read 64 contiguous
-//     bytes per load instruction)
-//   GEMM2, K-step r (4 steps, row j2 = 4 g + r of the block):
-//                                A = B2[4 g + r][lo2 + i]
-//                                B = T1[4 g + r][i] = register r of GEMM1
-//   D2: T2[lo2 + 4 g + r][lo1 + i], summed over the row blocks of the chunk.
-// T2 of each j3 is weighted by B3[j3, d] into a register ring of p3 + 1
-// slabs of k3; a slab whose k3 leaves the band of the next j3 is final for
-// this task and goes to its partial window.  adj_gather (sg_adjoint.hip)
-// then sums the few partial windows that hold each control point.
+// Both run on v_mfma_f32_16x16x4f32 or v_mfma_f64_16x16x4f64 (products and
+// sums of the array's own type).  With lane l = 16 g + i, these take A[i][g]
+// and B[g][i] from lane l and leave D[drow(g, r)][i] in register r, where
+// drow is 4 g + r (FP32) or g + 4 r (FP64).  So:
+//   GEMM1, K-step s (4 NQ steps): A = ebar[j1_0 + samp(g, s), row i]
+//                                 B = B1[j1_0 + samp(g, s)][lo1 + i]
+//     (samp: lane l reads 16-byte pieces of its row, and the four lanes of a
+//     row read 64 contiguous bytes per load instruction)
+//   GEMM2, K-step r (4 steps, row j2 = drow(g, r) of the 16):
+//                                 A = B2[drow(g, r)][lo2 + i]
+//                                 B = T1[drow(g, r)][i] = register r of GEMM1
+//   D2: T2[lo2 + drow(g, r)][lo1 + i].
 //
-// One wave is one task (64 samples x a chunk of up to 64 rows x a range of
-// samples j3, every channel in turn); waves share nothing, so there is no
-// LDS and no barrier.  Only one channel's T2 and ring are live at a time;
-// the ebar buffers take most registers (two waves per SIMD): a wave keeps
-// kBufs - 1 row blocks of ebar in flight ahead of the one it multiplies,
-// across row blocks, samples j3 and channels.
+// 3-D: a wave holds 16 rows and walks a run of samples j3; T2 of each j3 is
+// weighted by B3[j3, d] into a register ring of p3 + 1 slabs of k3.  2-D: a
+// wave walks 16-row blocks and T2 accumulates.  The NW waves of a workgroup
+// (4, 2 or 1) hold neighbouring rows whose bands share one window of 16
+// control points k2, so a slab that is final (its k3 leaves the band of the
+// next j3) is summed over the waves through LDS, in wave order, and one
+// partial window per workgroup goes to HBM; adj_gather (sg_adjoint.hip) then
+// sums the few partial windows that hold each control point.
+//
+// Bound: HBM reads of ebar (a kernel that only reads ebar in this tile pattern
+// takes 76 us of the 82 here on 400 x 400 x 200 samples x 3, 147 of 154 on
+// 512 x 512 x 256 x 3).  With the gather: FP32 400 x 400 x 200 x 3 88 us (91
+// with the channels and 64 rows in one wave); FP32 251 x 197 x 123 x 3 24 us
+// (50: rows of odd length took 4-byte loads); FP64 200 x 201 x 99 x 3 33 us
+// (154 with a sliding window of FMAs and LDS); NURBS 512 x 512 x 256 x 3 181 us
+// (327 with 1 / w(x) written by a pass of its own and read back).  What the
+// layout is for:
+//  - a wave holds one unit (16 rows x 16 NQ samples, 4 KB in FP32, 8 in FP64 at
+//    NQ = 4) and has the next in flight, three to five waves per SIMD;
+//  - the channels are workgroups of their own (plain adjoint), so small grids
+//    fill the chip with fewer, longer runs of j3 and fewer partial windows;
+//  - ebar is read with raw buffer loads: one descriptor per (j3, channel)
+//    plane and per-lane byte offsets.  Any element-aligned row takes the
+//    16-byte loads (gfx950 loads need dword alignment only), the hardware
+//    returns 0 for every dword past the plane, and offsets past it mask rows
+//    past the chunk and samples past m1 without a branch (branches around
+//    loads make the compiler wait for every load in flight at the merge).
+#include <algorithm>
+
 #include "sg_mma_ops.hpp"
+#include "sg_plan_host.hpp"
 
 namespace sg {
 
 namespace {
 
-typedef float f4 __attribute__((ext_vector_type(4)));
+constexpr int kWin = kAdjMmaWin;  // control points per MFMA tile edge
+constexpr int kSlab = kWin * kWin;
 
-constexpr int kTile1 = 64;     // samples j1 per task
-constexpr int kMmaWin = kAdjMmaWin;  // control points per MFMA tile edge
-constexpr int kBufs = 8;  // ebar units per unrolled group; kBufs - 1 are in flight
+template <typename T>
+struct Mfma;
+template <>
+struct Mfma<float> {
+  typedef float D __attribute__((ext_vector_type(4)));
+  typedef float Ld __attribute__((ext_vector_type(4)));  // one 16-byte load
+  static constexpr int VW = 4;                           // elements per load
+  __device__ static constexpr int drow(int g, int r) { return 4 * g + r; }
+  // sample (of 16) of element r of lane group g, and of A row / B column i
+  __device__ static constexpr int samp(int g, int r) { return 4 * g + r; }
+  __device__ static constexpr int column(int i) { return i; }
+  __device__ static D mma(float a, float b, D c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Mfma<double> {
+  typedef double D __attribute__((ext_vector_type(4)));
+  typedef double Ld __attribute__((ext_vector_type(2)));
+  static constexpr int VW = 2;
+  __device__ static constexpr int drow(int g, int r) { return g + 4 * r; }
+  __device__ static constexpr int samp(int g, int r) { return 8 * (r >> 1) + 2 * g + (r & 1); }
+  // D row rho = drow(g, r) holds sample samp(g, r)
+  __device__ static constexpr int column(int i) { return samp(i & 3, i >> 2); }
+  __device__ static D mma(double a, double b, D c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+};
 
+template <typename T>
 struct AdjMmaArgs {
-  const float* E;
-  const float* S;  // scale field [m3][m2][m1] applied to E as it loads (SCALE)
-  float* part;
-  const float* tab1;  // [m1][p1+1]
-  const float* tab2;  // [m2][p2+1]
-  const float* tab3;  // [m3][P3+1]; 2-D grids pass m3 = 1, P3 = 0, B3 = 1
+  const T* E;
+  const T* W;  // NURBS: weights [n3][n2][n1]
+  T* part;
+  const T* tab1;  // [m1][p1+1]
+  const T* tab2;  // [m2][p2+1]
+  const T* tab3;  // [m3][P3+1] (3-D)
   const int32_t* span1;
   const int32_t* span2;
   const int32_t* span3;
-  int m1, m2, m3, p1, p2;
-  int c0, nc, nout;  // channels c0 .. c0 + nc - 1 of nout
-  int chunk, j3_per_task;
-  int ntx, nty, ntasks, w3max;
+  int m1, m2, m3, p1, p2, n1, n2, n3;
+  int nout;
+  int rows, chunk, j3_per_block;
+  int ntx, nty, nz, w1max, w2max, w3max, xcd_map;
   long long m12, nsamp;
 };
 
-// K-step s of GEMM1 takes sample j1_0 + j1_of(g, s): the four lanes of a row
-// (g = 0..3) read 64 contiguous bytes in each 16-byte load q = s / 4.
-__device__ inline int j1_of(int g, int s) { return 16 * (s >> 2) + 4 * g + (s & 3); }
+// Byte offsets at or past a plane's size read 0 (planes are < 2 GiB).
+constexpr unsigned kOff = 0x80000000u;
+constexpr int kRsrcWord3 = 0x00020000;  // raw buffer, 32-bit elements (gfx9)
 
-// ebar is read with raw buffer loads: one descriptor per (sample j3,
-// channel) plane and fixed per-lane byte offsets.  An offset at or past the
-// plane's size returns 0 without a memory access, which masks rows past the
-// chunk and samples past m1 without a branch (branches around loads make
-// the compiler wait for every load in flight at the next merge).
-constexpr unsigned kOff = 0x80000000u;   // always past a plane (< 2 GiB)
-constexpr int kRsrcWord3 = 0x00020000;   // raw buffer, 32-bit elements (gfx9)
+// Units per unrolled group, one register buffer each: KB - 1 are in flight.
+// One unit ahead and three to five waves per SIMD read faster than five ahead
+// and three waves (400 x 400 x 200 samples x 3: 92 us with six buffers, 90
+// with four, 88 with two; 512 x 512 x 256 x 3: 173, 173, 164 us).
+template <int NC>
+constexpr int unit_buffers() {
+  return NC == 1 ? 2 : NC;
+}
 
-// SCALE: ebar times the field S, loaded at the same offsets into buffers of
-// its own; half as many units in flight keeps the registers of both.
-// CM (every tier and the scaled form, p3 <= kCmMaxP3): the units go
-// sample by sample, the channels (at most kCmChannels per launch) of a
-// sample together, each channel with a ring of its own: B3 rows and ring
-// moves once per sample rather than once per channel and sample, and a unit
-// of S is read again by the next channel while it is still in L2 rather
-// than once per channel pass over the task (C4: 95.3 -> 90.6 us; the split-FP16
-// and BF16 tiers 100 -> 98 and 95 us).
-constexpr int kCmMaxP3 = 3;
-constexpr int kCmChannels = 3;
+// NURBS: ebar is multiplied by 1 / w(x) as its units arrive.  The weight
+// field of a unit is two more small products with the same operand trick,
+//   V[k2][j1] = sum_k1 Gw[k2][k1] B1[j1][k1],  w^T[j1][j2] = sum_k2 V[k2][j1] B2[j2][k2],
+// Gw a plane of the window of weights; w^T lands in the lanes and registers
+// that hold ebar's samples.  3-D: a register ring keeps w^T of the p3 + 1
+// planes k3 of the band, so the products run once per plane and a sample j3
+// takes p3 + 1 FMAs per value (the products once per j3 took 32 MFMA of 92).
+// The NC channels of a workgroup share it (units go sample j3 by sample,
+// the channels of a sample together, each channel with a ring of its own).
+template <typename T, int NIN, int P3, int NQ, int NC, int TIER, bool NURBS>
+__global__ __launch_bounds__(kThreads, NURBS && sizeof(T) == 8 ? 1 : 2) void adj_mma(
+    AdjMmaArgs<T> a) {
+  using M = Mfma<T>;
+  using D = typename M::D;
+  using Ld = typename M::Ld;
+  constexpr int VW = M::VW;
+  constexpr int NL = 16 * NQ / 4 / VW;  // 16-byte loads per unit and lane
+  constexpr int KB = unit_buffers<NC>();
+  constexpr int NS = 4 * NQ;  // K-steps of GEMM1, samples per lane
+  static_assert(KB % NC == 0, "the channel of a buffer position must be constant");
+  extern __shared__ __align__(16) unsigned char smem[];
+  T* red = reinterpret_cast<T*>(smem);  // [2][NW][kSlab]
 
-template <int P3, int NB, bool VEC, int TIER, bool SCALE>
-__global__ __launch_bounds__(kThreads) void adj_mma(AdjMmaArgs a) {
-  constexpr int KB = SCALE ? kBufs / 2 : kBufs;  // buffer positions
-  constexpr bool CM = P3 <= kCmMaxP3;
-  constexpr int NCM = CM ? kCmChannels : 1;
-  static_assert(KB % NB == 0, "row block of a buffer position must be constant");
   const int lane = threadIdx.x & (kLanes - 1);
-  const int task = static_cast<int>(blockIdx.x) * kWaves +
-                   __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
-  if (task >= a.ntasks) return;  // whole wave; nothing below synchronises
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+  const int nw = static_cast<int>(blockDim.x) / kLanes;
   const int g = lane >> 4, i = lane & 15;
-  const int bx = task % a.ntx, by = (task / a.ntx) % a.nty, bz = task / (a.ntx * a.nty);
-  const int j1_0 = bx * kTile1;
+  int rest = xcd_logical_block(a.xcd_map, a.ntx);
+  const int bx = rest % a.ntx;
+  rest /= a.ntx;
+  const int by = rest % a.nty;
+  rest /= a.nty;
+  const int bz = rest % a.nz;
+  const int c0 = rest / a.nz * NC;
+  const int nc = NC == 1 ? 1 : min(NC, a.nout - c0);
+  const int j1_0 = bx * 16 * NQ;
   const int r0 = by * a.chunk, r1 = min(r0 + a.chunk, a.m2);
-  const int j3a = bz * a.j3_per_task, j3b = min(j3a + a.j3_per_task, a.m3);
+  const int rb = min(r0 + wave * a.rows, r1), re = min(rb + a.rows, r1);
   const int p1 = a.p1, p2 = a.p2;
   const int lo1 = a.span1[j1_0] - p1;
   const int lo2 = a.span2[r0] - p2;
-  const int W1 = a.span1[min(j1_0 + kTile1, a.m1) - 1] - lo1 + 1;  // <= 16
+  const int W1 = a.span1[min(j1_0 + 16 * NQ, a.m1) - 1] - lo1 + 1;  // <= 16
   const int W2 = a.span2[r1 - 1] - lo2 + 1;                          // <= 16
-  const int lo3 = a.span3[j3a] - P3;
+  const int left = a.m1 - j1_0;             // samples j1 from the tile's first
+  const bool tail = left < 16 * NQ && (left & (VW - 1)) != 0;  // a load crosses the row's end
 
   // Operand tables.  Every load below is unconditional, at a clamped index,
-  // and multiplied by a 0/1 mask afterwards (table values are finite), so
-  // that each group of loads is issued at once and costs one memory latency;
-  // a select would let the compiler move each load under its own branch and
-  // wait for it there.
-  // GEMM1 B operand: B1 at (j1_0 + j1_of(g, s), lo1 + i), 0 off the band
-  float b1[16];
+  // and masked afterwards (table values are finite), so that each group of
+  // loads is issued at once and costs one memory latency.
+  auto b1_at = [&](int j1, int sp, int k1) {
+    const int off = lo1 + k1 - (sp - p1);
+    const T v = a.tab1[static_cast<size_t>(min(j1, a.m1 - 1)) * (p1 + 1) + min(max(off, 0), p1)];
+    return v * ((j1 < a.m1 && off >= 0 && off <= p1) ? T(1) : T(0));
+  };
+  auto b2_at = [&](int j2, int sp, int k2) {
+    const int off = lo2 + k2 - (sp - p2);
+    const T v = a.tab2[static_cast<size_t>(min(j2, r1 - 1)) * (p2 + 1) + min(max(off, 0), p2)];
+    return v * ((j2 < re && off >= 0 && off <= p2) ? T(1) : T(0));
+  };
+  // GEMM1 B operand: B1 at (j1_0 + sample, lo1 + i), 0 off the band
+  T b1[NS];
   {
-    int sp[16];
+    int sp[NS];
 #pragma unroll
-    for (int s = 0; s < 16; ++s) sp[s] = a.span1[min(j1_0 + j1_of(g, s), a.m1 - 1)];
+    for (int s = 0; s < NS; ++s)
+      sp[s] = a.span1[min(j1_0 + 16 * (s >> 2) + M::samp(g, s & 3), a.m1 - 1)];
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int j1 = j1_0 + j1_of(g, s);
-      const int off = lo1 + i - (sp[s] - p1);
-      const float v = a.tab1[static_cast<size_t>(min(j1, a.m1 - 1)) * (p1 + 1) +
-                             min(max(off, 0), p1)];
-      b1[s] = v * ((j1 < a.m1 && off >= 0 && off <= p1) ? 1.f : 0.f);
-    }
+    for (int s = 0; s < NS; ++s) b1[s] = b1_at(j1_0 + 16 * (s >> 2) + M::samp(g, s & 3), sp[s], i);
   }
   // MFMA tiers: GEMM1 on 16x16x32 FP16 / BF16 products.  K block h of a
-  // unit holds samples j1_0 + 32 h + 0..31; element e of lane (g, i) is
-  // sample 16 (2 h + e / 4) + 4 g + e % 4 in both operands -- element e % 4
-  // of its 16-byte load 2 h + e / 4, and K-step 8 h + e of the FP32 path.
-  // B1 is scaled by 2^-eb (split FP16: max|B1| of the task below 1) and
-  // converted once per task.
-  Operand8<TIER == SG_TIER_NATIVE ? SG_TIER_BF16 : TIER> b1op[2];
+  // unit holds samples j1_0 + 32 h + 0..31; element e of a lane is its
+  // K-step 8 h + e of the FP32 path in both operands.  B1 is scaled by 2^-eb
+  // (split FP16: max|B1| of the wave's tile below 1) and converted once.
+  constexpr bool MT = TIER != SG_TIER_NATIVE;
+  Operand8<MT ? TIER : SG_TIER_BF16> b1op[MT ? NQ / 2 : 1];
   int eb = 0;
-  if constexpr (TIER != SG_TIER_NATIVE) {
+  if constexpr (MT) {
     float sb = 1.f;
     if constexpr (TIER == SG_TIER_SPLIT_F16) {
       float m = 0.f;
 #pragma unroll
-      for (int s = 0; s < 16; ++s) m = fmaxf(m, fabsf(b1[s]));
+      for (int s = 0; s < NS; ++s) m = fmaxf(m, fabsf(static_cast<float>(b1[s])));
       eb = scale_exponent(wave_max(m));
       sb = ldexpf(1.f, -eb);
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < NQ / 2; ++h)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) b1op[h].set(e, b1[8 * h + e] * sb);
+      for (int e = 0; e < 8; ++e) b1op[h].set(e, static_cast<float>(b1[8 * h + e]) * sb);
   }
-  // GEMM2 A operand of row block b, K-step r: B2 at (r0 + 16 b + 4 g + r, lo2 + i)
-  float b2[NB][4];
-  {
-    int sp[NB][4];
+  // GEMM2 A operand of the 16 rows from row0, K-step r: B2 at
+  // (row0 + drow(g, r), lo2 + i); NURBS also B2 at (row0 + i, lo2 + drow(g, r))
+  T b2[4], b2t[NURBS ? 4 : 1];
+  auto load_b2 = [&](int row0) {
+    int sp[4];
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+    for (int r = 0; r < 4; ++r) sp[r] = a.span2[min(row0 + M::drow(g, r), r1 - 1)];
+    const int spi = NURBS ? a.span2[min(row0 + i, r1 - 1)] : 0;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sp[b][r] = a.span2[min(r0 + 16 * b + 4 * g + r, r1 - 1)];
+    for (int r = 0; r < 4; ++r) b2[r] = b2_at(row0 + M::drow(g, r), sp[r], i);
+    if constexpr (NURBS) {
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j2 = r0 + 16 * b + 4 * g + r;
-        const int off = lo2 + i - (sp[b][r] - p2);
-        const float v = a.tab2[static_cast<size_t>(min(j2, r1 - 1)) * (p2 + 1) +
-                               min(max(off, 0), p2)];
-        b2[b][r] = v * ((j2 < r1 && off >= 0 && off <= p2) ? 1.f : 0.f);
-      }
-  }
+      for (int r = 0; r < 4; ++r) b2t[r] = b2_at(row0 + i, spi, M::drow(g, r));
+    }
+  };
+  load_b2(rb);
 
-  // Units in order: channel c outermost, then sample j3, then row block b;
-  // unit (c, j3, b) is row r0 + 16 b + i (lane (g, i)) of sample j3 and
-  // channel c0 + c, and load q holds samples j1_0 + 16 q + 4 g .. + 3.
-  const int J = j3b - j3a;
-  const int U = a.nc * J * NB;
-  // byte offset of (row block b, load q) within a plane, or kOff
-  unsigned voff[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j2 = r0 + 16 * b + i;
-    voff[b] = j2 < r1 ? static_cast<unsigned>((j2 * a.m1 + j1_0 + 4 * g) * 4) : kOff;
-  }
-  const unsigned plane_bytes = static_cast<unsigned>(a.m12 * 4);
-  // Load cursor: the (channel, sample) plane of the next unit to load, kept
-  // as running scalar state (no division per load).  Units past the last
-  // read nothing: their descriptor has no records.
-  int lc = 0, ljl = 0;
-  const float* lplane = a.E + static_cast<long long>(j3a) * a.m12 + a.nsamp * a.c0;
-  const float* splane = SCALE ? a.S + static_cast<long long>(j3a) * a.m12 : nullptr;
-  auto load_plane = [&](const float* plane, f4 (&e)[4], int b) {
-    // units past the task's last read nothing: their descriptor has no records
-    const bool live = CM ? ljl < J : lc < a.nc;
+  const int j3a = NIN == 3 ? bz * a.j3_per_block : 0;
+  const int J = NIN == 3 ? min(a.j3_per_block, a.m3 - j3a) : 1;
+  // steps of NC units: samples j3 (3-D) or blocks of 16 rows (2-D)
+  const int steps = NIN == 3 ? J : (re - rb + 15) / 16;
+  const bool any = rb < re;
+
+  // Load cursor: the plane (3-D) and row offset (2-D) of the next unit, kept
+  // as running state; units past the last read nothing (no records).
+  const unsigned plane_bytes = static_cast<unsigned>(a.m12 * static_cast<long long>(sizeof(T)));
+  int lc = 0, lstep = 0;
+  const T* lplane = a.E + static_cast<long long>(j3a) * a.m12 + a.nsamp * c0;
+  auto load = [&](Ld (&e)[NL]) {
+    const int row = (NIN == 2 ? rb + 16 * lstep : rb) + i;
+    const unsigned base = static_cast<unsigned>(
+        (static_cast<long long>(row) * a.m1 + j1_0) * static_cast<long long>(sizeof(T)));
+    const bool live = any && lstep < steps && (NC == 1 || lc < nc);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(plane), 0, static_cast<int>(live ? plane_bytes : 0u), kRsrcWord3);
+        const_cast<T*>(lplane), 0, static_cast<int>(live ? plane_bytes : 0u), kRsrcWord3);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int j1 = j1_0 + 16 * q + 4 * g;
-      if constexpr (VEC) {
-        const unsigned o = j1 < a.m1 ? voff[b] + 64u * q : kOff;
-        // the b128 / b32 loads return raw 32-bit words: reinterpret, not convert
-        e[q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, static_cast<int>(o), 0, 0));
-      } else {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const unsigned o = j1 + w < a.m1 ? voff[b] + 64u * q + 4u * w : kOff;
-          e[q][w] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(o), 0, 0));
-        }
-      }
+    for (int q = 0; q < NL; ++q) {
+      const int s = 4 * VW * q + VW * g;  // the load's first sample
+      const unsigned o = row < re && s < left
+                             ? base + static_cast<unsigned>(s * static_cast<int>(sizeof(T)))
+                             : kOff;
+      // the b128 loads return raw 32-bit words: reinterpret, not convert
+      e[q] = __builtin_bit_cast(Ld, __builtin_amdgcn_raw_buffer_load_b128(rs, static_cast<int>(o), 0, 0));
     }
-  };
-  auto load = [&](f4 (&e)[4], f4 (&d)[4], int b) {
-    load_plane(lplane, e, b);
-    if constexpr (SCALE) load_plane(splane, d, b);
-    if (b == NB - 1) {  // the plane's last row block: advance the cursor
-      if constexpr (CM) {  // units (sample, channel, row block)
-        if (++lc == a.nc) {
-          lc = 0;
-          ++ljl;
-          splane += a.m12;
-        }
-        lplane = a.E + static_cast<long long>(j3a + ljl) * a.m12 + a.nsamp * (a.c0 + lc);
-      } else {  // units (channel, sample, row block)
-        lplane += a.m12;
-        if constexpr (SCALE) splane += a.m12;
-        if (++ljl == J) {
-          ljl = 0;
-          ++lc;
-          lplane = a.E + static_cast<long long>(j3a) * a.m12 + a.nsamp * (a.c0 + lc);
-          if constexpr (SCALE) splane = a.S + static_cast<long long>(j3a) * a.m12;
-        }
+    if (NC == 1) {
+      ++lstep;
+      if (NIN == 3) lplane += a.m12;
+    } else {
+      lplane += a.nsamp;
+      if (++lc == NC) {
+        lc = 0;
+        ++lstep;
+        lplane += (NIN == 3 ? a.m12 : 0) - NC * a.nsamp;
       }
     }
   };
 
-  // Units are taken in unrolled groups of KB with one register buffer per
-  // position: at position k the unit KB - 1 ahead is loaded into the
-  // buffer that position k - 1 has just used, so KB - 1 units are in
-  // flight and no buffer is ever copied (a copy of a register whose load is
-  // in flight waits for that load).  KB % NB == 0 keeps the row block of
-  // position k, k % NB, a constant.
-  f4 buf[KB][4];
-  f4 sbuf[SCALE ? KB : 1][4];  // the scale of each buffered unit (SCALE)
+  // At position k of a group the unit KB - 1 ahead is loaded into the buffer
+  // that position k - 1 has just used, so KB - 1 units are in flight and no
+  // buffer is ever copied (a copy of a register whose load is in flight
+  // waits for that load).
+  Ld buf[KB][NL];
 #pragma unroll
-  for (int k = 0; k < KB - 1; ++k) load(buf[k], sbuf[SCALE ? k : 0], k % NB);
+  for (int k = 0; k < KB - 1; ++k) load(buf[k]);
 
-  f4 R[P3 + 1];  // ring of the current channel: slot q holds k3 = cur3 - P3 + q
+  // NURBS: rw[d] holds w^T of plane k3 = cur3 - P3 + d at the lane's samples
+  // (2-D: the one plane of the current row block), wn the window of weights of
+  // the next plane, lane (g, i) at (k2 = lo2 + i, k1 = lo1 + 4 g + s), and b1t
+  // B1 at (sample column(i) of block q, lo1 + 4 g + s)
+  T rw[NURBS ? P3 + 1 : 1][NURBS ? NS : 1], b1t[NURBS ? NQ : 1][4], wn[4], inv[NURBS ? NS : 1];
+  const int lo3 = NIN == 3 ? a.span3[j3a] - P3 : 0;
+  int cur3 = lo3 + P3;
+  auto load_w = [&](int k3) {
+    if constexpr (NURBS) {
+      const T* src = a.W + (static_cast<long long>(min(k3, a.n3 - 1)) * a.n2 +
+                            min(lo2 + i, a.n2 - 1)) * a.n1;
 #pragma unroll
-  for (int q = 0; q <= P3; ++q) R[q] = f4{0.f, 0.f, 0.f, 0.f};
-  // CM: a ring per channel, and the B3 row of the current sample
-  f4 RC[NCM][CM ? P3 + 1 : 1];
-  float b3c[P3 + 1];
-  if constexpr (CM) {
+      for (int s = 0; s < 4; ++s) {
+        const T v = src[min(lo1 + 4 * g + s, a.n1 - 1)];
+        wn[s] = i < W2 && 4 * g + s < W1 ? v : T(0);
+      }
+    }
+  };
+  // the plane in wn at the tile's samples of the rows in b2t
+  auto plane_w = [&](T (&out)[NURBS ? NS : 1]) {
+    if constexpr (NURBS) {
 #pragma unroll
-    for (int ch = 0; ch < NCM; ++ch)
+      for (int q = 0; q < NQ; ++q) {
+        D v = {T(0), T(0), T(0), T(0)}, w = {T(0), T(0), T(0), T(0)};
 #pragma unroll
-      for (int q = 0; q <= P3; ++q) RC[ch][q] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < 4; ++s) v = M::mma(wn[s], b1t[q][s], v);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) w = M::mma(v[r], b2t[r], w);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[4 * q + r] = w[r];
+      }
+    }
+  };
+  // 1 / w; rows and samples outside the grid have w = 0, and their ebar reads 0
+  auto recip_w = [&](const T (&w)[NURBS ? NS : 1], int row0) {
+    const bool rowok = row0 + i < re;
+#pragma unroll
+    for (int s = 0; s < (NURBS ? NS : 1); ++s)
+      inv[s] = rowok && 16 * (s >> 2) + M::samp(g, s & 3) < left ? T(1) / w[s] : T(0);
+  };
+  if constexpr (NURBS) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int j1 = j1_0 + 16 * q + M::column(i);
+      const int sp = a.span1[min(j1, a.m1 - 1)];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) b1t[q][s] = b1_at(j1, sp, 4 * g + s);
+    }
+    load_w(lo3);
+    if constexpr (NIN == 3) {
+#pragma unroll
+      for (int d = 0; d <= P3; ++d) {
+        plane_w(rw[d]);
+        load_w(lo3 + d + 1);
+      }
+    }
   }
-  int cur3 = a.span3[j3a];
-  f4 acc = {0.f, 0.f, 0.f, 0.f};  // T2 of the current sample j3
-  // B3 row of the next sample, loaded one sample ahead (before that sample's
-  // ebar loads, so that waiting for it drains none of them)
-  float b3n[P3 + 1];
-#pragma unroll
-  for (int q = 0; q <= P3; ++q) b3n[q] = a.tab3[static_cast<size_t>(j3a) * (P3 + 1) + q];
 
-  // slot k3 of channel c is final: lane (g, i) writes
-  // part[task][k3 - lo3][c0 + c][4 g + r][i] inside the task's W2 x W1
-  // window (the gather reads no other entry)
-  auto flush = [&](const f4& slab, int c, int k3) {
-    float* dst = a.part + ((static_cast<size_t>(task) * a.w3max + (k3 - lo3)) * a.nout +
-                           a.c0 + c) * (kMmaWin * kMmaWin);
-    if (i >= W1) return;
+  // R[ch][d]: slab k3 = cur3 - P3 + d of channel c0 + ch (2-D: T2 itself)
+  D R[NC][P3 + 1];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (4 * g + r < W2) dst[(4 * g + r) * kMmaWin + i] = slab[r];
+  for (int ch = 0; ch < NC; ++ch)
+#pragma unroll
+    for (int d = 0; d <= P3; ++d) R[ch][d] = D{T(0), T(0), T(0), T(0)};
+
+  // Slab k3 of channel c0 + ch is final: summed over the waves in order, it
+  // goes to part[block][k3 - lo3][channel] inside the W2 x W1 window (the
+  // gather reads no other entry).  Two LDS slots in turn: a wave reaches the
+  // next use of a slot only past the barrier that follows every wave's reads
+  // of it.
+  int par = 0;
+  const size_t block = (static_cast<size_t>(bz) * a.nty + by) * a.ntx + bx;
+  auto flush = [&](const D& slab, int ch, int k3) {
+    T* dst = a.part + ((block * a.w3max + (k3 - lo3)) * a.nout + c0 + ch) *
+                          (static_cast<size_t>(a.w1max) * a.w2max);
+    if (nw == 1) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (M::drow(g, r) < W2 && i < W1) dst[M::drow(g, r) * a.w1max + i] = slab[r];
+      return;
+    }
+    T* slot = red + static_cast<size_t>(par) * nw * kSlab;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) slot[wave * kSlab + r * kLanes + lane] = slab[r];
+    __syncthreads();
+    for (int t = threadIdx.x; t < kSlab; t += nw * kLanes) {
+      T s = slot[t];
+      for (int w = 1; w < nw; ++w) s += slot[w * kSlab + t];
+      const int row = M::drow((t >> 4) & 3, t >> 6), col = t & 15;
+      if (row < W2 && col < W1) dst[row * a.w1max + col] = s;
+    }
+    par ^= 1;
   };
 
-  // compute cursor: channel and sample of the unit being multiplied
-  int cc = 0, cjl = 0;
-  for (int u0 = 0; u0 < U; u0 += KB) {
+  // B3 rows and spans through the constant address space: the index is
+  // uniform, so they are scalar loads and wait for no ebar load
+  Constant<const T>* tab3 = constant_ptr(a.tab3);
+  Constant<const int32_t>* span3 = constant_ptr(a.span3);
+  T b3[P3 + 1];
+  for (int s0 = 0; s0 < steps; s0 += KB / NC) {
 #pragma unroll
     for (int k = 0; k < KB; ++k) {
-      const int u = u0 + k;
-      load(buf[(k + KB - 1) % KB], sbuf[SCALE ? (k + KB - 1) % KB : 0], (k + KB - 1) % NB);
-      if (u < U) {
-        const int b = k % NB;
-        if constexpr (SCALE) {
+      const int ch = k % NC;          // the unit's channel
+      const int step = s0 + k / NC;   // its sample j3 - j3a, or row block
+      load(buf[(k + KB - 1) % KB]);
+      if (step < steps) {
+        if (ch == 0) {
+          if constexpr (NIN == 3) {
+            const int j3 = j3a + step;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) buf[k][q] *= sbuf[k][q];
-        }
-        f4 d1 = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (TIER == SG_TIER_NATIVE) {
+            for (int d = 0; d <= P3; ++d) b3[d] = tab3[static_cast<size_t>(j3) * (P3 + 1) + d];
+            const int s3 = span3[j3];
+            while (cur3 < s3) {  // every ring moves to the sample's band
 #pragma unroll
-          for (int s = 0; s < 16; ++s)
-            d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(buf[k][s >> 2][s & 3], b1[s], d1, 0, 0, 0);
-        } else {
-          // split FP16: the unit's ebar scaled by 2^-eu (max below 1), and
-          // T1 scaled back by 2^(eu + eb); BF16 needs no scaling
-          int eu = 0;
-          float su = 1.f;
-          if constexpr (TIER == SG_TIER_SPLIT_F16) {
-            float m = 0.f;
+              for (int cc = 0; cc < NC; ++cc) {
+                if (cc < nc) flush(R[cc][0], cc, cur3 - P3);
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-              for (int t = 0; t < 4; ++t) m = fmaxf(m, fabsf(buf[k][q][t]));
-            eu = scale_exponent(wave_max(m));
-            su = ldexpf(1.f, -eu);
-          }
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            Operand8<TIER> op;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) op.set(e, buf[k][2 * h + e / 4][e % 4] * su);
-            d1 = Operand8<TIER>::mma(op, b1op[h], d1);
-          }
-          if constexpr (TIER == SG_TIER_SPLIT_F16) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) d1[r] = ldexpf(d1[r], eu + eb);
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b2[b][r], d1[r], acc, 0, 0, 0);
-        if (CM && b == NB - 1) {
-          // T2 of sample j3, channel c is complete: at the sample's first
-          // channel every ring moves to the sample's band; then channel c's
-          // ring takes it
-          const int c = cc, jl = cjl;
-          const int j3 = j3a + jl;
-          if (++cc == a.nc) {
-            cc = 0;
-            ++cjl;
-          }
-          if (c == 0) {
-#pragma unroll
-            for (int q = 0; q <= P3; ++q) b3c[q] = b3n[q];
-            const int j3n = jl + 1 < J ? j3 + 1 : j3;
-#pragma unroll
-            for (int q = 0; q <= P3; ++q)
-              b3n[q] = a.tab3[static_cast<size_t>(j3n) * (P3 + 1) + q];
-            const int s3 = a.span3[j3];
-            while (cur3 < s3) {
-#pragma unroll
-              for (int ch = 0; ch < NCM; ++ch) {
-                if (ch < a.nc) flush(RC[ch][0], ch, cur3 - P3);
-#pragma unroll
-                for (int q = 0; q < P3; ++q) RC[ch][q] = RC[ch][q + 1];
-                RC[ch][P3] = f4{0.f, 0.f, 0.f, 0.f};
+                for (int d = 0; d < P3; ++d) R[cc][d] = R[cc][d + 1];
+                R[cc][P3] = D{T(0), T(0), T(0), T(0)};
               }
               ++cur3;
-            }
-          }
+              if constexpr (NURBS) {
 #pragma unroll
-          for (int ch = 0; ch < NCM; ++ch)
-            if (ch == c) {  // c is uniform: a scalar branch, no register indexing
+                for (int d = 0; d < P3; ++d)
 #pragma unroll
-              for (int q = 0; q <= P3; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) RC[ch][q][r] += b3c[q] * acc[r];
-            }
-          acc = f4{0.f, 0.f, 0.f, 0.f};
-          if (jl == J - 1 && c == a.nc - 1) {  // the task's last unit: every ring is final
-#pragma unroll
-            for (int ch = 0; ch < NCM; ++ch)
-              if (ch < a.nc) {
-#pragma unroll
-                for (int q = 0; q <= P3; ++q) flush(RC[ch][q], ch, cur3 - P3 + q);
+                  for (int s = 0; s < NS; ++s) rw[d][s] = rw[d + 1][s];
+                plane_w(rw[P3]);
+                load_w(cur3 + 1);
               }
-          }
-        } else if (!CM && b == NB - 1) {
-          // T2 of sample j3 is complete: weight it into the ring
-          const int c = cc, jl = cjl;
-          const int j3 = j3a + jl;
-          if (++cjl == J) {
-            cjl = 0;
-            ++cc;
-          }
-          float b3[P3 + 1];
-#pragma unroll
-          for (int q = 0; q <= P3; ++q) b3[q] = b3n[q];
-          const int j3n = jl + 1 < J ? j3 + 1 : j3a;  // the next channel restarts at j3a
-#pragma unroll
-          for (int q = 0; q <= P3; ++q) b3n[q] = a.tab3[static_cast<size_t>(j3n) * (P3 + 1) + q];
-          const int s3 = a.span3[j3];
-          while (cur3 < s3) {
-            flush(R[0], c, cur3 - P3);
-#pragma unroll
-            for (int q = 0; q < P3; ++q) R[q] = R[q + 1];
-            R[P3] = f4{0.f, 0.f, 0.f, 0.f};
-            ++cur3;
-          }
-#pragma unroll
-          for (int q = 0; q <= P3; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) R[q][r] += b3[q] * acc[r];
-          acc = f4{0.f, 0.f, 0.f, 0.f};
-          if (jl == J - 1) {  // last sample of channel c: the ring is final
-#pragma unroll
-            for (int q = 0; q <= P3; ++q) {
-              flush(R[q], c, cur3 - P3 + q);
-              R[q] = f4{0.f, 0.f, 0.f, 0.f};
             }
-            cur3 = a.span3[j3a];
+            if constexpr (NURBS) {
+              T w[NS];
+#pragma unroll
+              for (int s = 0; s < NS; ++s) {
+                w[s] = T(0);
+#pragma unroll
+                for (int d = 0; d <= P3; ++d) w[s] += b3[d] * rw[d][s];
+              }
+              recip_w(w, rb);
+            }
+          } else {
+            if (step > 0) load_b2(rb + 16 * step);
+            if constexpr (NURBS) {
+              plane_w(rw[0]);
+              recip_w(rw[0], rb + 16 * step);
+            }
+          }
+        }
+        if (any && (NC == 1 || ch < nc)) {
+          T e[NS];
+#pragma unroll
+          for (int s = 0; s < NS; ++s) e[s] = buf[k][s / VW][s % VW];
+          if (tail) {  // elements past the row's end are the next row's
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+              e[s] = 16 * (s >> 2) + M::samp(g, s & 3) < left ? e[s] : T(0);
+          }
+          if constexpr (NURBS) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) e[s] *= inv[s];
+          }
+          D d1 = {T(0), T(0), T(0), T(0)};
+          if constexpr (!MT) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) d1 = M::mma(e[s], b1[s], d1);
+          } else {
+            // split FP16: the unit's ebar scaled by 2^-eu (max below 1), and
+            // T1 scaled back by 2^(eu + eb); BF16 needs no scaling
+            int eu = 0;
+            float su = 1.f;
+            if constexpr (TIER == SG_TIER_SPLIT_F16) {
+              float m = 0.f;
+#pragma unroll
+              for (int s = 0; s < NS; ++s) m = fmaxf(m, fabsf(e[s]));
+              eu = scale_exponent(wave_max(m));
+              su = ldexpf(1.f, -eu);
+            }
+#pragma unroll
+            for (int h = 0; h < NQ / 2; ++h) {
+              Operand8<TIER> op;
+#pragma unroll
+              for (int x = 0; x < 8; ++x) op.set(x, e[8 * h + x] * su);
+              d1 = Operand8<TIER>::mma(op, b1op[h], d1);
+            }
+            if constexpr (TIER == SG_TIER_SPLIT_F16) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r) d1[r] = ldexpf(d1[r], eu + eb);
+            }
+          }
+          if constexpr (NIN == 2) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) R[ch][0] = M::mma(b2[r], d1[r], R[ch][0]);
+          } else {
+            D t2 = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) t2 = M::mma(b2[r], d1[r], t2);
+#pragma unroll
+            for (int d = 0; d <= P3; ++d)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) R[ch][d][r] += b3[d] * t2[r];
           }
         }
       }
     }
   }
+  // the run's last band is final
+#pragma unroll
+  for (int d = 0; d <= P3; ++d)
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc)
+      if (cc < nc) flush(R[cc][d], cc, cur3 - P3 + d);
 }
 
-using AdjMmaKernel = void (*)(AdjMmaArgs);
+template <typename T>
+using AdjMmaKernel = void (*)(AdjMmaArgs<T>);
 
-template <int P3, int NB, bool VEC>
-AdjMmaKernel pick_tier(int tier, bool scale) {
-  if (scale)  // the scaled form: native tier only
-    return tier == SG_TIER_NATIVE ? adj_mma<P3, NB, VEC, SG_TIER_NATIVE, true> : nullptr;
-  switch (tier) {
-    case SG_TIER_NATIVE: return adj_mma<P3, NB, VEC, SG_TIER_NATIVE, false>;
-    case SG_TIER_SPLIT_F16: return adj_mma<P3, NB, VEC, SG_TIER_SPLIT_F16, false>;
-    case SG_TIER_BF16: return adj_mma<P3, NB, VEC, SG_TIER_BF16, false>;
+template <typename T, int NIN, int P3, int NQ>
+AdjMmaKernel<T> pick_tier(int tier, int nurbs_nc) {
+  if constexpr (sizeof(T) == 4) {
+    if constexpr (P3 <= kSharedMaxP3)
+      if (nurbs_nc == 3) return adj_mma<T, NIN, P3, NQ, 3, SG_TIER_NATIVE, true>;
+    if (nurbs_nc == 1) return adj_mma<T, NIN, P3, NQ, 1, SG_TIER_NATIVE, true>;
+    switch (tier) {
+      case SG_TIER_NATIVE: return adj_mma<T, NIN, P3, NQ, 1, SG_TIER_NATIVE, false>;
+      case SG_TIER_SPLIT_F16: return adj_mma<T, NIN, P3, NQ, 1, SG_TIER_SPLIT_F16, false>;
+      case SG_TIER_BF16: return adj_mma<T, NIN, P3, NQ, 1, SG_TIER_BF16, false>;
+    }
+    return nullptr;
+  } else {
+    return nurbs_nc ? adj_mma<T, NIN, P3, NQ, 1, SG_TIER_NATIVE, true>
+                    : adj_mma<T, NIN, P3, NQ, 1, SG_TIER_NATIVE, false>;
+  }
+}
+
+template <typename T, int NIN, int P3>
+AdjMmaKernel<T> pick_nq(int tile_width, int tier, int nurbs_nc) {
+  return tile_width == 64 ? pick_tier<T, NIN, P3, 4>(tier, nurbs_nc)
+                          : pick_tier<T, NIN, P3, 2>(tier, nurbs_nc);
+}
+
+template <typename T>
+AdjMmaKernel<T> pick_adj_mma(const Plan& pl, int tier, int nurbs_nc) {
+  const int tw = pl.adjm.tile_width();
+  if (pl.nin == 2) return pick_nq<T, 2, 0>(tw, tier, nurbs_nc);
+  switch (pl.dims[2].p) {
+    case 0: return pick_nq<T, 3, 0>(tw, tier, nurbs_nc);
+    case 1: return pick_nq<T, 3, 1>(tw, tier, nurbs_nc);
+    case 2: return pick_nq<T, 3, 2>(tw, tier, nurbs_nc);
+    case 3: return pick_nq<T, 3, 3>(tw, tier, nurbs_nc);
+    case 4: return pick_nq<T, 3, 4>(tw, tier, nurbs_nc);
+    case 5: return pick_nq<T, 3, 5>(tw, tier, nurbs_nc);
   }
   return nullptr;
 }
 
-template <int P3, int NB>
-AdjMmaKernel pick_vec(bool vec, int tier, bool scale) {
-  return vec ? pick_tier<P3, NB, true>(tier, scale) : pick_tier<P3, NB, false>(tier, scale);
+long long plane_samples(const Plan& pl) {
+  return static_cast<long long>(pl.dims[0].m) * pl.dims[1].m;
 }
 
-template <int P3>
-AdjMmaKernel pick_nb(int nb, bool vec, int tier, bool scale) {
-  switch (nb) {
-    case 1: return pick_vec<P3, 1>(vec, tier, scale);
-    case 2: return pick_vec<P3, 2>(vec, tier, scale);
-    case 4: return pick_vec<P3, 4>(vec, tier, scale);
+template <typename T>
+hipError_t launch_mma(const Plan& pl, int tier, const int32_t* orders, const T* E, const T* W,
+                      T* Pbar, int accumulate, hipStream_t s) {
+  const Tiling& tl = pl.adjm;
+  const DimDev& d1 = pl.dims[0];
+  const DimDev& d2 = pl.dims[1];
+  const auto table = [](const DimDev& d, int order) {
+    const size_t at = static_cast<size_t>(order) * d.m * (d.p + 1);
+    if constexpr (sizeof(T) == 4)
+      return static_cast<const T*>(d.ktab32 + at);
+    else
+      return static_cast<const T*>(d.ktab64 + at);
+  };
+  AdjMmaArgs<T> a{};
+  a.E = E;
+  a.W = W;
+  a.part = static_cast<T*>(pl.work);
+  a.tab1 = table(d1, orders[0]);
+  a.tab2 = table(d2, orders[1]);
+  a.span1 = d1.span;
+  a.span2 = d2.span;
+  a.m1 = d1.m;
+  a.m2 = d2.m;
+  a.m3 = 1;
+  a.p1 = d1.p;
+  a.p2 = d2.p;
+  a.n1 = d1.n;
+  a.n2 = d2.n;
+  a.n3 = 1;
+  if (pl.nin == 3) {
+    const DimDev& d3 = pl.dims[2];
+    a.tab3 = table(d3, orders[2]);
+    a.span3 = d3.span;
+    a.m3 = d3.m;
+    a.n3 = d3.n;
   }
-  return nullptr;
+  a.nout = pl.nout;
+  a.rows = tl.rows_per_wave;
+  a.chunk = tl.chunk_rows();
+  a.j3_per_block = tl.j3_per_block;
+  a.ntx = tl.n_tiles1;
+  a.nty = tl.n_chunks2;
+  a.nz = tl.n_z;
+  a.xcd_map = tl.xcd_map;
+  a.w1max = tl.w1max;
+  a.w2max = tl.w2max;
+  a.w3max = tl.w3max;
+  a.m12 = plane_samples(pl);
+  a.nsamp = a.m12 * a.m3;
+  const int nurbs_nc = !W ? 0 : sizeof(T) == 4 && adjoint_shares_weights(pl) ? 3 : 1;
+  const int per = std::max(nurbs_nc, 1);
+  AdjMmaKernel<T> k = pick_adj_mma<T>(pl, tier, nurbs_nc);
+  if (!k) return hipErrorInvalidValue;
+  const int nw = tl.chunk_rows() / tl.rows_per_wave;
+  const unsigned blocks = static_cast<unsigned>(tl.n_tiles1) * tl.n_chunks2 * tl.n_z *
+                          ((pl.nout + per - 1) / per);
+  const size_t lds = nw > 1 ? 2 * static_cast<size_t>(nw) * kSlab * sizeof(T) : 0;
+  hipLaunchKernelGGL(k, dim3(blocks), dim3(nw * kLanes), lds, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_adjoint_gather(pl, tl, pl.work, Pbar, sizeof(T) == 4 ? SG_F32 : SG_F64,
+                               accumulate, s, W);
 }
-
-AdjMmaKernel pick_adj_mma(int p3, int nb, bool vec, int tier, bool scale = false) {
-  switch (p3) {
-    case 0: return pick_nb<0>(nb, vec, tier, scale);
-    case 1: return pick_nb<1>(nb, vec, tier, scale);
-    case 2: return pick_nb<2>(nb, vec, tier, scale);
-    case 3: return pick_nb<3>(nb, vec, tier, scale);
-    case 4: return pick_nb<4>(nb, vec, tier, scale);
-    case 5: return pick_nb<5>(nb, vec, tier, scale);
-  }
-  return nullptr;
-}
-
-int plan_p3(const Plan& pl) { return pl.nin == 3 ? pl.dims[2].p : 0; }
 
 }  // namespace
 
-bool adjoint_mma_shape_ok(const Plan& pl) {
+bool adjoint_mma_shape_ok(const Plan& pl, int dtype) {
   // one (sample j3, channel) plane of ebar must stay below the out-of-range
   // offset of the buffer loads
-  const long long m12 = static_cast<long long>(pl.dims[0].m) * pl.dims[1].m;
-  return (pl.nin == 2 || pl.nin == 3) && plan_p3(pl) <= kMaxStreamDegree &&
-         m12 * 4 < static_cast<long long>(kOff) - 64;
+  return (pl.nin == 2 || pl.nin == 3) && (pl.nin == 2 || pl.dims[2].p <= kMaxStreamDegree) &&
+         plane_samples(pl) * (dtype == SG_F32 ? 4 : 8) < static_cast<long long>(kOff) - 64;
 }
 
 int adjoint_mma_resident_waves(const Plan& pl) {
-  AdjMmaKernel k = pick_adj_mma(plan_p3(pl), pl.adjm.chunk_rows() / 16, true, SG_TIER_NATIVE);
+  AdjMmaKernel<float> k = pick_adj_mma<float>(pl, SG_TIER_NATIVE, 0);
   if (!k) return 0;
   int blocks = 0, cus = 0, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
@@ -479,62 +625,19 @@ size_t adjoint_mma_work_bytes(const Plan& pl) {
   const Tiling& t = pl.adjm;
   if (t.n_tiles1 == 0) return 0;
   const size_t units = static_cast<size_t>(t.n_tiles1) * t.n_chunks2 * t.n_z;
-  return units * t.w3max * pl.nout * kMmaWin * kMmaWin * sizeof(float);
+  return units * t.w3max * pl.nout * t.w1max * t.w2max * sizeof(double);
 }
 
-hipError_t launch_adjoint_mma(const Plan& pl, int tier, const int32_t* orders, const float* E,
-                              float* Pbar, int accumulate, hipStream_t s, const float* scale) {
-  const Tiling& tl = pl.adjm;
-  const DimDev& d1 = pl.dims[0];
-  const DimDev& d2 = pl.dims[1];
-  AdjMmaArgs a{};
-  a.E = E;
-  a.S = scale;
-  a.part = static_cast<float*>(pl.work);
-  a.tab1 = d1.ktab32 + static_cast<size_t>(orders[0]) * d1.m * (d1.p + 1);
-  a.tab2 = d2.ktab32 + static_cast<size_t>(orders[1]) * d2.m * (d2.p + 1);
-  a.span1 = d1.span;
-  a.span2 = d2.span;
-  a.m1 = d1.m;
-  a.m2 = d2.m;
-  a.m3 = 1;
-  a.p1 = d1.p;
-  a.p2 = d2.p;
-  if (pl.nin == 3) {
-    const DimDev& d3 = pl.dims[2];
-    a.tab3 = d3.ktab32 + static_cast<size_t>(orders[2]) * d3.m * (d3.p + 1);
-    a.span3 = d3.span;
-    a.m3 = d3.m;
-  } else {  // one sample j3 = 0 with span 0 and B3 = 1
-    a.tab3 = pl.unit_tab;
-    a.span3 = pl.unit_span;
-  }
-  a.nout = pl.nout;
-  a.chunk = tl.chunk_rows();
-  a.j3_per_task = tl.j3_per_block;
-  a.ntx = tl.n_tiles1;
-  a.nty = tl.n_chunks2;
-  a.ntasks = tl.n_tiles1 * tl.n_chunks2 * tl.n_z;
-  a.w3max = tl.w3max;
-  a.m12 = static_cast<long long>(d1.m) * d2.m;
-  a.nsamp = a.m12 * a.m3;
-  // 16-byte loads need 16-byte rows: m1 % 4 == 0 and an aligned base
-  const bool vec = (d1.m % 4 == 0) && (reinterpret_cast<uintptr_t>(E) % 16 == 0) &&
-                   (reinterpret_cast<uintptr_t>(scale) % 16 == 0);
-  const dim3 grid(static_cast<unsigned>((a.ntasks + kWaves - 1) / kWaves));
-  AdjMmaKernel k = pick_adj_mma(plan_p3(pl), tl.chunk_rows() / 16, vec, tier, scale != nullptr);
-  if (!k) return hipErrorInvalidValue;
-  // channels in the middle: kCmChannels per launch
-  const int per = plan_p3(pl) <= kCmMaxP3 ? kCmChannels : pl.nout;
-  hipError_t e = hipSuccess;
-  for (int c0 = 0; c0 < pl.nout && e == hipSuccess; c0 += per) {
-    a.c0 = c0;
-    a.nc = std::min(per, pl.nout - c0);
-    hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, s, a);
-    e = hipGetLastError();
-  }
-  if (e != hipSuccess) return e;
-  return launch_adjoint_gather(pl, tl, pl.work, Pbar, SG_F32, accumulate, s);
+hipError_t launch_adjoint_mma(const Plan& pl, int tier, const int32_t* orders, const void* E,
+                              const void* W, void* Pbar, int dtype, int accumulate,
+                              hipStream_t s) {
+  if (dtype == SG_F32)
+    return launch_mma<float>(pl, tier, orders, static_cast<const float*>(E),
+                             static_cast<const float*>(W), static_cast<float*>(Pbar), accumulate,
+                             s);
+  return launch_mma<double>(pl, tier, orders, static_cast<const double*>(E),
+                            static_cast<const double*>(W), static_cast<double*>(Pbar), accumulate,
+                            s);
 }
 
 }  // namespace sg

@@ -173,22 +173,19 @@ int validate_desc(const sg_grid_desc* desc) {
 }
 
 // Uploads the gather lists of tiling tl (partial windows w1 x w2 x w3max per
-// channel): the lists adj_gather walks.
+// channel) as the tables adj_gather reads.
 static hipError_t upload_gather_lists(Plan& pl, Tiling& tl, int w1, int w2) {
-  GatherLists g = gather_lists(pl, tl, w1, w2);
-  std::vector<int32_t>* ptr = g.ptr;
-  std::vector<long long>* off = g.off;
+  const GatherLists g = gather_lists(pl, tl, w1, w2);
   tl.gchan = g.gchan;
-  tl.gfast = g.gfast;
+  tl.gwindows = 1;
   hipError_t e = hipSuccess;
   for (int d = 0; d < 3 && e == hipSuccess; ++d) {
-    e = dalloc(pl, &tl.gptr[d], ptr[d].size());
-    if (e == hipSuccess) e = dalloc(pl, &tl.goff[d], off[d].size());
+    int most = 0;
+    const std::vector<long long> table = gather_table(g, d, most);
+    tl.gwindows *= most;
+    e = dalloc(pl, &tl.glist[d], table.size());
     if (e == hipSuccess)
-      e = hipMemcpy(tl.gptr[d], ptr[d].data(), ptr[d].size() * sizeof(int32_t),
-                    hipMemcpyHostToDevice);
-    if (e == hipSuccess && !off[d].empty())
-      e = hipMemcpy(tl.goff[d], off[d].data(), off[d].size() * sizeof(long long),
+      e = hipMemcpy(tl.glist[d], table.data(), table.size() * sizeof(long long),
                     hipMemcpyHostToDevice);
   }
   return e;
@@ -278,22 +275,14 @@ int build_plan(const sg_grid_desc* desc, hipStream_t s, bool want_adjoint, Plan*
   }
   if (rc != SG_OK) return rc;
 
-  plan_tilings(*pl, want_adjoint, adjoint_mma_shape_ok(*pl), adjoint_mma_resident_waves);
-  const bool ok = pl->stream_ok;
-  if (ok && (pl->adj.n_tiles1 > 0 || pl->adjm.n_tiles1 > 0)) {
+  plan_tilings(*pl, want_adjoint, adjoint_mma_shape_ok(*pl, SG_F32), adjoint_mma_resident_waves);
+  // adj_stream is reached only where the matrix-core adjoint is not: without
+  // its tiling, or (FP64) with planes past its buffer loads
+  if (pl->adjm.n_tiles1 > 0 && adjoint_mma_shape_ok(*pl, SG_F64)) pl->adj = Tiling();
+  if (pl->stream_ok && (pl->adj.n_tiles1 > 0 || pl->adjm.n_tiles1 > 0)) {
     hipError_t e = hipSuccess;
-    if (pl->adj.n_tiles1 > 0) e = upload_gather_lists(*pl, pl->adj, pl->adj.w1max, pl->adj.w2max);
-    if (e == hipSuccess && pl->adjm.n_tiles1 > 0)
-      e = upload_gather_lists(*pl, pl->adjm, kAdjMmaWin, kAdjMmaWin);
-    if (e == hipSuccess && pl->adjm.n_tiles1 > 0 && pl->nin == 2) {
-      const float one = 1.f;
-      const int32_t zero = 0;
-      e = dalloc(*pl, &pl->unit_tab, 1);
-      if (e == hipSuccess) e = dalloc(*pl, &pl->unit_span, 1);
-      if (e == hipSuccess) e = hipMemcpy(pl->unit_tab, &one, sizeof(one), hipMemcpyHostToDevice);
-      if (e == hipSuccess)
-        e = hipMemcpy(pl->unit_span, &zero, sizeof(zero), hipMemcpyHostToDevice);
-    }
+    for (Tiling* t : {&pl->adj, &pl->adjm})
+      if (e == hipSuccess && t->n_tiles1 > 0) e = upload_gather_lists(*pl, *t, t->w1max, t->w2max);
     pl->work_bytes = std::max(adjoint_work_bytes(*pl), adjoint_mma_work_bytes(*pl));
     unsigned char* w = nullptr;
     if (e == hipSuccess) e = dalloc(*pl, &w, pl->work_bytes);
@@ -389,7 +378,10 @@ int sg_plan_describe(const sg_plan* plan, char* text, int32_t capacity) {
   tiling("fwd", pl.fwd);
   tiling("mma", pl.mma);
   const char* slow = (pl.stream_ok && pl.adj.n_tiles1 > 0) ? "stream" : "csr";
-  os << "adjoint=" << (pl.adjm.n_tiles1 > 0 ? "mma_f32+" : "") << slow << " ";
+  const bool mma = pl.adjm.n_tiles1 > 0;
+  os << "adjoint=" << (mma ? "mma_f32" : slow);
+  if (mma) os << "+" << (adjoint_mma_shape_ok(pl, SG_F64) ? "mma_f64" : slow);
+  os << " ";
   tiling("adj", pl.adj);
   tiling("adjm", pl.adjm);
   os << "work_bytes=" << pl.work_bytes;
@@ -576,7 +568,7 @@ int sg_evaluate_rational_adjoint(sg_plan* plan, const void* weights, const void*
   if (rc != SG_OK) return rc;
   const Plan& pl = plan->p;
   if (n_control(pl) == 0) return SG_OK;
-  if (!weights || !control_points || !workspace || (!eval && n_samples(pl) > 0))
+  if (!weights || !control_points || (!workspace && need > 0) || (!eval && n_samples(pl) > 0))
     return fail(SG_ERR_INVALID, "null device pointer");
   if (workspace_bytes < need)
     return fail(SG_ERR_INVALID, "workspace too small: " + std::to_string(need) + " bytes needed");
@@ -606,9 +598,8 @@ int sg_evaluate_adjoint(sg_plan* plan, const int32_t* derivative_order, const vo
   DeviceGuard guard(pl.device);
   if (guard.err != hipSuccess) return hip_fail(guard.err, "hipSetDevice");
   if (tier != SG_TIER_NATIVE && n_samples(pl) > 0)
-    return checked(launch_adjoint_mma(pl, tier, derivative_order,
-                                      static_cast<const float*>(eval),
-                                      static_cast<float*>(control_points), accumulate ? 1 : 0,
+    return checked(launch_adjoint_mma(pl, tier, derivative_order, eval, nullptr, control_points,
+                                      dtype, accumulate ? 1 : 0,
                                       static_cast<hipStream_t>(stream)),
                    "adjoint launch");
   return checked(launch_adjoint(pl, derivative_order, eval, control_points, dtype,

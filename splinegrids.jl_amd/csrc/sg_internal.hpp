@@ -18,9 +18,11 @@ namespace sg {
 constexpr int kLanes = 64;
 constexpr int kWaves = 4;               // waves per workgroup
 constexpr int kThreads = kLanes * kWaves;
+constexpr int kCus = 256;               // compute units of an MI355X
 constexpr int kMaxStreamDegree = 5;     // streaming kernels: p1, p2 <= 5
 constexpr int kMaxLds = 64 * 1024;      // LDS bytes one workgroup may claim
 constexpr int kAdjMmaWin = 16;         // matrix-core adjoint: window edge (one MFMA tile)
+constexpr int kGatherRow = 6;          // entries of a gather_table row (sg_plan_host.hpp)
 
 // Workgroup copy of n >= 1 elements of NF sources into LDS:
 // store(f, i, load(f, i)) for f < NF, i < n.  Each thread issues all NF * U
@@ -121,14 +123,11 @@ struct Tiling {
   int xcd_map = 0;            // workgroup numbering, see xcd_logical_block
   // adjoint only: samples of dimension 3 per workgroup and their k3 windows
   int j3_per_block = 1, n_z = 1, w3max = 1;
-  // adjoint gather: for dimension d and control point k, the windows that
-  // hold k, [gptr[d][k], gptr[d][k + 1]) in goff[d], each as the part of the
-  // element offset in the partial buffer that dimension d contributes (the
-  // offsets of the three dimensions and the channel add up)
-  int32_t* gptr[3] = {nullptr, nullptr, nullptr};  // [n_d + 1]
-  long long* goff[3] = {nullptr, nullptr, nullptr};
+  // adjoint gather: gather_table of each dimension, and the most windows that
+  // hold one control point
+  long long* glist[3] = {nullptr, nullptr, nullptr};
+  long long gwindows = 0;
   long long gchan = 0;  // element offset between the channels of a window
-  int gfast = 0;        // window counts small enough for udiv_fast in the gather
   // explicit tile width / chunk height (0: derived from wx, rows_per_wave)
   int tile_w = 0, chunk_h = 0;
   int tile_width() const { return tile_w ? tile_w : kLanes * wx; }
@@ -140,9 +139,7 @@ struct Plan {
   std::vector<DimDev> dims;
   bool stream_ok = false;     // streaming (sum-factorised) kernels apply
   Tiling fwd, adj, mma;
-  Tiling adjm;                // FP32 matrix-core adjoint (n_tiles1 == 0: not used)
-  float* unit_tab = nullptr;  // {1.0f} and {0}: dimension 3 of a 2-D grid for
-  int32_t* unit_span = nullptr;  //   the matrix-core adjoint
+  Tiling adjm;                // matrix-core adjoint (n_tiles1 == 0: not used)
   int nt_stores = 0;          // non-temporal stores of eval
   void* work = nullptr;       // adjoint partial slabs (either adjoint path)
   size_t work_bytes = 0;
@@ -245,20 +242,22 @@ hipError_t launch_adjoint(const Plan& plan, const int32_t* orders,
                           int accumulate, hipStream_t s);
 size_t adjoint_work_bytes(const Plan& plan);
 // Sum the partial windows [unit][w3max][nout][w2][w1] of tiling tl into
-// Pbar (overwrite or accumulate), one thread per control point.
+// Pbar (overwrite or accumulate); with W not
+// null the sum of control point k is multiplied by W[k] (NURBS adjoint).
 hipError_t launch_adjoint_gather(const Plan& plan, const Tiling& tl,
                                  const void* part, void* Pbar, int dtype, int accumulate,
-                                 hipStream_t s);
+                                 hipStream_t s, const void* W = nullptr);
 
 // ---- sg_adjoint_mma.hip ----
-bool adjoint_mma_shape_ok(const Plan& plan);
+bool adjoint_mma_shape_ok(const Plan& plan, int dtype);
 int adjoint_mma_resident_waves(const Plan& plan);  // on the current device
 size_t adjoint_mma_work_bytes(const Plan& plan);
-// scale (native tier only): when not null, ebar is multiplied sample by
-// sample by the field scale[j3][j2][j1], shared by the channels, as it is
-// loaded (the NURBS adjoint's 1 / w(x))
-hipError_t launch_adjoint_mma(const Plan& plan, int tier, const int32_t* orders, const float* ebar,
-                              float* Pbar, int accumulate, hipStream_t s,
-                              const float* scale = nullptr);
+// The adjoint on matrix cores (plan.adjm not empty, shape ok for dtype).
+// Tiers other than native take FP32 arrays.  W not null: the adjoint of the
+// NURBS map in its control points, Pbar_k = w_k [B^T (ebar / w(x))]_k,
+// native tier and derivative order 0 only.
+hipError_t launch_adjoint_mma(const Plan& plan, int tier, const int32_t* orders,
+                              const void* ebar, const void* W, void* Pbar, int dtype,
+                              int accumulate, hipStream_t s);
 
 }  // namespace sg

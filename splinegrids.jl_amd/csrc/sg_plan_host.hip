@@ -2,6 +2,7 @@
 // runtime calls, no kernels.  Built into the library, and on its own under
 // the sanitizers by the CPU test of tests/native/plan_check.cpp.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <numeric>
@@ -111,46 +112,102 @@ size_t mma_lds(const Plan& pl, int nch, int nf) {
          static_cast<size_t>(t.chunk_rows()) * sizeof(int);
 }
 
+bool adjoint_shares_weights(const Plan& pl) {
+  return pl.nurbs && pl.nout > 1 && (pl.nin == 2 || pl.dims[2].p <= kSharedMaxP3);
+}
+
 namespace {
 
 size_t adjoint_lds_min(const Plan& pl) {  // one channel, FP64
   return adjoint_stream_lds(pl, 1, sizeof(double));
 }
 
-// Matrix-core adjoint (FP32): 64-sample tiles along dimension 1 and chunks
-// of 64, 32 or 16 rows along dimension 2 whose band windows fit one 16 x 16
-// MFMA tile; samples of dimension 3 per task chosen so that all tasks (one
-// wave each) are resident at once.  Leaves pl.adjm empty when the bands do
-// not fit.
+// Rows of a wave when `waves` waves of at most `most` rows share a chunk: the
+// chunks of dimension 2 as even as whole rows allow (a last chunk of a few
+// rows would leave most of its workgroup idle).
+void balanced_rows(const Plan& pl, Tiling& t, int most, int waves) {
+  const int m2 = pl.dims[1].m;
+  const int chunks = (m2 + most * waves - 1) / (most * waves);
+  const int rows = (m2 + chunks * waves - 1) / (chunks * waves);
+  t.chunk_h = rows * waves;
+  compute_tiling(pl, t, rows);
+}
+
+// Matrix-core adjoint: tiles of 64 (or 32) samples j1 and workgroups of 4, 2
+// or 1 waves of up to 16 rows j2 (2-D: up to 128) whose band windows fit one
+// 16 x 16 MFMA tile, and runs of samples j3 (see below).  Leaves pl.adjm
+// empty when the bands do not fit.
 void plan_adjoint_mma(Plan& pl, const std::function<int(const Plan&)>& resident_waves) {
   Tiling& t = pl.adjm;
-  t = Tiling();
-  t.tile_w = kLanes;
-  bool fits = false;
-  for (int ch : {64, 32, 16}) {
-    t.chunk_h = ch;
-    compute_tiling(pl, t, ch / kWaves);
-    if (t.w1max > 16) break;
-    if (t.w2max <= 16) {
-      fits = true;
-      break;
+  // workgroups per tile, chunk and run: the channels, or with NURBS weights
+  // the groups of three that share a weight field
+  const long long groups = adjoint_shares_weights(pl) ? (pl.nout + 2) / 3 : pl.nout;
+  const auto fit = [&](int tile, int most) {  // most waves per workgroup that fit
+    t = Tiling();
+    t.tile_w = tile;
+    for (int waves : {4, 2, 1}) {
+      balanced_rows(pl, t, most, waves);
+      if (t.w1max > kAdjMmaWin) return false;
+      if (t.w2max <= kAdjMmaWin) return true;
     }
-  }
-  if (!fits) {
+    t.chunk_h = 16;  // every chunk of a multiple of 16 rows that fits holds these
+    compute_tiling(pl, t, 16);
+    return t.w2max <= kAdjMmaWin;
+  };
+  const int tile = fit(64, 16) ? 64 : fit(32, 16) ? 32 : 0;
+  if (tile == 0) {
     t = Tiling();
     return;
   }
+  if (pl.nin == 2) {
+    // more rows per wave amortise a wave's set-up, as long as every CU keeps
+    // two workgroups and the chunk's window fits
+    const Tiling one = t;
+    if (one.chunk_rows() == 4 * one.rows_per_wave) {
+      for (int most : {128, 64, 32}) {
+        t = Tiling();
+        t.tile_w = tile;
+        balanced_rows(pl, t, most, 4);
+        if (t.w2max <= kAdjMmaWin && groups * t.n_tiles1 * t.n_chunks2 >= 512) break;
+        t = one;
+      }
+    }
+    compute_ztiling(pl, t, 1);
+    return;
+  }
   int j3 = env_int("SG_ADJM_J3", 0);
-  if (j3 <= 0 && pl.nin == 3) {
-    const long long xy = static_cast<long long>(t.n_tiles1) * t.n_chunks2;
-    const long long m3 = pl.dims[2].m;
-    // about one task (wave) per SIMD: with seven row blocks in flight a wave
-    // keeps HBM busy, and fewer, longer tasks leave fewer partial windows to
-    // gather (400 x 400 x 200 samples: 94 us here against 100 us with every
-    // resident slot filled)
-    const long long slots = std::max(resident_waves(pl) / 2, 1);
-    j3 = static_cast<int>(std::max<long long>(1, (xy * m3 + slots - 1) / slots));
-    while (j3 < m3 && xy * ((m3 + j3 - 1) / j3) > slots) ++j3;
+  if (j3 <= 0) {
+    // Runs of j3: the number that minimises a fit to measured times (14
+    // grids of 2 to 805 MB, FP32 and FP64, every run length; the fit picks
+    // within 2 % of the best on average, 7 % at worst).  Few long runs leave
+    // few partial windows; what costs is a last round of workgroups that
+    // leaves CUs idle (400 x 400 x 200 samples: 88 us with 735 workgroups,
+    // 100 us with 588), and less than 32 KB of ebar in flight per CU (one
+    // unit per wave).  A run is never cut so short that not all workgroups
+    // are resident at once.
+    const long long xy = groups * t.n_tiles1 * t.n_chunks2;
+    const int m3 = pl.dims[2].m;
+    const int waves = t.chunk_rows() / t.rows_per_wave;
+    const long long most = std::max<long long>(resident_waves(pl) / waves, 1);
+    const double unit = 16.0 * t.tile_w * 4 * waves, window = t.w1max * t.w2max;
+    const double samples = 1.0 * pl.dims[0].m * pl.dims[1].m * m3;
+    double best = 0.0;
+    for (int runs = 1, last = 0; runs <= m3 && (runs == 1 || xy * runs <= most); ++runs) {
+      const int len = (m3 + runs - 1) / runs, n = (m3 + len - 1) / len;
+      if (len == last) continue;
+      last = len;
+      compute_ztiling(pl, t, len);
+      const double per_cu = static_cast<double>(xy) * n / kCus;
+      const double idle = std::ceil(per_cu) / per_cu - 1.0;
+      const double hungry = std::max(32768.0 / (unit * per_cu) - 1.0, 0.0);
+      const double partial = 1.0 * t.n_tiles1 * t.n_chunks2 * n * t.w3max * window / samples;
+      const double cost = 1.0 * len * n / m3 * (1.0 + 0.2 * idle) * (1.0 + 0.15 * hungry) +
+                          4.0 * partial;
+      if (j3 <= 0 || cost < best) {
+        best = cost;
+        j3 = len;
+      }
+    }
   }
   compute_ztiling(pl, t, j3);
 }
@@ -218,8 +275,10 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
   pl.stream_ok = ok;
   const char* adj_mma_env = std::getenv("SG_ADJ_MMA");  // "0": streaming kernel only
   if (ok && want_adjoint && !(adj_mma_env && std::strcmp(adj_mma_env, "0") == 0) &&
-      adjm_shape_ok)
+      adjm_shape_ok) {
     plan_adjoint_mma(pl, resident_waves);
+    pl.adjm.xcd_map = pl.adj.xcd_map;
+  }
 }
 
 // Gather lists of a tiling whose partial windows are w1 x w2 x w3max per
@@ -257,15 +316,26 @@ GatherLists gather_lists(const Plan& pl, const Tiling& tl, int w1, int w2) {
     g.off[2] = {0};
   }
   g.gchan = plane;
-  // the gather splits a window number f < n1 n2 n3 (per-point counts) into
-  // (i1, i2, i3) with udiv_fast when f * n1 n2 and f12 * n1 stay below 2^32
-  long long nmax[3] = {1, 1, 1};
-  for (int d = 0; d < 3; ++d)
-    for (size_t k = 0; k + 1 < g.ptr[d].size(); ++k)
-      nmax[d] = std::max<long long>(nmax[d], g.ptr[d][k + 1] - g.ptr[d][k]);
-  const long long n12 = nmax[0] * nmax[1];
-  g.gfast = (n12 * n12 * nmax[2] < (1LL << 32) && nmax[0] * n12 < (1LL << 32)) ? 1 : 0;
   return g;
+}
+
+std::vector<long long> gather_table(const GatherLists& g, int d, int& most) {
+  const size_t n = g.ptr[d].size() - 1;
+  std::vector<long long> table(n * kGatherRow, 0);
+  most = 0;
+  for (size_t k = 0; k < n; ++k) {
+    const auto first = g.off[d].begin() + g.ptr[d][k], last = g.off[d].begin() + g.ptr[d][k + 1];
+    const int count = static_cast<int>(last - first);
+    most = std::max(most, count);
+    table[k * kGatherRow] = count;
+    if (count <= kGatherRow - 2) {
+      std::copy(first, last, table.begin() + k * kGatherRow + 2);
+    } else {
+      table[k * kGatherRow + 1] = static_cast<long long>(table.size());
+      table.insert(table.end(), first, last);
+    }
+  }
+  return table;
 }
 
 void band_lists(const DimDev& D, std::vector<int32_t>& ptr, std::vector<int32_t>& js) {

@@ -31,6 +31,11 @@ size_t forward_lds_worst(const Plan& pl, const Tiling& t);
 size_t adjoint_stream_lds(const Plan& pl, int nc, size_t elem);
 // LDS of an MFMA forward launch: nch window channels, nf fields.
 size_t mma_lds(const Plan& pl, int nch, int nf);
+// NURBS adjoint in FP32: three channels share a workgroup and its weight field
+// (else every channel is a workgroup of its own).  Their rings and the
+// field's fit 256 registers, two waves per SIMD, up to p3 = kSharedMaxP3.
+constexpr int kSharedMaxP3 = 2;
+bool adjoint_shares_weights(const Plan& pl);
 // Workgroup numbering of a plan's launches (see xcd_logical_block).
 int default_xcd_map(const Plan& pl);
 
@@ -45,14 +50,18 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
 // For dimension d and control point k, the element offsets (in the partial
 // windows of tiling t, w1 x w2 x t.w3max per channel) of the windows that
 // hold k: ptr[d][k] .. ptr[d][k + 1] index off[d].  gchan: offset between
-// channels; gfast: window counts small enough for udiv_fast in the gather.
+// channels.
 struct GatherLists {
   std::vector<int32_t> ptr[3];
   std::vector<long long> off[3];
   long long gchan = 0;
-  int gfast = 0;
 };
 GatherLists gather_lists(const Plan& pl, const Tiling& t, int w1, int w2);
+// Dimension d's lists as rows of kGatherRow entries, one per control point:
+// the list's length, then the list itself where it fits the row, so that both
+// come from one cache line; a longer list follows the rows, from the index in
+// the row's second entry.  most: the longest list.
+std::vector<long long> gather_table(const GatherLists& g, int d, int& most);
 
 // Transposed band lists of a dimension: the (sample, term) pairs whose band
 // holds control point k, j * (p + 1) + a, in sample order, at

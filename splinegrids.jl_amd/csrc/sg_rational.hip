@@ -4,11 +4,10 @@
 // src/adjoint.jl:57).
 //
 // Adjoint: with the weights fixed R is linear in P, R = B (w P) / w(x), so
-// Pbar_k = w_k [B^T (ebar / w(x))]_k.  FP32 grids on the matrix-core adjoint:
-// 1 / w(x) in one streaming pass (the weight field in registers, as the
-// B-spline forward computes it), then the B-spline adjoint multiplying ebar
-// by it as it loads ebar, then a product.  Otherwise ebar / w(x) is written
-// by that pass and the B-spline adjoint reads it.
+// Pbar_k = w_k [B^T (ebar / w(x))]_k.  Grids on the matrix-core adjoint take
+// one pass over ebar, which forms 1 / w(x) on the matrix cores as ebar
+// arrives (sg_adjoint_mma.hip).  Otherwise ebar / w(x) is written by a
+// streaming pass and the B-spline adjoint reads it.
 //
 // Two passes.  (1) The homogeneous control points (w P_c, w) go through the
 // B-spline forward (launch_forward on a view of the plan without weights and
@@ -389,7 +388,7 @@ void* combine_kernel_k(int k) {
 // ebar / w(x) for every channel in one pass: the forward's tiles over the
 // weights as a one-channel B-spline (stage 1 window of w, the register
 // window over k2), and each row's w(x) divides the row of ebar of every
-// channel as it is read; with E null, the pass writes 1 / w(x) instead.
+// channel as it is read.
 template <typename T>
 struct DivArgs {
   BandSrc<T> src;  // P = the weights, one channel
@@ -466,10 +465,7 @@ __global__ __launch_bounds__(kThreads) void divide_by_weight_field(
 #pragma unroll
     for (int q = 0; q <= P2; ++q) w += bb[q] * V[q];
     const T inv = T(1) / w;
-    if (a.E == nullptr)
-      a.out[o] = inv;
-    else
-      for (int c = 0; c < a.nout; ++c) a.out[o + a.nsamp * c] = a.E[o + a.nsamp * c] * inv;
+    for (int c = 0; c < a.nout; ++c) a.out[o + a.nsamp * c] = a.E[o + a.nsamp * c] * inv;
   }
 }
 
@@ -497,8 +493,8 @@ __global__ void divide_by_field(const T* E, const T* D, T* out, long long nsamp,
     out[i + nsamp * c] = static_cast<T>(static_cast<double>(E[i + nsamp * c]) * inv);
 }
 
-// The one-pass division (or, with E null, 1 / w(x) alone): streaming grids
-// (2-D, 3-D) whose weight window fits; false otherwise.
+// The one-pass division: streaming grids (2-D, 3-D) whose weight window
+// fits; false otherwise.
 template <typename T>
 bool divide_streaming(const Plan& pl, const T* W, const T* E, T* out, hipStream_t s,
                       hipError_t& e) {
@@ -557,6 +553,13 @@ __global__ void weight_products(const T* Q, const T* W, T* Pbar, long long ncp, 
   }
 }
 
+// The whole rational adjoint runs on the matrix-core adjoint.
+bool rational_adjoint_mma(const Plan& pl, int dtype) {
+  for (const DimDev& d : pl.dims)
+    if (d.m == 0) return false;
+  return pl.adjm.n_tiles1 > 0 && adjoint_mma_shape_ok(pl, dtype);
+}
+
 template <typename T>
 hipError_t rational_adjoint(const Plan& pl, const T* W, const T* E, T* Pbar, void* work,
                             int accumulate, hipStream_t s) {
@@ -565,26 +568,17 @@ hipError_t rational_adjoint(const Plan& pl, const T* W, const T* E, T* Pbar, voi
     ncp *= d.n;
     nsamp *= d.m;
   }
+  const int dtype = sizeof(T) == 4 ? SG_F32 : SG_F64;
+  const int32_t zero[SG_MAX_NIN] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (rational_adjoint_mma(pl, dtype))
+    return launch_adjoint_mma(pl, SG_TIER_NATIVE, zero, E, W, Pbar, dtype, accumulate, s);
   // workspace: w(x) [nsamp], ebar / w(x) [nsamp][nout], B^T (ebar / w) [ncp][nout]
   T* D = static_cast<T*>(work);
   T* Et = D + nsamp;
   T* Q = Et + nsamp * pl.nout;
-  const int dtype = sizeof(T) == 4 ? SG_F32 : SG_F64;
-  const int32_t zero[SG_MAX_NIN] = {0, 0, 0, 0, 0, 0, 0, 0};
   hipError_t e = hipSuccess;
   Plan bp = pl;  // a view: the B-spline adjoint of the same dimensions
   bp.nurbs = 0;
-  if constexpr (sizeof(T) == 4) {
-    // 1 / w(x) into D, then the matrix-core adjoint scales ebar as it loads
-    if (nsamp > 0 && pl.adjm.n_tiles1 > 0 && divide_streaming<T>(pl, W, nullptr, D, s, e)) {
-      if (e != hipSuccess) return e;
-      e = launch_adjoint_mma(bp, SG_TIER_NATIVE, zero, E, Q, 0, s, D);
-      if (e != hipSuccess) return e;
-      hipLaunchKernelGGL(weight_products<T>, dim3(static_cast<unsigned>((ncp + 255) / 256)),
-                         dim3(256), 0, s, Q, W, Pbar, ncp, pl.nout, accumulate);
-      return hipGetLastError();
-    }
-  }
   if (nsamp > 0 && !divide_streaming(pl, W, E, Et, s, e)) {
     Plan wp = pl;  // a view: the weights as a one-channel B-spline
     wp.nurbs = 0;
@@ -752,6 +746,7 @@ hipError_t launch_rational(const Plan& pl, int nf, const int32_t* orders, const 
 }
 
 size_t rational_adjoint_workspace_bytes(const Plan& pl, size_t elem) {
+  if (rational_adjoint_mma(pl, elem == sizeof(float) ? SG_F32 : SG_F64)) return 0;
   long long ncp = 1, nsamp = 1;
   for (const DimDev& d : pl.dims) {
     ncp *= d.n;
