@@ -18,7 +18,7 @@ from .control_points import (DefaultControlPoints, LocallyRefinedControlPoints,
                              evaluate_adjoint_control_points_, evaluate_control_points_,
                              obtain, set_unit_cp_grid_)
 from .spline_dimension import SplineDimension, evaluate_dimension_
-from .utils import (colmajor_zeros, current_stream_handle, dtype_code,
+from .utils import (colmajor_strides, colmajor_zeros, current_stream_handle, dtype_code,
                     is_colmajor)
 from .validation import validate_partial_derivatives, validate_spline_grid
 
@@ -49,6 +49,37 @@ class Plan:
                                         ctypes.byref(handle)))
         self.handle = handle
         self.dims = [(s.degree, s.max_derivative_order, s.n_sample_points) for s in dims]
+        self.index = index
+        # shapes and column-major strides of the arrays a call takes (weights:
+        # those of the control points without the channel)
+        cp = tuple(s.n_basis_functions for s in dims) + (int(nout),)
+        ev = tuple(s.n_sample_points for s in dims) + (int(nout),)
+        self.cp_layout = (cp, colmajor_strides(cp))
+        self.eval_layout = (ev, colmajor_strides(ev))
+        self.weight_layout = (cp[:-1], self.cp_layout[1][:-1])
+        self._orders: dict = {}
+
+    def takes(self, t: torch.Tensor, layout, dtype) -> bool:
+        """t is exactly an array of this layout, on the plan's device (False
+        also for some arrays that fit: callers then check in full)."""
+        return (t.shape == layout[0] and t.stride() == layout[1] and t.dtype == dtype
+                and t.device == self.device)
+
+    def orders(self, orders) -> ctypes.Array:
+        """The C array of a tuple of derivative orders, kept per tuple (calls
+        with orders past the dimensions' maximum are refused before this)."""
+        a = self._orders.get(orders)
+        if a is None:
+            a = self._orders[orders] = _lib.i32_array(orders)
+        return a
+
+    def call(self, fn, *args) -> None:
+        """fn(*args, stream) with the plan's device current."""
+        if torch.cuda.current_device() == self.index:
+            _lib.check(fn(*args, current_stream_handle(self.index)))
+        else:
+            with torch.cuda.device(self.index):
+                _lib.check(fn(*args, current_stream_handle(self.index)))
 
     def basis(self, dim: int):
         """(FP64 table (m, p+1, D+1) Fortran order, 1-based sample indices)."""
@@ -143,11 +174,22 @@ class SplineGrid:
     def plan(self) -> Plan:
         """The C-ABI plan of this grid, rebuilt when a dimension has been
         re-evaluated (new sample points or knots) since it was built."""
-        key = self._dims_key()
-        if self._plan is None or self._plan_key != key:
+        plan = self._current_plan()
+        if plan is None:
+            key = self._dims_key()
             self._plan = None
-            self._plan = Plan(self.spline_dimensions, self.Nout, self.is_nurbs, self.device)
+            self._plan = plan = Plan(self.spline_dimensions, self.Nout, self.is_nurbs,
+                                     self.device)
             self._plan_key = key
+        return plan
+
+    def _current_plan(self) -> Optional[Plan]:
+        """The plan, if one is built and no dimension has changed since."""
+        if self._plan is None:
+            return None
+        for s, (i, version) in zip(self.spline_dimensions, self._plan_key):
+            if id(s) != i or s.version != version:
+                return None
         return self._plan
 
     def __repr__(self):
@@ -183,6 +225,27 @@ def _check_array(name: str, t: torch.Tensor, grid: SplineGrid) -> None:
         raise ValueError(f"{name} must be column-major (Julia layout); see reshape_colmajor")
 
 
+def _checked_plan(grid: SplineGrid, P: torch.Tensor, ev: torch.Tensor,
+                  W: Optional[torch.Tensor], dtype) -> Plan:
+    """The grid's plan, once the arrays of a call fit the grid.  Arrays with
+    the plan's own layouts, the usual case, cost three comparisons each; any
+    others are checked one property at a time, with a message for each."""
+    plan = grid._current_plan()
+    if (plan is not None and plan.takes(P, plan.cp_layout, dtype)
+            and plan.takes(ev, plan.eval_layout, dtype)
+            and (W is None or plan.takes(W, plan.weight_layout, dtype))
+            and obtain(grid.control_points).shape == P.shape and grid.eval.shape == ev.shape):
+        return plan
+    assert tuple(P.shape) == tuple(obtain(grid.control_points).shape), \
+        "size(control_points) == size(spline_grid.control_points)"
+    assert tuple(ev.shape) == tuple(grid.eval.shape), "size(eval) == size(spline_grid.eval)"
+    _check_array("control_points", P, grid)
+    _check_array("eval", ev, grid)
+    if W is not None:
+        _check_array("weights", W, grid)
+    return grid.plan()
+
+
 def evaluate_(obj, *, derivative_order=None, control_points=None, eval=None,
               tier: str = "native", synchronize: bool = False) -> None:
     """evaluate!: dispatches like the reference.
@@ -195,36 +258,29 @@ def evaluate_(obj, *, derivative_order=None, control_points=None, eval=None,
       (src/spline_grid.jl:200-230); eval is overwritten.  ``tier`` picks the
       arithmetic of the contraction ("native", "split_f16", "bf16").
     """
-    if isinstance(obj, SplineDimension):
-        evaluate_dimension_(obj)
-        return None
-    if isinstance(obj, DefaultControlPoints) or isinstance(obj, torch.Tensor):
-        return None
-    if isinstance(obj, LocallyRefinedControlPoints):
-        evaluate_control_points_(obj)
-        return None
+    if not isinstance(obj, SplineGrid):
+        if isinstance(obj, SplineDimension):
+            evaluate_dimension_(obj)
+            return None
+        if isinstance(obj, DefaultControlPoints) or isinstance(obj, torch.Tensor):
+            return None
+        if isinstance(obj, LocallyRefinedControlPoints):
+            evaluate_control_points_(obj)
+            return None
     grid: SplineGrid = obj
     orders = _orders(grid, derivative_order)
-    validate_partial_derivatives(grid, orders)
+    if derivative_order is not None:  # orders 0 are always available
+        validate_partial_derivatives(grid, orders)
     P = obtain(grid.control_points if control_points is None else control_points)
     ev = grid.eval if eval is None else eval
-    assert tuple(P.shape) == tuple(obtain(grid.control_points).shape), \
-        "size(control_points) == size(spline_grid.control_points)"
-    assert tuple(ev.shape) == tuple(grid.eval.shape), "size(eval) == size(spline_grid.eval)"
-    _check_array("control_points", P, grid)
-    _check_array("eval", ev, grid)
-    W = grid.weights
-    if W is not None:
-        _check_array("weights", W, grid)
-    plan = grid.plan()
+    W, dtype = grid.weights, grid.dtype
+    plan = _checked_plan(grid, P, ev, W, dtype)
     L = _lib.lib()
-    with torch.cuda.device(grid.device):
-        stream = current_stream_handle(grid.device)
-        _lib.check(L.sg_evaluate(plan.handle, _lib.i32_array(orders), P.data_ptr(),
-                                 None if W is None else W.data_ptr(), ev.data_ptr(),
-                                 dtype_code(grid.dtype), _lib.TIERS[tier], stream))
-        if synchronize:
-            _lib.check(L.sg_stream_synchronize(stream))
+    plan.call(L.sg_evaluate, plan.handle, plan.orders(orders), P.data_ptr(),
+              None if W is None else W.data_ptr(), ev.data_ptr(), dtype_code(dtype),
+              _lib.TIERS[tier])
+    if synchronize:
+        plan.call(L.sg_stream_synchronize)
     return None
 
 
@@ -332,30 +388,25 @@ def evaluate_adjoint_(grid, *, derivative_order=None, control_points=None,
     On a control-point container it is the adjoint of that container's
     evaluate_: nothing for DefaultControlPoints, the reversed THB chain for
     LocallyRefinedControlPoints (src/adjoint.jl:172-205)."""
-    if isinstance(grid, (DefaultControlPoints, torch.Tensor)):
-        return None
-    if isinstance(grid, LocallyRefinedControlPoints):
-        evaluate_adjoint_control_points_(grid)
-        return None
+    if not isinstance(grid, SplineGrid):
+        if isinstance(grid, (DefaultControlPoints, torch.Tensor)):
+            return None
+        if isinstance(grid, LocallyRefinedControlPoints):
+            evaluate_adjoint_control_points_(grid)
+            return None
     assert not grid.is_nurbs, "Adjoint evaluation not supported for NURBS."
     orders = _orders(grid, derivative_order)
-    validate_partial_derivatives(grid.spline_dimensions, orders)
+    if derivative_order is not None:  # orders 0 are always available
+        validate_partial_derivatives(grid.spline_dimensions, orders)
     P = obtain(grid.control_points if control_points is None else control_points)
     ev = grid.eval if eval is None else eval
-    assert tuple(P.shape) == tuple(obtain(grid.control_points).shape), \
-        "size(control_points) == size(spline_grid.control_points)"
-    assert tuple(ev.shape) == tuple(grid.eval.shape), "size(eval) == size(spline_grid.eval)"
-    _check_array("control_points", P, grid)
-    _check_array("eval", ev, grid)
-    plan = grid.plan()
+    dtype = grid.dtype
+    plan = _checked_plan(grid, P, ev, None, dtype)
     L = _lib.lib()
-    with torch.cuda.device(grid.device):
-        stream = current_stream_handle(grid.device)
-        _lib.check(L.sg_evaluate_adjoint(plan.handle, _lib.i32_array(orders), ev.data_ptr(),
-                                         P.data_ptr(), dtype_code(grid.dtype),
-                                         _lib.TIERS[tier], int(bool(accumulate)), stream))
-        if synchronize:
-            _lib.check(L.sg_stream_synchronize(stream))
+    plan.call(L.sg_evaluate_adjoint, plan.handle, plan.orders(orders), ev.data_ptr(),
+              P.data_ptr(), dtype_code(dtype), _lib.TIERS[tier], int(bool(accumulate)))
+    if synchronize:
+        plan.call(L.sg_stream_synchronize)
     return None
 
 

@@ -11,6 +11,8 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from ._lib import SG_F32, SG_F64
+
 _NP_FLOAT = {np.float32: np.float32, np.float64: np.float64,
              torch.float32: np.float32, torch.float64: np.float64,
              "float32": np.float32, "float64": np.float64}
@@ -39,8 +41,6 @@ def torch_float(t):
 
 
 def dtype_code(dtype) -> int:
-    from ._lib import SG_F32, SG_F64
-
     if dtype == torch.float32:
         return SG_F32
     if dtype == torch.float64:
@@ -48,10 +48,18 @@ def dtype_code(dtype) -> int:
     raise TypeError(f"unsupported value type {dtype}; use float32 or float64")
 
 
+def colmajor_strides(shape) -> tuple:
+    """Element strides of a column-major array."""
+    strides, step = [], 1
+    for size in shape:
+        strides.append(step)
+        step *= max(size, 1)
+    return tuple(strides)
+
+
 def colmajor_empty(shape, dtype, device) -> torch.Tensor:
     shape = tuple(int(s) for s in shape)
-    base = torch.empty(shape[::-1], dtype=dtype, device=device)
-    return base.permute(*range(len(shape) - 1, -1, -1))
+    return torch.empty_strided(shape, colmajor_strides(shape), dtype=dtype, device=device)
 
 
 def colmajor_zeros(shape, dtype, device) -> torch.Tensor:
@@ -93,4 +101,7 @@ def to_numpy_colmajor(t: torch.Tensor) -> np.ndarray:
 
 
 def current_stream_handle(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The hipStream_t of torch's current stream on a device (or its index)."""
+    if not isinstance(device, int):
+        device = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(device)
