@@ -196,15 +196,15 @@ int sg_evaluate_adjoint(sg_plan* plan, const int32_t* derivative_order,
 /* synchronize(backend) after a launch (e.g. src/spline_grid.jl:228). */
 int sg_stream_synchronize(void* stream);
 
-/* ---- batches: many independent grids in one persistent launch ----------
+/* ---- batches: many independent grids in one launch ---------------------
  * No counterpart in the reference, which evaluates one grid per evaluate!
  * call; the batch is for callers that hold many small grids (the per-grid
  * loop of evaluate! calls is what it replaces).  Every grid is evaluated
  * with derivative order 0 on FP32 arrays. */
 typedef struct sg_batch sg_batch;
 
-/* Build per-grid FP64 tables and one list of tiles over all grids, sorted
- * largest first; allocates all device memory of the batch. */
+/* Build per-grid FP64 tables and one list of tiles over all grids, costliest
+ * first; allocates all device memory of the batch. */
 int sg_batch_create(const sg_grid_desc* grids, int32_t n_grids, void* stream,
                     sg_batch** batch);
 int sg_batch_destroy(sg_batch* batch);
@@ -214,9 +214,10 @@ int sg_batch_destroy(sg_batch* batch);
 int sg_batch_set_arrays(sg_batch* batch, const void* const* control_points,
                         const void* const* weights, void* const* evals);
 
-/* Enqueue the evaluation of every grid: a small kernel that resets the
- * work-queue counters, then the persistent kernel.  Only kernel launches, so
- * the call can be captured into a hipGraph and replayed.  tier: native, or
+/* Enqueue the evaluation of every grid: one kernel over the tiles of all of
+ * them (the MFMA tiers: after a small one that resets their queues).  Only
+ * kernel launches, so the call can be captured into a hipGraph
+ * and replayed.  tier: native, or
  * split-FP16 / BF16 when every grid of the batch takes the MFMA tiers
  * (SG_ERR_UNSUPPORTED otherwise); each grid then gets the result of its own
  * sg_evaluate with that tier. */
@@ -234,8 +235,8 @@ int sg_batch_evaluate_each(sg_batch* batch, void* stream);
  * retune (SG_ERR_INVALID): autotune first, then capture. */
 int sg_batch_autotune(sg_batch* batch, int32_t reps, void* stream);
 
-/* Totals of the batch: tiles, sample points, grids evaluated by the
- * persistent kernel, and the tuned rows per wave / workgroups per CU. */
+/* Totals of the batch: tiles, sample points, grids evaluated by the batch
+ * kernel, and the rows per wave / workgroups per CU it is tiled for. */
 int sg_batch_info(const sg_batch* batch, int64_t* n_tiles, int64_t* n_samples,
                   int32_t* n_persistent, int32_t* rows_per_wave,
                   int32_t* blocks_per_cu);

@@ -1,8 +1,8 @@
-"""SplineGridBatch: many FP32 grids evaluated by one persistent launch.
+"""SplineGridBatch: many FP32 grids evaluated by one launch.
 
 The reference evaluates one grid per evaluate! call; a caller with many
 small grids loops over them.  A batch builds every grid's tables once and
-evaluates all of them with one persistent kernel fed by a device work queue
+evaluates all of them with one kernel, a workgroup per tile of any grid
 (sg_batch_* in include/splinegrids_hip.h).  evaluate_ launches only kernels,
 so it can be captured in a torch.cuda.CUDAGraph and replayed.
 """
@@ -71,7 +71,7 @@ class SplineGridBatch:
         _lib.check(self._lib.sg_batch_set_arrays(self.handle, P, W, E))
 
     def evaluate_(self, tier: str = "native") -> None:
-        """evaluate! of every grid (derivative order 0), one persistent launch."""
+        """evaluate! of every grid (derivative order 0), one launch."""
         with torch.cuda.device(self.device):
             _lib.check(self._lib.sg_batch_evaluate(self.handle, _lib.TIERS[tier],
                                                    current_stream_handle(self.device)))

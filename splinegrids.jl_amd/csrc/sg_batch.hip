@@ -1,18 +1,17 @@
-// sg_batch.hip -- many independent grids in one persistent launch.
+// sg_batch.hip -- many independent grids in one launch.
 //
 // A batch holds one plan (FP64 tables, spans) per grid and a single list of
 // tiles over all grids -- the same tiles as fwd_stream: 64 samples of
 // dimension 1 x a chunk of rows of dimension 2 x one sample of dimension 3
 // -- in one queue per XCD.  Grids are assigned whole to the eight queues,
 // largest first onto the least loaded one, so each grid's control points are
-// fetched into one XCD's L2 rather than into all eight.  A persistent kernel
-// with a few workgroups per CU takes tiles from the queue of its own XCD
-// (workgroups are dispatched to XCDs round-robin, so workgroup b runs on XCD
-// b mod 8) through an atomic counter in global memory, and once that queue
-// is empty from the other queues in turn, so uneven grids still balance
-// across the chip.  The counters are reset by a small kernel before each
-// launch.  Degrees, channel counts, NURBS weights and sizes are per tile at
-// run time; the p2+1 register window is selected by a switch over p2.
+// fetched into one XCD's L2 rather than into all eight; within a queue the
+// grids of costly tiles come first, so that the last tiles to start are short
+// (256 uneven grids: 215 -> 206 us).  One kernel covers every queue, a
+// workgroup per tile (workgroups are dispatched to XCDs round-robin, so
+// workgroup b runs on XCD b mod 8).  Degrees, channel counts, NURBS weights
+// and sizes are per tile at run time; the p2+1 register window is selected by
+// a switch over p2.
 #include <algorithm>
 #include <numeric>
 #include <cstring>
@@ -461,46 +460,36 @@ __device__ __attribute__((always_inline)) void batch_tile_p2(const BGrid& g, con
   }
 }
 
+// Workgroup b takes tile b / 8 of queue b mod 8 (the queue of its XCD), the
+// queues' costliest tiles first; those past a queue's end leave at once.
+// One tile per workgroup: a workgroup that goes on to another tile waits, at
+// that tile's first load, for every store of the one before it (loads and
+// stores share a counter), while one that ends leaves its stores to drain.
+// 256 uneven grids, 500 MB: 198 us with four workgroups per CU taking tiles
+// from the queues in turn, 183 like this; 100 grids 99 and 84 us; 16 grids 41
+// and 23 us.  Bound: latency and VALU of the tiles (window staging alone 66
+// us, rows without their stores 60 us, the stores 73 us).
 // At most 128 VGPRs (four waves per SIMD): the row loop keeps a window
 // column's LDS reads in flight together and the row tables in registers,
 // which outweighs the residency of six workgroups per CU.
-__global__ __launch_bounds__(kThreads, 4) void batch_persistent(const BGrid* __restrict__ grids,
-                                                             const BTile* __restrict__ tiles,
-                                                             int* counters) {
+__global__ __launch_bounds__(kThreads, 4) void batch_tiles(const BGrid* __restrict__ grids,
+                                                        const BTile* __restrict__ tiles,
+                                                        const int* __restrict__ queues) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   float* smem = reinterpret_cast<float*>(smem_raw);
-  __shared__ int s_tile[2];
   const int lane = threadIdx.x & (kLanes - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
-  const int home = static_cast<int>(blockIdx.x) % kXcds;
-  int visited = 0;  // thread 0: queues found empty so far
-  int slot = 0;     // s_tile[slot]: the tile to take next
-  if (threadIdx.x == 0) s_tile[0] = pop_tile(counters, home, visited);
-  for (;;) {
-    __syncthreads();
-    // every thread read the same value: the exit is uniform, and with the
-    // index in a scalar register the tile and grid records are scalar loads
-    // (branches on them stay scalar branches)
-    const int ti = wave_uniform(s_tile[slot]);
-    if (ti < 0) break;
-    // thread 0 claims the following tile now and publishes it once this one
-    // is done, so the queue's atomic round trip overlaps this tile's work
-    int next = -1;
-    if (threadIdx.x == 0) next = pop_tile(counters, home, visited);
-    const BTile t = tiles[ti];
-    const BGrid g = grids[wave_uniform(t.grid)];
-    switch (g.p1) {
-      case 0: batch_tile_p2<0>(g, t, smem, lane, wave); break;
-      case 1: batch_tile_p2<1>(g, t, smem, lane, wave); break;
-      case 2: batch_tile_p2<2>(g, t, smem, lane, wave); break;
-      case 3: batch_tile_p2<3>(g, t, smem, lane, wave); break;
-      case 4: batch_tile_p2<4>(g, t, smem, lane, wave); break;
-      default: batch_tile_p2<5>(g, t, smem, lane, wave); break;
-    }
-    // every thread read s_tile[slot] before the barriers of the tile; the
-    // barrier at the top of the loop publishes the other slot
-    if (threadIdx.x == 0) s_tile[slot ^ 1] = next;
-    slot ^= 1;
+  const int ti = queue_tile(queues);
+  if (ti < 0) return;
+  const BTile t = tiles[ti];
+  const BGrid g = grids[t.grid];
+  switch (g.p1) {
+    case 0: batch_tile_p2<0>(g, t, smem, lane, wave); break;
+    case 1: batch_tile_p2<1>(g, t, smem, lane, wave); break;
+    case 2: batch_tile_p2<2>(g, t, smem, lane, wave); break;
+    case 3: batch_tile_p2<3>(g, t, smem, lane, wave); break;
+    case 4: batch_tile_p2<4>(g, t, smem, lane, wave); break;
+    default: batch_tile_p2<5>(g, t, smem, lane, wave); break;
   }
 }
 
@@ -512,7 +501,7 @@ using namespace sg;
 
 struct sg_batch {
   std::vector<Plan*> plans;       // one per grid
-  std::vector<int> candidates;    // grids the persistent kernel can take
+  std::vector<int> candidates;    // grids the batch kernel can take
   std::vector<int> persistent;    // ... and takes under the current tiling
   std::vector<int> fixed_separate;  // grids that always need their own launch
   std::vector<int> separate;      // grids evaluated with their own launches
@@ -520,7 +509,7 @@ struct sg_batch {
   BGrid* dgrids = nullptr;
   BTile* dtiles = nullptr;
   float* dlists = nullptr;  // plane lists of the 3-D grids' tile rows
-  int* counters = nullptr;  // kQueueInts: queue counters, then queue starts
+  int* counters = nullptr;  // kQueueInts: the queue buffer
   // MFMA tiers: one argument record per (grid, channel block) and their tiles
   // in queues of their own; mma_ok when every grid takes the tiers
   bool mma_ok = false;
@@ -533,6 +522,7 @@ struct sg_batch {
   size_t lds_m = 0;
   std::vector<int> separate_m;  // grids whose windows exceed the tier batch's LDS cap
   int n_tiles = 0;
+  int queue_len = 0;  // tiles of the longest queue
   size_t lds = 0;
   int rows_per_wave = 16;
   int blocks_per_cu = 3;
@@ -601,7 +591,7 @@ hipError_t upload_plane_lists(sg_batch* b, hipStream_t s) {
 // are filled into the records by sg_batch_set_arrays).  Leaves mma_ok false
 // when a grid cannot take the tiers.  A workgroup reserves at most the LDS
 // that lets kMmaBatchPerCu of them share a CU; grids whose windows need more
-// are evaluated with their own tier launches after the persistent one.
+// are evaluated with their own tier launches after the batch's.
 constexpr int kMmaBatchPerCu = 4;
 
 int build_mma_tiles(sg_batch* b) {
@@ -673,7 +663,7 @@ int build_mma_tiles(sg_batch* b) {
   return SG_OK;
 }
 
-// Tiles of every persistent grid in one queue per XCD.  Each grid takes the
+// Tiles of every grid the kernel takes in one queue per XCD.  Each grid takes the
 // batch's rows per wave, halved until its tiles fit in the LDS share of one
 // of `blocks_per_cu` workgroups; a grid whose tiles never fit is evaluated
 // with its own launch instead.  Grids go whole to the least loaded queue,
@@ -741,6 +731,7 @@ int build_tiles(sg_batch* b, int rows_per_wave, int blocks_per_cu) {
   if (e != hipSuccess) return hip_fail(e, "batch tile upload");
   b->persistent = persistent;
   b->n_tiles = static_cast<int>(sorted.size());
+  b->queue_len = longest_queue(host_q);
   b->lds = lds;
   b->rows_per_wave = rows_per_wave;
   b->blocks_per_cu = blocks_per_cu;
@@ -748,12 +739,8 @@ int build_tiles(sg_batch* b, int rows_per_wave, int blocks_per_cu) {
 }
 
 hipError_t launch_batch(sg_batch* b, hipStream_t s) {
-  if (b->n_tiles == 0 || !b->counters) return hipSuccess;  // nothing persistent to run
-  hipLaunchKernelGGL(queue_reset, dim3(1), dim3(64), 0, s, b->counters);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int blocks = std::max(1, std::min(b->n_tiles, b->blocks_per_cu * b->n_cu));
-  hipLaunchKernelGGL(batch_persistent, dim3(blocks), dim3(kThreads), b->lds, s, b->dgrids,
+  if (b->n_tiles == 0 || !b->counters) return hipSuccess;  // no tile to run
+  hipLaunchKernelGGL(batch_tiles, dim3(kXcds * b->queue_len), dim3(kThreads), b->lds, s, b->dgrids,
                      b->dtiles, b->counters);
   return hipGetLastError();
 }
@@ -835,7 +822,9 @@ int sg_batch_create(const sg_grid_desc* grids, int32_t n_grids, void* stream, sg
     if (e != hipSuccess) return bail(hip_fail(e, "batch allocation"));
   }
   if ((e = upload_plane_lists(b, s)) != hipSuccess) return bail(hip_fail(e, "batch plane lists"));
-  int rc = build_tiles(b, 16, 3);
+  std::vector<const Plan*> taken;
+  for (int i : b->candidates) taken.push_back(b->plans[i]);
+  int rc = build_tiles(b, batch_default_rows(taken, b->n_cu), kBatchPerCu);
   if (rc != SG_OK) return bail(rc);
   if (n_grids > 0 && (rc = build_mma_tiles(b)) != SG_OK) return bail(rc);
   if (n_grids == 0) b->mma_ok = true;  // nothing to evaluate in any tier
@@ -1031,7 +1020,7 @@ int sg_batch_describe(const sg_batch* b, char* text, int32_t capacity) {
   if (!b || !text || capacity < 1) return fail(SG_ERR_INVALID, "NULL argument");
   int resident = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &resident, reinterpret_cast<const void*>(batch_persistent), kThreads, b->lds) !=
+          &resident, reinterpret_cast<const void*>(batch_tiles), kThreads, b->lds) !=
       hipSuccess)
     resident = -1;
   std::ostringstream os;

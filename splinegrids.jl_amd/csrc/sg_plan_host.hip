@@ -349,7 +349,7 @@ void band_lists(const DimDev& D, std::vector<int32_t>& ptr, std::vector<int32_t>
     for (int a = 0; a <= D.p; ++a) js[fill[D.h_span[j] - D.p + a]++] = j * (D.p + 1) + a;
 }
 
-// LDS of one CU; a persistent launch of `bpc` workgroups per CU gives each
+// LDS of one CU; a launch meant to keep `bpc` workgroups per CU gives each
 // at most a bpc-th of it, or fewer workgroups than asked are resident.
 constexpr size_t kLdsPerCu = 160 * 1024;
 
@@ -400,6 +400,17 @@ GridTiling batch_grid_tiling(const Plan& pl, int rows_per_wave, size_t cap) {
   return t2.lds <= cap ? t2 : t1;
 }
 
+int batch_default_rows(const std::vector<const Plan*>& plans, int cus) {
+  long long tiles = 0;  // at 16 rows
+  for (const Plan* pl : plans) {
+    const GridTiling t = batch_grid_tiling(*pl, 16, lds_cap(kBatchPerCu));
+    const int nz = pl->nin == 3 ? (pl->dims[2].m + kWaves - 1) / kWaves : 1;
+    tiles += static_cast<long long>(t.ntx) * t.nty * nz;
+  }
+  const long long slots = static_cast<long long>(kBatchPerCu) * cus;
+  return tiles < slots ? 8 : tiles < 6 * slots ? 16 : 32;
+}
+
 int plane_list_host(const int32_t* span3, const float* tab3, int p3, int j3_0, int planes,
                     float* list) {
   const int cap = plane_list_floats(p3);
@@ -437,6 +448,14 @@ void pack_queues(const std::vector<std::vector<BTile>>& grid_tiles,
     load[q] += grid_cost[g];
     queue_grids[q].push_back(g);
   }
+  // a queue hands out its grids of costly tiles first, so that the last tiles
+  // to start are short
+  const auto tile_cost = [&](size_t g) {
+    return static_cast<double>(grid_cost[g]) / std::max<size_t>(1, grid_tiles[g].size());
+  };
+  for (std::vector<size_t>& q : queue_grids)
+    std::stable_sort(q.begin(), q.end(),
+                     [&](size_t a, size_t c) { return tile_cost(a) > tile_cost(c); });
   sorted.clear();
   std::fill(host_q, host_q + kQueueInts, 0);
   int* start = host_q + kXcds * kQueueStride;

@@ -68,7 +68,7 @@ std::vector<long long> gather_table(const GatherLists& g, int d, int& most);
 // js[ptr[k] .. ptr[k + 1]).
 void band_lists(const DimDev& D, std::vector<int32_t>& ptr, std::vector<int32_t>& js);
 
-// ---- the batch's persistent launch (sg_batch.hip) ----
+// ---- the batch's launch (sg_batch.hip) ----
 
 constexpr int kBC = 4;  // value channels per pass; the weight is slab 4
 // 3-D tiles' plane list: entries of kEntry floats, weights then k3 at
@@ -118,6 +118,16 @@ GridTiling grid_tiling(const Plan& pl, int rows, int vec = 1);
 // rows (on C5 that beats one sample per lane even with fewer rows), else
 // one.  lds > cap when nothing fits (the grid then needs its own launch).
 GridTiling batch_grid_tiling(const Plan& pl, int rows_per_wave, size_t cap);
+
+// Workgroups per CU a batch is tiled for (its LDS share; the kernel's 128
+// registers allow four waves per SIMD), and its rows per wave by the number of
+// tiles that 16 rows give: 8 below one tile per resident workgroup (16 grids,
+// 256 tiles: 26.4 us with 16 rows, 23.1 with 8), 32 from six on, where the
+// window staging weighs more than the last tiles (256 grids, 7 681 tiles:
+// 214 and 194 us; 1024 grids: 745 and 697 us), else 16 (64 grids, 1 878 tiles:
+// 55.3, 51.5, 54.7 us with 8, 16, 32; 180 grids, 5 207 tiles: 151, 143, 142).
+constexpr int kBatchPerCu = 4;
+int batch_default_rows(const std::vector<const Plan*>& plans, int cus);
 
 // The queues of a tile list: grids go whole to the least loaded queue,
 // largest first; a queue holds its grids in that order.  Writes the tiles in

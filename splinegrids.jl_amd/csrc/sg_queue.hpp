@@ -1,11 +1,14 @@
 // sg_queue.hpp -- device work queues of the batched launches.
 //
 // A batch's tiles sit in one queue per XCD: queue q holds tiles[start[q] ..
-// start[q + 1]) and is drained through the atomic counter
-// counters[q * kQueueStride] (one 256-byte line each); start[] is stored
-// after the counters.  Workgroup b of a persistent launch runs on XCD b mod 8
-// (workgroups are dispatched to the XCDs round-robin), takes tiles from that
-// XCD's queue first and then from the other queues in turn.
+// start[q + 1]); start[] is stored after one counter per queue.  Workgroup b
+// of a launch runs on XCD b mod 8 (workgroups are dispatched to the XCDs
+// round-robin).  The native batch takes one tile per workgroup (queue_tile).
+// The MFMA tiers, whose tiles are several times as many and shorter, run
+// persistent workgroups that drain the queues through the atomic counters
+// counters[q * kQueueStride] (one 256-byte line each), that of their XCD first
+// and then the others in turn (1024 grids: 1.69 ms, with a workgroup per tile
+// 1.80 ms).
 #pragma once
 
 #include "sg_internal.hpp"
@@ -20,6 +23,23 @@ struct BTile {
 
 constexpr int kQueueStride = 64;
 constexpr int kQueueInts = kXcds * kQueueStride + kXcds + 1;
+
+// The tile of this workgroup, or -1 past the end of its queue.
+__device__ inline int queue_tile(const int* __restrict__ queues) {
+  const int* start = queues + kXcds * kQueueStride;
+  const int q = static_cast<int>(blockIdx.x) % kXcds;
+  const int i = start[q] + static_cast<int>(blockIdx.x) / kXcds;
+  return i < start[q + 1] ? i : -1;
+}
+
+// Tiles of the longest queue: queue_tile's launch takes kXcds times as many
+// workgroups.
+inline int longest_queue(const int* host_q) {
+  const int* start = host_q + kXcds * kQueueStride;
+  int most = 0;
+  for (int q = 0; q < kXcds; ++q) most = start[q + 1] - start[q] > most ? start[q + 1] - start[q] : most;
+  return most;
+}
 
 namespace {
 
