@@ -375,7 +375,8 @@ int sg_plan_describe(const sg_plan* plan, char* text, int32_t capacity) {
        << t.w2max << "x" << t.w3max << " ";
   };
   os << "forward=" << (pl.stream_ok ? "stream" : "direct") << " ";
-  tiling("fwd", pl.fwd);
+  tiling("fwd", pl.fwd[0]);
+  tiling("fwd_f64", pl.fwd[1]);
   tiling("mma", pl.mma);
   const char* slow = (pl.stream_ok && pl.adj.n_tiles1 > 0) ? "stream" : "csr";
   const bool mma = pl.adjm.n_tiles1 > 0;

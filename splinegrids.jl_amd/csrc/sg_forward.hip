@@ -344,7 +344,7 @@ const double* ktab<double>(const DimDev& d, int order) {
 
 // LDS of fwd_stream: the band window G of nc (+1 weight) channels.
 size_t fwd_stream_lds(const Plan& pl, int nc, size_t elem) {
-  const Tiling& t = pl.fwd;
+  const Tiling& t = pl.forward(elem);
   return static_cast<size_t>(nc + (pl.nurbs ? 1 : 0)) * t.w1max * t.w2max * elem;
 }
 
@@ -356,6 +356,7 @@ hipError_t forward_stream(const Plan& pl, int nf, const int32_t* orders,
                           hipStream_t s) {
   const DimDev& d1 = pl.dims[0];
   const DimDev& d2 = pl.dims[1];
+  const Tiling& t = pl.forward(sizeof(T));
   const bool nurbs = pl.nurbs != 0;
   const int nin = pl.nin;
   StreamArgs<T> a{};
@@ -367,11 +368,11 @@ hipError_t forward_stream(const Plan& pl, int nf, const int32_t* orders,
   a.m1 = d1.m;
   a.m2 = d2.m;
   a.p1 = d1.p;
-  a.rows_per_wave = pl.fwd.rows_per_wave;
-  a.wx = pl.fwd.wx;
-  a.ntx = pl.fwd.n_tiles1;
-  a.nty = pl.fwd.n_chunks2;
-  a.xcd_map = pl.fwd.xcd_map;
+  a.rows_per_wave = t.rows_per_wave;
+  a.wx = t.wx;
+  a.ntx = t.n_tiles1;
+  a.nty = t.n_chunks2;
+  a.xcd_map = t.xcd_map;
   a.nt = pl.nt_stores;
   a.src.ncp = 1;
   a.nsamp = 1;
@@ -386,7 +387,7 @@ hipError_t forward_stream(const Plan& pl, int nf, const int32_t* orders,
     a.src.p3 = d3.p;
     gz = static_cast<unsigned>(d3.m);
   }
-  const dim3 grid(pl.fwd.n_tiles1 * pl.fwd.n_chunks2 * gz);
+  const dim3 grid(t.n_tiles1 * t.n_chunks2 * gz);
 
   // Fields that share the dimension-3 order share stage 1; launch each group
   // in blocks of up to 4 fields (B-splines) and each channel block.

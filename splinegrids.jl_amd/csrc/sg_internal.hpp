@@ -138,13 +138,15 @@ struct Plan {
   int nin = 0, nout = 0, nurbs = 0, device = 0;
   std::vector<DimDev> dims;
   bool stream_ok = false;     // streaming (sum-factorised) kernels apply
-  Tiling fwd, adj, mma;
+  Tiling fwd[2];              // forward streaming kernels: FP32, FP64 outputs
+  Tiling adj, mma;
   Tiling adjm;                // matrix-core adjoint (n_tiles1 == 0: not used)
   int nt_stores = 0;          // non-temporal stores of eval
   void* work = nullptr;       // adjoint partial slabs (either adjoint path)
   size_t work_bytes = 0;
   size_t device_bytes = 0;
   std::vector<void*> allocations;
+  const Tiling& forward(size_t elem) const { return fwd[elem == sizeof(double)]; }
 };
 
 // Workgroups are dispatched round-robin over the 8 XCDs of an MI355X, each

@@ -212,6 +212,62 @@ void plan_adjoint_mma(Plan& pl, const std::function<int(const Plan&)>& resident_
   compute_ztiling(pl, t, j3);
 }
 
+// Forward tiles.  What bounds these kernels is the rate of their stores, and
+// that is set by how close together in time the pieces of one line and of one
+// DRAM page are written; so the waves of a workgroup stand side by side along
+// dimension 1 (as many as a row fills to 0.7) and few rows deep:
+//   - rows of whole 64-byte sectors: no sector is shared, the launch order is
+//     kept.  16 rows: 512x512x256, 3 channels, NURBS 145 us (32 rows of one
+//     wave 156); 4096x4096 with derivatives 56 (63).
+//   - other rows: the sector at a tile's edge waits in L2 for its other half,
+//     so workgroups are numbered in contiguous ranges per XCD, and the more
+//     bytes a sample has over the channels the fewer rows pass before that half
+//     comes: 8 rows from 12 bytes on (2-D grids, with fewer rows in all: 16).
+//     300x300x300, 4 channels 98 us (128; 16 rows 130); 1027x1773x20, 3
+//     channels 115 (126); 8001x6001, 3 channels 16 rows 114 (8 rows 129; 171).
+//     Rows of one or two waves' width keep 16 at 12 bytes (33x700x300: 23, 8
+//     rows 29).
+//   - one FP32 channel: a wave writes so little per row that its first columns
+//     (stage 1, first band) weigh more than the stores: 32 rows.  200^3 cubic
+//     20.4 us (25; 16 rows 21.2), 512x512x256 66 (65; 16 rows 82).
+// Small grids take fewer rows, to two workgroups per CU: 1027x773, 3 channels
+// 7.4 us at 8 rows, 7.8 at 16.  (Earlier figures in brackets.)
+struct ForwardShape {
+  int rows = 16, wx = 1, xcd_map = 0;
+};
+
+ForwardShape forward_shape(const Plan& pl, size_t elem) {
+  const DimDev& d1 = pl.dims[0];
+  const int m1 = d1.m, m2 = pl.dims[1].m;
+  const long long m3 = pl.nin == 3 ? pl.dims[2].m : 1;
+  const size_t sample = elem * std::max(pl.nout, 1);
+  ForwardShape s;
+  auto tiles = [&](int wx) { return (m1 + kLanes * wx - 1) / (kLanes * wx); };
+  while (s.wx < kWaves && tiles(s.wx) > 1 &&
+         m1 >= 0.7 * kLanes * 2 * s.wx * tiles(2 * s.wx))
+    s.wx *= 2;
+  auto chunks = [&](int rows) {
+    const int h = rows * (kWaves / s.wx);
+    return (m2 + h - 1) / h;
+  };
+  const bool whole = m1 * elem % 64 == 0;
+  s.xcd_map = whole && sample > sizeof(float) ? 0 : 1;
+  if (sample <= sizeof(float)) {
+    const int h = 32 * (kWaves / s.wx);
+    if (m2 >= 0.8 * h * chunks(32)) s.rows = 32;
+  } else if (!whole && (sample >= 16 || (sample >= 12 && pl.nin == 3 && m1 > 2 * kLanes))) {
+    s.rows = 8;
+  }
+  auto groups = [&](int rows) { return m3 * tiles(s.wx) * chunks(rows); };
+  while (s.rows > 8 && groups(s.rows) < 2 * kCus) s.rows /= 2;
+  while (s.rows < 32 && groups(s.rows) > (1 << 23)) s.rows *= 2;  // grid limit: 2^24
+  s.wx = env_int("SG_FWD_WX", s.wx);
+  if (s.wx != 1 && s.wx != 2 && s.wx != 4) s.wx = 1;
+  s.rows = env_int("SG_FWD_ROWS", s.rows);
+  if (const char* xm = std::getenv("SG_XCD_MAP"); xm && *xm) s.xcd_map = std::atoi(xm);
+  return s;
+}
+
 }  // namespace
 
 void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
@@ -224,22 +280,27 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
   if (ok) {
     const char* xm = std::getenv("SG_XCD_MAP");
     const int xcd = (xm && *xm) ? std::atoi(xm) : default_xcd_map(pl);
-    // forward: one wave per 64 samples of dimension 1; 32 rows per wave when
-    // dimension 2 splits into whole chunks of 128 rows, else 16 (a ragged
-    // last chunk of 32-row waves leaves most of its workgroup idle)
-    int wx = env_int("SG_FWD_WX", 1);
-    if (wx != 1 && wx != 2 && wx != 4) wx = 1;
-    int rows = env_int("SG_FWD_ROWS", pl.dims[1].m % (32 * kWaves) == 0 ? 32 : 16);
-    compute_tiling(pl, pl.fwd, rows, wx);
-    while (forward_lds_worst(pl, pl.fwd) > static_cast<size_t>(kMaxLds) &&
-           (rows > 1 || wx > 1)) {
-      if (wx > 1)
-        wx /= 2;
-      else
-        rows /= 2;
-      compute_tiling(pl, pl.fwd, rows, wx);
+    for (int k = 0; k < 2; ++k) {
+      ForwardShape f = forward_shape(pl, k ? sizeof(double) : sizeof(float));
+      Tiling& fwd = pl.fwd[k];
+      compute_tiling(pl, fwd, f.rows, f.wx);
+      // four windows of one channel: the NURBS gradient's least (two fields of
+      // numerator and denominator), which a wider tile must not push out
+      auto fits = [&]() {
+        const size_t four = 4 * sizeof(double) * fwd.w1max * fwd.w2max;
+        return std::max(forward_lds_worst(pl, fwd), f.wx > 1 ? four : 0) <=
+               static_cast<size_t>(kMaxLds);
+      };
+      while (!fits() && (f.rows > 1 || f.wx > 1)) {
+        if (f.wx > 1)
+          f.wx /= 2;
+        else
+          f.rows /= 2;
+        compute_tiling(pl, fwd, f.rows, f.wx);
+      }
+      fwd.xcd_map = f.xcd_map;
+      ok = ok && forward_lds_worst(pl, fwd) <= static_cast<size_t>(kMaxLds);
     }
-    pl.fwd.xcd_map = xcd;
     // MFMA tiers: 64-sample tiles, each wave 16 samples of dimension 1
     // (LDS: the widest channel block, or four fields of one channel)
     const int mnch = std::max(std::min(pl.nout, 4) + (pl.nurbs ? 1 : 0), 1);
@@ -254,7 +315,6 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
     }
     if (mma_worst() > static_cast<size_t>(kMaxLds)) pl.mma = Tiling();
     pl.mma.xcd_map = xcd;
-    ok = forward_lds_worst(pl, pl.fwd) <= static_cast<size_t>(kMaxLds);
   }
   // adjoint tilings for NURBS plans too: the rational adjoint runs the
   // B-spline adjoint on the same dimensions

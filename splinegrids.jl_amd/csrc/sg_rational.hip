@@ -255,7 +255,7 @@ int rat_grad_channels(const Plan& pl, int nf, const int32_t* orders, size_t elem
     if (total > 1 || seen[kind]++) return 0;
     d3 = d3 || kind == 3;
   }
-  const Tiling& t = pl.fwd;
+  const Tiling& t = pl.forward(elem);
   for (int nc = std::min(kRatGradMaxNC, pl.nout); nc >= 1; --nc) {
     const size_t lds = static_cast<size_t>(d3 ? 2 : 1) * (nc + 1) * t.w1max * t.w2max * elem;
     if (lds <= static_cast<size_t>(kMaxLds)) return nc;
@@ -268,6 +268,7 @@ hipError_t rational_first_order(const Plan& pl, int nf, const int32_t* orders, c
                                 const T* W, T* const* outs, int nc_max, hipStream_t s) {
   const DimDev& d1 = pl.dims[0];
   const DimDev& d2 = pl.dims[1];
+  const Tiling& t = pl.forward(sizeof(T));
   RatGradArgs<T> a{};
   T* out[4] = {nullptr, nullptr, nullptr, nullptr};
   for (int f = 0; f < nf; ++f) {
@@ -286,11 +287,11 @@ hipError_t rational_first_order(const Plan& pl, int nf, const int32_t* orders, c
   a.m1 = d1.m;
   a.m2 = d2.m;
   a.p1 = d1.p;
-  a.rows_per_wave = pl.fwd.rows_per_wave;
-  a.wx = pl.fwd.wx;
-  a.ntx = pl.fwd.n_tiles1;
-  a.nty = pl.fwd.n_chunks2;
-  a.xcd_map = pl.fwd.xcd_map;
+  a.rows_per_wave = t.rows_per_wave;
+  a.wx = t.wx;
+  a.ntx = t.n_tiles1;
+  a.nty = t.n_chunks2;
+  a.xcd_map = t.xcd_map;
   a.nsamp = static_cast<long long>(d1.m) * d2.m;
   // order-1 tables only where a derivative is asked for (D may be 0 elsewhere)
   a.tab1[0] = order_table<T>(d1, 0);
@@ -309,7 +310,7 @@ hipError_t rational_first_order(const Plan& pl, int nf, const int32_t* orders, c
     a.nsamp *= D3.m;
     gz = static_cast<unsigned>(D3.m);
   }
-  const dim3 grid(pl.fwd.n_tiles1 * pl.fwd.n_chunks2 * gz);
+  const dim3 grid(t.n_tiles1 * t.n_chunks2 * gz);
   for (int c0 = 0; c0 < pl.nout; c0 += nc_max) {
     const int nc = std::min(nc_max, pl.nout - c0);
     RatGradKernel<T> k = pl.nin == 2 ? pick_rat_grad_p2<T, 2, false>(d2.p, nc)
@@ -318,8 +319,7 @@ hipError_t rational_first_order(const Plan& pl, int nf, const int32_t* orders, c
     if (!k) return hipErrorInvalidValue;
     a.c0 = c0;
     a.src.c0 = c0;
-    const size_t lds = static_cast<size_t>(d3 ? 2 : 1) * (nc + 1) * pl.fwd.w1max *
-                       pl.fwd.w2max * sizeof(T);
+    const size_t lds = static_cast<size_t>(d3 ? 2 : 1) * (nc + 1) * t.w1max * t.w2max * sizeof(T);
     hipLaunchKernelGGL(k, grid, dim3(kThreads), lds, s, a, d2.span, tb2, tb2d, out[0], out[1],
                        out[2], out[3]);
     const hipError_t e = hipGetLastError();
@@ -499,7 +499,8 @@ template <typename T>
 bool divide_streaming(const Plan& pl, const T* W, const T* E, T* out, hipStream_t s,
                       hipError_t& e) {
   if (!pl.stream_ok || (pl.nin != 2 && pl.nin != 3)) return false;
-  const size_t lds = static_cast<size_t>(pl.fwd.w1max) * pl.fwd.w2max * sizeof(T);
+  const Tiling& t = pl.forward(sizeof(T));
+  const size_t lds = static_cast<size_t>(t.w1max) * t.w2max * sizeof(T);
   if (lds > static_cast<size_t>(kMaxLds)) return false;
   const DimDev& d1 = pl.dims[0];
   const DimDev& d2 = pl.dims[1];
@@ -516,11 +517,11 @@ bool divide_streaming(const Plan& pl, const T* W, const T* E, T* out, hipStream_
   a.m2 = d2.m;
   a.p1 = d1.p;
   a.nout = pl.nout;
-  a.rows_per_wave = pl.fwd.rows_per_wave;
-  a.wx = pl.fwd.wx;
-  a.ntx = pl.fwd.n_tiles1;
-  a.nty = pl.fwd.n_chunks2;
-  a.xcd_map = pl.fwd.xcd_map;
+  a.rows_per_wave = t.rows_per_wave;
+  a.wx = t.wx;
+  a.ntx = t.n_tiles1;
+  a.nty = t.n_chunks2;
+  a.xcd_map = t.xcd_map;
   a.nsamp = static_cast<long long>(d1.m) * d2.m;
   unsigned gz = 1;
   if (pl.nin == 3) {
@@ -534,7 +535,7 @@ bool divide_streaming(const Plan& pl, const T* W, const T* E, T* out, hipStream_
   }
   auto k = pl.nin == 2 ? pick_divide<T, 2>(d2.p) : pick_divide<T, 3>(d2.p);
   if (!k) return false;
-  hipLaunchKernelGGL(k, dim3(pl.fwd.n_tiles1 * pl.fwd.n_chunks2 * gz), dim3(kThreads), lds, s, a,
+  hipLaunchKernelGGL(k, dim3(t.n_tiles1 * t.n_chunks2 * gz), dim3(kThreads), lds, s, a,
                      d2.span, order_table<T>(d2, 0));
   e = hipGetLastError();
   return true;
