@@ -215,18 +215,21 @@ void plan_adjoint_mma(Plan& pl, const std::function<int(const Plan&)>& resident_
 // Forward tiles.  What bounds these kernels is the rate of their stores, and
 // that is set by how close together in time the pieces of one line and of one
 // DRAM page are written; so the waves of a workgroup stand side by side along
-// dimension 1 (as many as a row fills to 0.7) and few rows deep:
-//   - rows of whole 64-byte sectors: no sector is shared, the launch order is
-//     kept.  16 rows: 512x512x256, 3 channels, NURBS 145 us (32 rows of one
+// dimension 1 (unless that leaves over 11 % more of their lanes past the row's
+// end: 439x111x60, 3 channels, four fields 61 us with four, 55 with one), few
+// rows deep:
+//   - rows of whole 64-byte sectors: no sector is shared; the launch order is
+//     kept, or by rows where a 128-byte line is shared.  16 rows: 512x512x256, 3 channels, NURBS 145 us (32 rows of one
 //     wave 156); 4096x4096 with derivatives 56 (63).
 //   - other rows: the sector at a tile's edge waits in L2 for its other half,
-//     so workgroups are numbered in contiguous ranges per XCD, and the more
-//     bytes a sample has over the channels the fewer rows pass before that half
-//     comes: 8 rows from 12 bytes on (2-D grids, with fewer rows in all: 16).
-//     300x300x300, 4 channels 98 us (128; 16 rows 130); 1027x1773x20, 3
-//     channels 115 (126); 8001x6001, 3 channels 16 rows 114 (8 rows 129; 171).
-//     Rows of one or two waves' width keep 16 at 12 bytes (33x700x300: 23, 8
-//     rows 29).
+//     so workgroups are numbered in contiguous ranges per XCD.  16 rows too,
+//     but 8 for volumes of 100 MB and more and of 12 bytes per sample (16 where
+//     two waves span the row): the wider a row of the volume, the fewer rows
+//     may pass before that half comes.  300x300x300, 4 channels 98 us (128; 16
+//     rows 130); 603x301x99, 3 channels 54 (67; 16 rows 60).  Smaller outputs
+//     stay in the last-level cache, where the columns that 8 rows compute
+//     again weigh more (362x32x240, 4 channels: 16.7 us in 8 rows, 14.8);
+//     2-D grids have 16 (8001x6001, 3 channels 114 us, 8 rows 129; 171).
 //   - one FP32 channel: a wave writes so little per row that its first columns
 //     (stage 1, first band) weigh more than the stores: 32 rows.  200^3 cubic
 //     20.4 us (25; 16 rows 21.2), 512x512x256 66 (65; 16 rows 82).
@@ -243,19 +246,19 @@ ForwardShape forward_shape(const Plan& pl, size_t elem) {
   const size_t sample = elem * std::max(pl.nout, 1);
   ForwardShape s;
   auto tiles = [&](int wx) { return (m1 + kLanes * wx - 1) / (kLanes * wx); };
-  while (s.wx < kWaves && tiles(s.wx) > 1 &&
-         m1 >= 0.7 * kLanes * 2 * s.wx * tiles(2 * s.wx))
-    s.wx *= 2;
+  for (int wx : {2, 4})
+    if (tiles(wx / 2) > 1 && tiles(1) >= 0.89 * wx * tiles(wx)) s.wx = wx;
   auto chunks = [&](int rows) {
     const int h = rows * (kWaves / s.wx);
     return (m2 + h - 1) / h;
   };
   const bool whole = m1 * elem % 64 == 0;
-  s.xcd_map = whole && sample > sizeof(float) ? 0 : 1;
+  s.xcd_map = !whole || sample <= sizeof(float) ? 1 : m1 * elem % 128 == 0 ? 0 : 2;
   if (sample <= sizeof(float)) {
     const int h = 32 * (kWaves / s.wx);
     if (m2 >= 0.8 * h * chunks(32)) s.rows = 32;
-  } else if (!whole && (sample >= 16 || (sample >= 12 && pl.nin == 3 && m1 > 2 * kLanes))) {
+  } else if (!whole && pl.nin == 3 && tiles(1) > 1 && sample >= (m1 > 2 * kLanes ? 12 : 16) &&
+             1.0 * m1 * m2 * m3 * sample >= 1e8) {
     s.rows = 8;
   }
   auto groups = [&](int rows) { return m3 * tiles(s.wx) * chunks(rows); };

@@ -18,12 +18,13 @@ CASES = [  # n, p, m, nout, tile FP32, tile FP64
     ((4, 5, 4), (1, 2, 2), (1, 7, 5), 1, "64x32", "64x32"),
     ((9, 8, 6), (2, 3, 1), (45, 33, 30), 2, "64x32", "64x32"),
     ((9, 8, 6), (3, 2, 3), (64, 40, 10), 2, "64x32", "64x32"),
-    ((30, 12, 8), (2, 2, 2), (300, 100, 40), 4, "128x16", "128x16"),
+    ((30, 12, 8), (2, 2, 2), (300, 100, 40), 4, "64x32", "64x32"),
+    ((30, 15, 14), (2, 2, 2), (300, 150, 140), 4, "64x32", "64x32"),
     ((20, 14, 12), (3, 3, 3), (203, 130, 110), 1, "256x32", "256x16"),
-    ((16, 9, 12), (3, 1, 2), (130, 65, 90), 3, "64x32", "64x32"),
-    ((13, 9, 20), (2, 3, 2), (127, 70, 200), 3, "128x32", "128x16"),
-    ((60, 70), (3, 3), (1501, 1700), 3, "256x16", "256x8"),
-    ((40, 30), (2, 4), (1032, 900), 2, "256x8", "256x8"),
+    ((16, 9, 12), (3, 1, 2), (130, 65, 90), 3, "64x64", "64x64"),
+    ((13, 9, 20), (2, 3, 2), (127, 70, 200), 3, "128x32", "128x32"),
+    ((60, 70), (3, 3), (1501, 1700), 3, "256x16", "256x16"),
+    ((40, 30), (2, 4), (1032, 900), 2, "128x16", "128x16"),
 ]
 
 
