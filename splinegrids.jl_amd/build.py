@@ -18,9 +18,9 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libsplinegrids_hip.so")
 # the write-bandwidth probe bench.py --workload ceiling runs (not in the library)
 CEILING = os.path.join(HERE, "store_ceiling")
-SOURCES = ["sg_basis.hip", "sg_forward.hip", "sg_mfma.hip", "sg_adjoint.hip", "sg_adjoint_mma.hip",
-           "sg_batch.hip", "sg_rational.hip", "sg_noalloc.hip", "sg_refine.hip", "sg_plan_host.hip",
-           "sg_api.cpp"]
+SOURCES = ["sg_basis.hip", "sg_forward.hip", "sg_forward_sweep.hip", "sg_mfma.hip",
+           "sg_adjoint.hip", "sg_adjoint_mma.hip", "sg_batch.hip", "sg_rational.hip",
+           "sg_noalloc.hip", "sg_refine.hip", "sg_plan_host.hip", "sg_api.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

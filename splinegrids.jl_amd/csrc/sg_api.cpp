@@ -374,7 +374,8 @@ int sg_plan_describe(const sg_plan* plan, char* text, int32_t capacity) {
        << t.n_tiles1 << "x" << t.n_chunks2 << "x" << t.n_z << ",win=" << t.w1max << "x"
        << t.w2max << "x" << t.w3max << " ";
   };
-  os << "forward=" << (pl.stream_ok ? "stream" : "direct") << " ";
+  os << "forward=" << (pl.sweep[0].threads_x > 0 ? "sweep" : pl.stream_ok ? "stream" : "direct")
+     << " ";
   tiling("fwd", pl.fwd[0]);
   tiling("fwd_f64", pl.fwd[1]);
   tiling("mma", pl.mma);

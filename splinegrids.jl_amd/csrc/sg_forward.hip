@@ -476,6 +476,11 @@ hipError_t launch_forward(const Plan& pl, int nf, const int32_t* orders,
   long long nsamp = 1;
   for (const DimDev& d : pl.dims) nsamp *= d.m;
   if (nsamp == 0) return hipSuccess;
+  // one field of a large scalar volume (plan_sweep); several fields share the
+  // streaming kernel's stage 1 and row loop (75x150x435, four fields: 41 us,
+  // swept one by one 51)
+  if (nf == 1 && pl.nout == 1 && !pl.nurbs && pl.sweep[dtype == SG_F64].threads_x > 0)
+    return launch_forward_sweep(pl, orders, P, outs[0], dtype, s);
   if (dtype == SG_F32) {
     auto o = reinterpret_cast<float* const*>(outs);
     auto p = static_cast<const float*>(P);

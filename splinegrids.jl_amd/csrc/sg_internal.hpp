@@ -134,12 +134,21 @@ struct Tiling {
   int chunk_rows() const { return chunk_h ? chunk_h : rows_per_wave * (kWaves / wx); }
 };
 
+// Tiles of the swept forward (sg_forward_sweep.hip): threads_x threads along
+// dimension 1 times rows of dimension 2, for a run of j3.
+struct Sweep {
+  int threads_x = 0;  // 0: the plan does not sweep
+  int rows = 1, ntx = 0, nty = 0, nz = 0, run = 0, xcd_map = 0;
+  size_t lds_elements = 0;  // control planes of a run x rows x window of dimension 1
+};
+
 struct Plan {
   int nin = 0, nout = 0, nurbs = 0, device = 0;
   std::vector<DimDev> dims;
   bool stream_ok = false;     // streaming (sum-factorised) kernels apply
   Tiling fwd[2];              // forward streaming kernels: FP32, FP64 outputs
   Tiling adj, mma;
+  Sweep sweep[2];             // FP32, FP64
   Tiling adjm;                // matrix-core adjoint (n_tiles1 == 0: not used)
   int nt_stores = 0;          // non-temporal stores of eval
   void* work = nullptr;       // adjoint partial slabs (either adjoint path)
@@ -208,6 +217,12 @@ size_t fwd_stream_lds(const Plan& plan, int nc, size_t elem);
 hipError_t launch_forward(const Plan& plan, int nf, const int32_t* orders,
                           const void* P, const void* W, void* const* outs,
                           int dtype, hipStream_t s);
+
+// ---- sg_forward_sweep.hip ----
+bool forward_sweep_shape_ok(const Plan& plan);
+// One field (orders of its nin dimensions) of a plan that sweeps.
+hipError_t launch_forward_sweep(const Plan& plan, const int32_t* orders, const void* P, void* out,
+                                int dtype, hipStream_t s);
 
 // ---- sg_mfma.hip ----
 bool mma_supported(const Plan& plan);

@@ -271,6 +271,64 @@ ForwardShape forward_shape(const Plan& pl, size_t elem) {
   return s;
 }
 
+// The swept forward's tiles, where it is the faster kernel: one channel, and
+// enough samples to pay for its longer prologue (1.5 M; 115x64x53 is launch
+// time in both).  Runs are as long as leaves two workgroups per CU: 200x200x200
+// 15.5 us in runs of 8 (1000 workgroups), 16.9 in 16, 19.0 in 4.  With two
+// channels the ring takes the registers that hide the prologue (500x500x100:
+// 57.8 us, streamed 46.3; 256x256x200 quartic: 39, 34; 40x700x700: 41, 45), and
+// where stage 1 computes more than 0.75 of the samples' number it is the larger
+// part (200x200x80 of 160x160x64 control points: 35.2, 35.3).
+void plan_sweep(const Plan& pl, size_t elem, Sweep& t) {
+  const DimDev &d1 = pl.dims[0], &d2 = pl.dims[1];
+  if (!forward_sweep_shape_ok(pl) || pl.nt_stores) return;
+  const DimDev& d3 = pl.dims[2];
+  const double samples = 1.0 * d1.m * d2.m * d3.m;
+  if (samples < 1000.0 * env_int("SG_SWEEP_MIN", 1500)) return;  // thousands
+  const int vec = 16 / static_cast<int>(elem);
+  const int across = (d1.m + vec - 1) / vec;  // threads that a row takes
+  const int ntx = (across + kThreads - 1) / kThreads;
+  const int tx = (across + ntx - 1) / ntx;
+  // rows: the tile that leaves the fewest lanes of its waves idle, larger
+  // tiles where that is equal to 2 %
+  int rows = 1;
+  double best = 0.0;
+  for (int r = 1; r * tx <= kThreads && r <= d2.m; ++r) {
+    const int waves = (r * tx + kLanes - 1) / kLanes;
+    const double full = 1.0 * r * tx / (kLanes * waves) + 0.01 * waves;
+    if (full > best + 0.02) {
+      best = full;
+      rows = r;
+    }
+  }
+  const int nty = (d2.m + rows - 1) / rows;
+  int w1 = 0;
+  for (int i = 0; i < ntx; ++i) {
+    const int a = i * tx * vec, b = std::min(a + tx * vec, d1.m) - 1;
+    w1 = std::max(w1, d1.h_span[b] - d1.h_span[a] + d1.p + 1);
+  }
+  for (int run = 16; run >= 4; run /= 2) {
+    const int nz = (d3.m + run - 1) / run;
+    if (run > 4 && 1.0 * ntx * nty * nz < 2 * kCus) continue;
+    int planes = 0;
+    for (int a = 0; a < d3.m; a += run)
+      planes = std::max(planes, d3.h_span[std::min(a + run, d3.m) - 1] - d3.h_span[a] + d3.p + 1);
+    const size_t elements = static_cast<size_t>(planes) * rows * w1;
+    if (elements * elem > static_cast<size_t>(kMaxLds) / 2) continue;
+    if (1.0 * elements > 0.75 * rows * tx * vec * run) continue;
+    if (1.0 * ntx * nty * nz > (1 << 23)) continue;  // grid limit
+    t.threads_x = tx;
+    t.rows = rows;
+    t.ntx = ntx;
+    t.nty = nty;
+    t.run = run;
+    t.nz = nz;
+    t.lds_elements = elements;
+    t.xcd_map = d1.m * elem % 64 == 0 ? 0 : 1;  // as the streaming kernel's rows
+    return;
+  }
+}
+
 }  // namespace
 
 void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
@@ -304,6 +362,8 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
       fwd.xcd_map = f.xcd_map;
       ok = ok && forward_lds_worst(pl, fwd) <= static_cast<size_t>(kMaxLds);
     }
+    for (int k = 0; k < 2; ++k)
+      if (ok) plan_sweep(pl, k ? sizeof(double) : sizeof(float), pl.sweep[k]);
     // MFMA tiers: 64-sample tiles, each wave 16 samples of dimension 1
     // (LDS: the widest channel block, or four fields of one channel)
     const int mnch = std::max(std::min(pl.nout, 4) + (pl.nurbs ? 1 : 0), 1);

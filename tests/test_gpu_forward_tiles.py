@@ -10,7 +10,8 @@ import numpy as np
 import pytest
 
 import oracle as O
-from helpers import TOL, eval_host, make_dims, oracle_dims, random_cp, rel_err
+from helpers import (TOL, clamped_knot_vector, eval_host, make_dims, oracle_dims,
+                     random_cp, rel_err)
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +50,42 @@ def test_forward_tiles_vs_oracle(gpu, case, nurbs, dtype):
     want = O.eval_direct(oracle_dims(dims), P.astype(np.float64),
                          W=W.astype(np.float64) if nurbs else None)
     assert rel_err(eval_host(sg, grid.eval), want) <= TOL[dtype]
+
+
+SWEPT = [  # n, p, m: scalar volumes of 1.5 M samples and more
+    ((60, 9, 30), (1, 2, 1), (517, 33, 90)),     # row tails of 1 sample; the last run is short
+    ((9, 30, 40), (4, 1, 4), (38, 203, 201)),    # many rows per tile, last tile not full
+    ((170, 8, 12), (3, 3, 2), (2051, 19, 40)),   # several tiles per row
+    ((4, 200, 24), (2, 4, 3), (3, 2100, 260)),   # rows shorter than one store
+    ((64, 40, 48), (3, 3, 3), (256, 128, 128)),  # whole tiles
+]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("case", SWEPT, ids=lambda c: f"m{c[2]}p{c[1]}")
+def test_swept_volume_vs_oracle(gpu, case, dtype):
+    """Scalar volumes on the swept kernel, value and mixed derivative; knot
+    lines doubled in dimension 3, so that a span advances by two."""
+    sg = gpu
+    n, p, m = case
+    rng = np.random.default_rng(sum(m))
+    kv3 = clamped_knot_vector(sg, np.linspace(0, 1, n[2] - p[2] - 1 + 2 * (p[2] < 2)), p[2], dtype,
+                              doubled=(2, 3) if p[2] > 1 else ())
+    dims = make_dims(sg, n, p, m, D=[1, 1, 1], dtype=dtype, knot_vectors=[None, None, kv3])
+    grid = sg.SplineGrid(tuple(dims), 1)
+    P = random_cp(rng, n, 1, dtype)
+    grid.control_points.copy_(sg.from_numpy_colmajor(P, grid.dtype, "cuda"))
+    assert "forward=sweep" in grid.plan().describe(), grid.plan().describe()
+    for orders in ((0, 0, 0), (1, 0, 1)):
+        grid.eval.fill_(float("nan"))
+        sg.evaluate_(grid, derivative_order=orders)
+        want = O.eval_direct(oracle_dims(dims), P.astype(np.float64), deriv=orders)
+        assert rel_err(eval_host(sg, grid.eval), want) <= TOL[dtype]
+
+
+def test_small_and_many_channel_volumes_stream(gpu):
+    sg = gpu
+    for n, m, nout in (((9, 9, 9), (64, 64, 64), 1), ((40, 30, 20), (200, 100, 90), 2),
+                       ((100, 100, 90), (120, 120, 110), 1)):
+        grid = sg.SplineGrid(tuple(make_dims(sg, n, (2, 3, 2), m)), nout)
+        assert "forward=stream" in grid.plan().describe(), grid.plan().describe()
