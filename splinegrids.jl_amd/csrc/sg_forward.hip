@@ -340,23 +340,13 @@ const double* ktab<double>(const DimDev& d, int order) {
   return d.ktab64 + static_cast<size_t>(order) * d.m * (d.p + 1);
 }
 
-}  // namespace
-
-// LDS of fwd_stream: the band window G of nc (+1 weight) channels.
-size_t fwd_stream_lds(const Plan& pl, int nc, size_t elem) {
-  const Tiling& t = pl.forward(elem);
-  return static_cast<size_t>(nc + (pl.nurbs ? 1 : 0)) * t.w1max * t.w2max * elem;
-}
-
-namespace {
-
 template <typename T>
 hipError_t forward_stream(const Plan& pl, int nf, const int32_t* orders,
                           const T* P, const T* W, T* const* outs,
                           hipStream_t s) {
   const DimDev& d1 = pl.dims[0];
   const DimDev& d2 = pl.dims[1];
-  const Tiling& t = pl.forward(sizeof(T));
+  const Tiling& t = pl.forward(sizeof(T), nf);
   const bool nurbs = pl.nurbs != 0;
   const int nin = pl.nin;
   StreamArgs<T> a{};
@@ -421,7 +411,8 @@ hipError_t forward_stream(const Plan& pl, int nf, const int32_t* orders,
       if (!k) return hipErrorInvalidValue;
       a.c0 = c0;
       a.src.c0 = c0;
-      const size_t lds = fwd_stream_lds(pl, nc, sizeof(T));
+      // the band window G of nc (+1 weight) channels
+      const size_t lds = static_cast<size_t>(nc + (nurbs ? 1 : 0)) * t.w1max * t.w2max * sizeof(T);
       hipLaunchKernelGGL(k, grid, dim3(kThreads), lds, s, a, d2.span, tab2[0], tab2[1],
                          tab2[2], tab2[3], out[0], out[1], out[2], out[3]);
       hipError_t e = hipGetLastError();

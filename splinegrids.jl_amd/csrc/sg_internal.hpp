@@ -146,7 +146,7 @@ struct Plan {
   int nin = 0, nout = 0, nurbs = 0, device = 0;
   std::vector<DimDev> dims;
   bool stream_ok = false;     // streaming (sum-factorised) kernels apply
-  Tiling fwd[2];              // forward streaming kernels: FP32, FP64 outputs
+  Tiling fwd[2][2];           // forward streaming kernels: [FP32, FP64][one field, several]
   Tiling adj, mma;
   Sweep sweep[2];             // FP32, FP64
   Tiling adjm;                // matrix-core adjoint (n_tiles1 == 0: not used)
@@ -155,7 +155,9 @@ struct Plan {
   size_t work_bytes = 0;
   size_t device_bytes = 0;
   std::vector<void*> allocations;
-  const Tiling& forward(size_t elem) const { return fwd[elem == sizeof(double)]; }
+  const Tiling& forward(size_t elem, int nf = 1) const {
+    return fwd[elem == sizeof(double)][nf > 1];
+  }
 };
 
 // Workgroups are dispatched round-robin over the 8 XCDs of an MI355X, each
@@ -212,7 +214,6 @@ hipError_t launch_copy_f64(const double* in, size_t count, double* out,
                            hipStream_t s);
 
 // ---- sg_forward.hip ----
-size_t fwd_stream_lds(const Plan& plan, int nc, size_t elem);
 // Fields: derivative orders [nf][nin]; one output pointer per field.
 hipError_t launch_forward(const Plan& plan, int nf, const int32_t* orders,
                           const void* P, const void* W, void* const* outs,

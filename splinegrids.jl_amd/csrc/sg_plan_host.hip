@@ -219,8 +219,8 @@ void plan_adjoint_mma(Plan& pl, const std::function<int(const Plan&)>& resident_
 // end: 439x111x60, 3 channels, four fields 61 us with four, 55 with one), few
 // rows deep:
 //   - rows of whole 64-byte sectors: no sector is shared; the launch order is
-//     kept, or by rows where a 128-byte line is shared.  16 rows: 512x512x256, 3 channels, NURBS 145 us (32 rows of one
-//     wave 156); 4096x4096 with derivatives 56 (63).
+//     kept, or by rows where a 128-byte line is shared.  16 rows: 512x512x256,
+//     3 channels, NURBS 145 us (32 rows of one wave 156).
 //   - other rows: the sector at a tile's edge waits in L2 for its other half,
 //     so workgroups are numbered in contiguous ranges per XCD.  16 rows too,
 //     but 8 for volumes of 100 MB and more and of 12 bytes per sample (16 where
@@ -230,20 +230,24 @@ void plan_adjoint_mma(Plan& pl, const std::function<int(const Plan&)>& resident_
 //     stay in the last-level cache, where the columns that 8 rows compute
 //     again weigh more (362x32x240, 4 channels: 16.7 us in 8 rows, 14.8);
 //     2-D grids have 16 (8001x6001, 3 channels 114 us, 8 rows 129; 171).
+//   - several fields in a launch are several streams of stores at one sample
+//     each: 16 rows (4096x4096, four fields 48 us, 52 with the tiles of one
+//     scalar; 203x311x160, 2 channels, four fields 91 us, 8 rows 105; 119).
 //   - one FP32 channel: a wave writes so little per row that its first columns
-//     (stage 1, first band) weigh more than the stores: 32 rows.  200^3 cubic
-//     20.4 us (25; 16 rows 21.2), 512x512x256 66 (65; 16 rows 82).
+//     (stage 1, first band) weigh more than the stores: 32 rows.  3001x3001
+//     14.6 us (16 rows 14.9), 251x250x251 22 (16 rows 26).
 // Small grids take fewer rows, to two workgroups per CU: 1027x773, 3 channels
 // 7.4 us at 8 rows, 7.8 at 16.  (Earlier figures in brackets.)
 struct ForwardShape {
   int rows = 16, wx = 1, xcd_map = 0;
 };
 
-ForwardShape forward_shape(const Plan& pl, size_t elem) {
+ForwardShape forward_shape(const Plan& pl, size_t elem, bool several) {
   const DimDev& d1 = pl.dims[0];
   const int m1 = d1.m, m2 = pl.dims[1].m;
   const long long m3 = pl.nin == 3 ? pl.dims[2].m : 1;
   const size_t sample = elem * std::max(pl.nout, 1);
+  const bool thin = sample <= sizeof(float) && !several;
   ForwardShape s;
   auto tiles = [&](int wx) { return (m1 + kLanes * wx - 1) / (kLanes * wx); };
   for (int wx : {2, 4})
@@ -253,12 +257,12 @@ ForwardShape forward_shape(const Plan& pl, size_t elem) {
     return (m2 + h - 1) / h;
   };
   const bool whole = m1 * elem % 64 == 0;
-  s.xcd_map = !whole || sample <= sizeof(float) ? 1 : m1 * elem % 128 == 0 ? 0 : 2;
-  if (sample <= sizeof(float)) {
+  s.xcd_map = !whole || thin ? 1 : m1 * elem % 128 == 0 ? 0 : 2;
+  if (thin) {
     const int h = 32 * (kWaves / s.wx);
     if (m2 >= 0.8 * h * chunks(32)) s.rows = 32;
-  } else if (!whole && pl.nin == 3 && tiles(1) > 1 && sample >= (m1 > 2 * kLanes ? 12 : 16) &&
-             1.0 * m1 * m2 * m3 * sample >= 1e8) {
+  } else if (!several && !whole && pl.nin == 3 && tiles(1) > 1 &&
+             sample >= (m1 > 2 * kLanes ? 12 : 16) && 1.0 * m1 * m2 * m3 * sample >= 1e8) {
     s.rows = 8;
   }
   auto groups = [&](int rows) { return m3 * tiles(s.wx) * chunks(rows); };
@@ -341,9 +345,9 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
   if (ok) {
     const char* xm = std::getenv("SG_XCD_MAP");
     const int xcd = (xm && *xm) ? std::atoi(xm) : default_xcd_map(pl);
-    for (int k = 0; k < 2; ++k) {
-      ForwardShape f = forward_shape(pl, k ? sizeof(double) : sizeof(float));
-      Tiling& fwd = pl.fwd[k];
+    for (int k = 0; k < 4; ++k) {
+      ForwardShape f = forward_shape(pl, k / 2 ? sizeof(double) : sizeof(float), k % 2 != 0);
+      Tiling& fwd = pl.fwd[k / 2][k % 2];
       compute_tiling(pl, fwd, f.rows, f.wx);
       // four windows of one channel: the NURBS gradient's least (two fields of
       // numerator and denominator), which a wider tile must not push out
