@@ -376,9 +376,9 @@ int sg_plan_describe(const sg_plan* plan, char* text, int32_t capacity) {
   };
   os << "forward=" << (pl.sweep[0].threads_x > 0 ? "sweep" : pl.stream_ok ? "stream" : "direct")
      << " ";
-  tiling("fwd", pl.fwd[0][0]);
-  tiling("fwd_f64", pl.fwd[1][0]);
-  tiling("fields", pl.fwd[0][1]);
+  tiling("fwd", pl.fwd);
+  tiling("fwd_f64", pl.fwd64);
+  tiling("fields", pl.fields);
   tiling("mma", pl.mma);
   const char* slow = (pl.stream_ok && pl.adj.n_tiles1 > 0) ? "stream" : "csr";
   const bool mma = pl.adjm.n_tiles1 > 0;

@@ -214,12 +214,6 @@ hipError_t launch(const Plan& pl, const int32_t* orders, const T* P, T* out, hip
 
 }  // namespace
 
-bool forward_sweep_shape_ok(const Plan& pl) {
-  auto in_range = [](const DimDev& d) { return d.p >= 1 && d.p <= 4; };
-  return pl.nin == 3 && in_range(pl.dims[0]) && in_range(pl.dims[2]) && pl.nout == 1 &&
-         !pl.nurbs;
-}
-
 hipError_t launch_forward_sweep(const Plan& pl, const int32_t* orders, const void* P, void* out,
                                 int dtype, hipStream_t s) {
   if (dtype == SG_F32)

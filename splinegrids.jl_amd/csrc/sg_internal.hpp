@@ -146,7 +146,8 @@ struct Plan {
   int nin = 0, nout = 0, nurbs = 0, device = 0;
   std::vector<DimDev> dims;
   bool stream_ok = false;     // streaming (sum-factorised) kernels apply
-  Tiling fwd[2][2];           // forward streaming kernels: [FP32, FP64][one field, several]
+  Tiling fwd, fwd64;          // forward streaming kernels, FP32 and FP64: one field
+  Tiling fields, fields64;    //   and launches of several
   Tiling adj, mma;
   Sweep sweep[2];             // FP32, FP64
   Tiling adjm;                // matrix-core adjoint (n_tiles1 == 0: not used)
@@ -156,7 +157,8 @@ struct Plan {
   size_t device_bytes = 0;
   std::vector<void*> allocations;
   const Tiling& forward(size_t elem, int nf = 1) const {
-    return fwd[elem == sizeof(double)][nf > 1];
+    if (nf > 1) return elem == sizeof(double) ? fields64 : fields;
+    return elem == sizeof(double) ? fwd64 : fwd;
   }
 };
 
@@ -220,7 +222,6 @@ hipError_t launch_forward(const Plan& plan, int nf, const int32_t* orders,
                           int dtype, hipStream_t s);
 
 // ---- sg_forward_sweep.hip ----
-bool forward_sweep_shape_ok(const Plan& plan);
 // One field (orders of its nin dimensions) of a plan that sweeps.
 hipError_t launch_forward_sweep(const Plan& plan, const int32_t* orders, const void* P, void* out,
                                 int dtype, hipStream_t s);

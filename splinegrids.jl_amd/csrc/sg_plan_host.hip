@@ -275,7 +275,8 @@ ForwardShape forward_shape(const Plan& pl, size_t elem, bool several) {
   return s;
 }
 
-// The swept forward's tiles, where it is the faster kernel: one channel, and
+// The swept forward's tiles, where it is the faster kernel: one channel (its
+// kernels take degrees 1 to 4 in dimensions 1 and 3), and
 // enough samples to pay for its longer prologue (1.5 M; 115x64x53 is launch
 // time in both).  Runs are as long as leaves two workgroups per CU: 200x200x200
 // 15.5 us in runs of 8 (1000 workgroups), 16.9 in 16, 19.0 in 4.  With two
@@ -285,7 +286,10 @@ ForwardShape forward_shape(const Plan& pl, size_t elem, bool several) {
 // part (200x200x80 of 160x160x64 control points: 35.2, 35.3).
 void plan_sweep(const Plan& pl, size_t elem, Sweep& t) {
   const DimDev &d1 = pl.dims[0], &d2 = pl.dims[1];
-  if (!forward_sweep_shape_ok(pl) || pl.nt_stores) return;
+  auto in_range = [](const DimDev& d) { return d.p >= 1 && d.p <= 4; };
+  if (pl.nin != 3 || pl.nout != 1 || pl.nurbs || pl.nt_stores || !in_range(d1) ||
+      !in_range(pl.dims[2]))
+    return;
   const DimDev& d3 = pl.dims[2];
   const double samples = 1.0 * d1.m * d2.m * d3.m;
   if (samples < 1000.0 * env_int("SG_SWEEP_MIN", 1500)) return;  // thousands
@@ -345,9 +349,10 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
   if (ok) {
     const char* xm = std::getenv("SG_XCD_MAP");
     const int xcd = (xm && *xm) ? std::atoi(xm) : default_xcd_map(pl);
+    Tiling* const tilings[4] = {&pl.fwd, &pl.fields, &pl.fwd64, &pl.fields64};
     for (int k = 0; k < 4; ++k) {
       ForwardShape f = forward_shape(pl, k / 2 ? sizeof(double) : sizeof(float), k % 2 != 0);
-      Tiling& fwd = pl.fwd[k / 2][k % 2];
+      Tiling& fwd = *tilings[k];
       compute_tiling(pl, fwd, f.rows, f.wx);
       // four windows of one channel: the NURBS gradient's least (two fields of
       // numerator and denominator), which a wider tile must not push out
