@@ -389,10 +389,9 @@ struct AdjCsrArgs {
 // every result is the same sum in the same order on every run.  Each entry
 // is two dependent loads (the list, then the table and ebar), so a lone
 // thread per control point waits through its whole list: G spreads it over
-// a wave or a workgroup (see csr_threads for the choice).  NIN1: curves, the
+// a wave or a workgroup (csr_threads in sg_plan_host.hip chooses).  NIN1: curves, the
 // list of dimension 1 alone, kCsrBatch entries in flight per thread.
 constexpr int kCsrBatch = 4;
-constexpr int kCsrBlock = 1024;  // the widest G: one workgroup per control point
 
 template <typename T, int G, bool NIN1>
 __global__ __launch_bounds__(G > 256 ? G : 256) void adj_csr(AdjCsrArgs<T> a) {
@@ -610,20 +609,6 @@ hipError_t gather(const Plan& pl, const Tiling& tl, const T* part, T* Pbar, int 
   hipLaunchKernelGGL((wide ? adj_gather<T, 4> : adj_gather<T, 1>),
                      dim3(static_cast<unsigned>(planes * g.blocks)), dim3(256), 0, s, g);
   return hipGetLastError();
-}
-
-// Threads per control point of adj_csr, from the mean entries of a list and
-// the outputs (control points times channels).  Short lists keep one thread
-// (20 000 control points x 3 of 40 entries: 15 us, a wave each 20 us).  A
-// wave otherwise (1 600 outputs of 150 entries: 31 -> 14 us; 131 072 of 410:
-// 562 -> 320 us), and a workgroup where the lists are long, sooner when the
-// outputs alone leave CUs empty (20 outputs of 8 000: a thread 1 167 us, a
-// wave 25 us, a workgroup 16 us; 1 296 of 1 296: 6 065 / 91 / 33 us; but
-// 3 200 of 1 600: 1 320 / 30 / 54 us).
-int csr_threads(long long outputs, double entries) {
-  if (entries <= 48.0) return 1;
-  if (entries > 64.0 * kLanes || (entries > 16.0 * kLanes && outputs <= 2048)) return kCsrBlock;
-  return kLanes;
 }
 
 template <typename T>

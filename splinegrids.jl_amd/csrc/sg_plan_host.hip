@@ -481,6 +481,21 @@ void band_lists(const DimDev& D, std::vector<int32_t>& ptr, std::vector<int32_t>
     for (int a = 0; a <= D.p; ++a) js[fill[D.h_span[j] - D.p + a]++] = j * (D.p + 1) + a;
 }
 
+// Short lists keep one thread (20 000 control points x 3 of 40 entries: 15 us,
+// a wave each 20 us).  A wave otherwise (1 600 outputs of 150 entries: 31 -> 14
+// us; 131 072 of 410: 562 -> 320 us), and a workgroup where the lists are long,
+// sooner when the outputs alone leave CUs empty (20 outputs of 8 000: a thread
+// 1 167 us, a wave 25 us, a workgroup 16 us; 1 296 of 1 296: 6 065 / 91 / 33
+// us; but 3 200 of 1 600: 1 320 / 30 / 54 us) -- and fewer threads where so
+// many outputs would pass the threads of a launch: they fill the chip anyway.
+int csr_threads(long long outputs, double entries) {
+  const auto fits = [&](int g) { return outputs <= (kMaxLaunch - kCsrBlock) / g; };
+  if (entries <= 48.0) return 1;
+  if ((entries > 64.0 * kLanes || (entries > 16.0 * kLanes && outputs <= 2048)) && fits(kCsrBlock))
+    return kCsrBlock;
+  return fits(kLanes) ? kLanes : 1;
+}
+
 // LDS of one CU; a launch meant to keep `bpc` workgroups per CU gives each
 // at most a bpc-th of it, or fewer workgroups than asked are resident.
 constexpr size_t kLdsPerCu = 160 * 1024;

@@ -36,6 +36,8 @@ size_t mma_lds(const Plan& pl, int nch, int nf);
 // field's fit 256 registers, two waves per SIMD, up to p3 = kSharedMaxP3.
 constexpr int kSharedMaxP3 = 2;
 bool adjoint_shares_weights(const Plan& pl);
+// Threads one launch may have per grid dimension: HIP refuses 2^32 and more.
+constexpr long long kMaxLaunch = (1LL << 32) - 1;
 // Workgroup numbering of a plan's launches (see xcd_logical_block).
 int default_xcd_map(const Plan& pl);
 
@@ -67,6 +69,12 @@ std::vector<long long> gather_table(const GatherLists& g, int d, int& most);
 // holds control point k, j * (p + 1) + a, in sample order, at
 // js[ptr[k] .. ptr[k + 1]).
 void band_lists(const DimDev& D, std::vector<int32_t>& ptr, std::vector<int32_t>& js);
+
+// Threads per control point and channel of the general adjoint (adj_csr): 1,
+// kLanes or kCsrBlock, for `outputs` control points times channels whose band
+// lists have `entries` entries on average.
+constexpr int kCsrBlock = 1024;  // one workgroup per control point
+int csr_threads(long long outputs, double entries);
 
 // ---- the batch's launch (sg_batch.hip) ----
 
