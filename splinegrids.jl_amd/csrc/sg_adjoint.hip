@@ -389,22 +389,26 @@ struct AdjCsrArgs {
 // every result is the same sum in the same order on every run.  Each entry
 // is two dependent loads (the list, then the table and ebar), so a lone
 // thread per control point waits through its whole list: G spreads it over
-// a wave or a workgroup (csr_threads in sg_plan_host.hip chooses).  NIN1: curves, the
-// list of dimension 1 alone, kCsrBatch entries in flight per thread.
+// a wave or a workgroup (csr_threads in sg_plan_host.hip chooses).  NIN = 1:
+// curves, the list of dimension 1 alone, kCsrBatch entries in flight per
+// thread.  G = 1: the lists of NIN dimensions held in registers, the next entry
+// by counting (300 x 300 x 3 control points of 67 entries 57 us, with the
+// digits of the wave's walk in up to 8 dimensions 72).  NIN = 0: a.nin.
 constexpr int kCsrBatch = 4;
 
-template <typename T, int G, bool NIN1>
+template <typename T, int G, int NIN>
 __global__ __launch_bounds__(G > 256 ? G : 256) void adj_csr(AdjCsrArgs<T> a) {
   constexpr int B = G > 256 ? G : 256;
   const long long idx = (static_cast<long long>(blockIdx.x) * B + threadIdx.x) / G;
   const int sub = static_cast<int>(threadIdx.x % G);
   const bool live = idx < a.ncp * a.nout;
+  if (G == 1 && !live) return;
   T sum = T(0);
   if (live) {
     const int c = static_cast<int>(idx / a.ncp);
     long long r = idx - static_cast<long long>(c) * a.ncp;
     const T* E = a.E + a.nsamp * c;
-    if constexpr (NIN1) {
+    if constexpr (NIN == 1) {
       const int e1 = a.ptr[0][r + 1];
       const int32_t* js = a.js[0];
       for (int e0 = a.ptr[0][r] + sub; e0 < e1; e0 += kCsrBatch * G) {
@@ -420,6 +424,40 @@ __global__ __launch_bounds__(G > 256 ? G : 256) void adj_csr(AdjCsrArgs<T> a) {
 #pragma unroll
         for (int u = 0; u < kCsrBatch; ++u)
           if (e0 + u * G < e1) sum += b[u] * v[u];
+      }
+    } else if constexpr (G == 1) {
+      int lo[NIN], hi[NIN], e[NIN];
+      bool empty = false;
+#pragma unroll
+      for (int d = 0; d < NIN; ++d) {
+        const int k = static_cast<int>(r % a.n[d]);
+        r /= a.n[d];
+        lo[d] = a.ptr[d][k];
+        hi[d] = a.ptr[d][k + 1];
+        e[d] = lo[d];
+        empty |= lo[d] >= hi[d];
+      }
+      while (!empty) {
+        T prod = T(1);
+        long long lin = 0;
+#pragma unroll
+        for (int d = 0; d < NIN; ++d) {
+          const int js = a.js[d][e[d]];
+          prod *= a.tab[d][js];
+          lin += static_cast<long long>(js / a.w[d]) * a.sst[d];
+        }
+        sum += prod * E[lin];
+        bool carry = true;
+#pragma unroll
+        for (int d = 0; d < NIN; ++d) {
+          if (carry) {
+            if (++e[d] < hi[d])
+              carry = false;
+            else
+              e[d] = lo[d];
+          }
+        }
+        if (carry) break;
       }
     } else {
       // digits of the thread's next entry and of the step G in the radices
@@ -612,6 +650,23 @@ hipError_t gather(const Plan& pl, const Tiling& tl, const T* part, T* Pbar, int 
 }
 
 template <typename T>
+void (*pick_csr(int g, int nin))(AdjCsrArgs<T>) {
+  if (g == kCsrBlock) return nin == 1 ? adj_csr<T, kCsrBlock, 1> : adj_csr<T, kCsrBlock, 0>;
+  if (g == kLanes) return nin == 1 ? adj_csr<T, kLanes, 1> : adj_csr<T, kLanes, 0>;
+  switch (nin) {
+    case 1: return adj_csr<T, 1, 1>;
+    case 2: return adj_csr<T, 1, 2>;
+    case 3: return adj_csr<T, 1, 3>;
+    case 4: return adj_csr<T, 1, 4>;
+    case 5: return adj_csr<T, 1, 5>;
+    case 6: return adj_csr<T, 1, 6>;
+    case 7: return adj_csr<T, 1, 7>;
+    case 8: return adj_csr<T, 1, 8>;
+  }
+  return nullptr;
+}
+
+template <typename T>
 hipError_t adjoint_csr(const Plan& pl, const int32_t* orders, const T* E,
                        T* Pbar, int accumulate, hipStream_t s) {
   AdjCsrArgs<T> a{};
@@ -640,12 +695,10 @@ hipError_t adjoint_csr(const Plan& pl, const int32_t* orders, const T* E,
     for (const DimDev& dd : pl.dims) len *= static_cast<double>(dd.m) * (dd.p + 1) / dd.n;
     return len;
   }();
-  const int g = csr_threads(total, entries);
+  const int g = csr_threads(total, entries, pl.nin);
   const int block = std::max(g, 256);
-  const bool one = pl.nin == 1;
-  void (*k)(AdjCsrArgs<T>) = g == kCsrBlock ? (one ? adj_csr<T, kCsrBlock, true> : adj_csr<T, kCsrBlock, false>)
-                             : g == kLanes  ? (one ? adj_csr<T, kLanes, true> : adj_csr<T, kLanes, false>)
-                                            : (one ? adj_csr<T, 1, true> : adj_csr<T, 1, false>);
+  void (*k)(AdjCsrArgs<T>) = pick_csr<T>(g, pl.nin);
+  if (!k) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k, dim3(static_cast<unsigned>((total * g + block - 1) / block)), dim3(block),
                      0, s, a);
   return hipGetLastError();

@@ -481,19 +481,26 @@ void band_lists(const DimDev& D, std::vector<int32_t>& ptr, std::vector<int32_t>
     for (int a = 0; a <= D.p; ++a) js[fill[D.h_span[j] - D.p + a]++] = j * (D.p + 1) + a;
 }
 
-// Short lists keep one thread (20 000 control points x 3 of 40 entries: 15 us,
-// a wave each 20 us).  A wave otherwise (1 600 outputs of 150 entries: 31 -> 14
-// us; 131 072 of 410: 562 -> 320 us), and a workgroup where the lists are long,
-// sooner when the outputs alone leave CUs empty (20 outputs of 8 000: a thread
-// 1 167 us, a wave 25 us, a workgroup 16 us; 1 296 of 1 296: 6 065 / 91 / 33
-// us; but 3 200 of 1 600: 1 320 / 30 / 54 us) -- and fewer threads where so
-// many outputs would pass the threads of a launch: they fill the chip anyway.
-int csr_threads(long long outputs, double entries) {
-  const auto fits = [&](int g) { return outputs <= (kMaxLaunch - kCsrBlock) / g; };
-  if (entries <= 48.0) return 1;
-  if ((entries > 64.0 * kLanes || (entries > 16.0 * kLanes && outputs <= 2048)) && fits(kCsrBlock))
-    return kCsrBlock;
-  return fits(kLanes) ? kLanes : 1;
+// One thread each walks short lists, and longer ones the more outputs there
+// are: they fill the chip by themselves, neighbouring threads read neighbouring
+// entries of ebar, and a wave's set-up and its reduction (0.6 to 0.9 ns per
+// output) are not paid.  A wave each overtook a thread at, in entries, on 2-D /
+// 3-D (degree 6) / 4-D (degree 2) grids: 45 / below 30 / below 30 at 50 000
+// outputs, 140 / 75 / 55 at 130 000, 240 / 200 / 120 at 270 000, 250 / 500 / 240
+// to 500 above a million (1.4 M outputs of 52 entries, 4-D: a thread 287 us, a
+// wave 1 386; 265 000 of 252, 3-D: 439 and 365).  Curves take a wave from 48
+// entries at any size: 600 000 outputs of 52, 1 278 and 181 us (a thread's
+// samples lie far from its neighbour's).  A workgroup pays where the lists are
+// long and the outputs few (1 458 outputs of 6 000: a wave 93, a workgroup 45
+// us; 11 858: 224 and 380).  And never more threads than a launch takes.
+int csr_threads(long long outputs, double entries, int nin) {
+  const double most = nin == 1 ? 48.0 : nin == 2 ? 256.0 : 512.0;
+  const double lone = std::max(std::min(outputs / (400.0 * nin), most), 48.0);
+  if (entries <= lone || outputs > (kMaxLaunch - kCsrBlock) / kLanes) return 1;
+  return (entries > 64.0 * kLanes && outputs <= 8192) ||
+                 (entries > 16.0 * kLanes && outputs <= 2048)
+             ? kCsrBlock
+             : kLanes;
 }
 
 // LDS of one CU; a launch meant to keep `bpc` workgroups per CU gives each

@@ -72,9 +72,9 @@ void band_lists(const DimDev& D, std::vector<int32_t>& ptr, std::vector<int32_t>
 
 // Threads per control point and channel of the general adjoint (adj_csr): 1,
 // kLanes or kCsrBlock, for `outputs` control points times channels whose band
-// lists have `entries` entries on average.
+// lists have `entries` entries on average, in nin dimensions.
 constexpr int kCsrBlock = 1024;  // one workgroup per control point
-int csr_threads(long long outputs, double entries);
+int csr_threads(long long outputs, double entries, int nin);
 
 // ---- the batch's launch (sg_batch.hip) ----
 

@@ -25,8 +25,9 @@ void require(bool ok, const std::string& what) {
 void check_csr_limit() {
   const double entries[] = {1, 48, 49, 100, 300, 1000, 1025, 4096, 4097, 6000, 1e5, 1e7};
   for (long long outputs = 1; outputs < (1LL << 32) - 512; outputs = outputs * 9 / 8 + 1)
-    for (double e : entries) {
-      const int g = csr_threads(outputs, e);
+    for (int k = 0; k < 12 * 4; ++k) {
+      const double e = entries[k / 4];
+      const int g = csr_threads(outputs, e, 1 + k % 4);
       require(g == 1 || g == kLanes || g == kCsrBlock, "threads per control point");
       const long long block = g > 256 ? g : 256;
       const long long threads = (outputs * g + block - 1) / block * block;
@@ -35,8 +36,22 @@ void check_csr_limit() {
     }
   // cubic volumes of 120^3 control points x 3 with 4.5 samples per control
   // point and dimension, unsorted; quadratic 4-D grids of 64^4 points x 4
-  require(csr_threads(3LL * 120 * 120 * 120, 18.0 * 18 * 18) == kLanes, "5 million outputs");
-  require(csr_threads(4LL << 24, 81.0) == 1, "67 million outputs");
+  require(csr_threads(3LL * 120 * 120 * 120, 18.0 * 18 * 18, 3) == kLanes, "5 million outputs");
+  require(csr_threads(4LL << 24, 81.0, 4) == 1, "67 million outputs");
+}
+
+// Where many outputs fill the chip a thread walks each list: shapes on which a
+// wave each took two to three times as long.
+void check_csr_many() {
+  require(csr_threads(995328, 52.8, 4) == 1, "24^4 x 3 linear control points");
+  require(csr_threads(270000, 66.7, 2) == 1, "300^2 x 3 control points of degree 6");
+  require(csr_threads(128000, 50.0, 3) == 1, "64 000 x 2 control points of degree 6");
+  // and the waves and workgroups that pay
+  require(csr_threads(600000, 52.0, 1) == kLanes, "a curve of 200 000 x 3 control points");
+  require(csr_threads(131072, 410.0, 3) == kLanes, "131 072 outputs of 410 entries");
+  require(csr_threads(11858, 6000.0, 2) == kLanes, "11 858 outputs of 6 000 entries");
+  require(csr_threads(1458, 6000.0, 2) == kCsrBlock, "1 458 outputs of 6 000 entries");
+  require(csr_threads(20, 8000.0, 1) == kCsrBlock, "20 outputs of 8 000 entries");
 }
 
 }  // namespace
@@ -45,6 +60,8 @@ int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "csr_limit")
     check_csr_limit();
+  else if (name == "csr_many")
+    check_csr_many();
   else
     require(false, "no check named '" + name + "'");
   std::printf("launch_check ok %s\n", name.c_str());
