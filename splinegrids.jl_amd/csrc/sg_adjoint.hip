@@ -296,6 +296,7 @@ struct AdjGatherArgs {
   const long long* lists[3];  // gather_table of each dimension
   int n1, n2, n3;
   int blocks;  // workgroups per (k3, channel) plane of control points
+  int plane0;  // the launch's first plane
   int fast;    // no point is held by 2^20 windows or more
   int accumulate;
   long long ncp, chan;
@@ -316,9 +317,9 @@ constexpr long long kGatherFill = 1 << 16;
 
 template <typename T, int LANES>
 __global__ __launch_bounds__(256) void adj_gather(AdjGatherArgs<T> a) {
-  const int plane = static_cast<int>(blockIdx.x) / a.blocks;
+  const int q = static_cast<int>(blockIdx.x) / a.blocks, plane = a.plane0 + q;
   const int c = plane / a.n3, k3 = plane - c * a.n3;
-  const int t = (static_cast<int>(blockIdx.x) - plane * a.blocks) * 256 + static_cast<int>(threadIdx.x);
+  const int t = (static_cast<int>(blockIdx.x) - q * a.blocks) * 256 + static_cast<int>(threadIdx.x);
   const int n12 = a.n1 * a.n2, sub = t % LANES;
   const bool live = t / LANES < n12;
   const int k12 = min(t / LANES, n12 - 1);  // dead lanes join the butterfly
@@ -644,9 +645,17 @@ hipError_t gather(const Plan& pl, const Tiling& tl, const T* part, T* Pbar, int 
   const bool wide = tl.gwindows > kGatherBatch && g.ncp * pl.nout <= kGatherFill;
   const int lanes = wide ? 4 : 1;
   g.blocks = static_cast<int>((n12 * lanes + 255) / 256);
-  hipLaunchKernelGGL((wide ? adj_gather<T, 4> : adj_gather<T, 1>),
-                     dim3(static_cast<unsigned>(planes * g.blocks)), dim3(256), 0, s, g);
-  return hipGetLastError();
+  // small planes are mostly idle threads: many of them take several launches
+  const long long per = launch_groups(256LL * g.blocks);
+  for (long long p0 = 0; p0 < planes; p0 += per) {
+    g.plane0 = static_cast<int>(p0);
+    const long long blocks = std::min(per, planes - p0) * g.blocks;
+    hipLaunchKernelGGL((wide ? adj_gather<T, 4> : adj_gather<T, 1>),
+                       dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, g);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 template <typename T>

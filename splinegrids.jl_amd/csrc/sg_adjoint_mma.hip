@@ -102,7 +102,7 @@ struct AdjMmaArgs {
   const int32_t* span2;
   const int32_t* span3;
   int m1, m2, m3, p1, p2, n1, n2, n3;
-  int nout;
+  int nout, group0;  // group0: the launch's first group of NC channels
   int rows, chunk, j3_per_block;
   int ntx, nty, nz, w1max, w2max, w3max, xcd_map;
   long long m12, nsamp;
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kThreads, NURBS && sizeof(T) == 8 ? 1 : 2) void adj
   const int by = rest % a.nty;
   rest /= a.nty;
   const int bz = rest % a.nz;
-  const int c0 = rest / a.nz * NC;
+  const int c0 = (a.group0 + rest / a.nz) * NC;
   const int nc = NC == 1 ? 1 : min(NC, a.nout - c0);
   const int j1_0 = bx * 16 * NQ;
   const int r0 = by * a.chunk, r1 = min(r0 + a.chunk, a.m2);
@@ -589,12 +589,19 @@ hipError_t launch_mma(const Plan& pl, int tier, const int32_t* orders, const T* 
   AdjMmaKernel<T> k = pick_adj_mma<T>(pl, tier, nurbs_nc);
   if (!k) return hipErrorInvalidValue;
   const int nw = tl.chunk_rows() / tl.rows_per_wave;
-  const unsigned blocks = static_cast<unsigned>(tl.n_tiles1) * tl.n_chunks2 * tl.n_z *
-                          ((pl.nout + per - 1) / per);
+  const long long blocks = static_cast<long long>(tl.n_tiles1) * tl.n_chunks2 * tl.n_z;
   const size_t lds = nw > 1 ? 2 * static_cast<size_t>(nw) * kSlab * sizeof(T) : 0;
-  hipLaunchKernelGGL(k, dim3(blocks), dim3(nw * kLanes), lds, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  // a plane's tiles are below 2^32 threads by its size (adjoint_mma_shape_ok),
+  // those of every channel need not be
+  const int groups = (pl.nout + per - 1) / per;
+  const int at_once =
+      static_cast<int>(std::min<long long>(launch_groups(blocks * nw * kLanes), groups));
+  for (a.group0 = 0; a.group0 < groups; a.group0 += at_once) {
+    const int n = std::min(at_once, groups - a.group0);
+    hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(blocks * n)), dim3(nw * kLanes), lds, s, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   return launch_adjoint_gather(pl, tl, pl.work, Pbar, sizeof(T) == 4 ? SG_F32 : SG_F64,
                                accumulate, s, W);
 }

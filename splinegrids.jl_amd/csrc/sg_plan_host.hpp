@@ -38,6 +38,10 @@ constexpr int kSharedMaxP3 = 2;
 bool adjoint_shares_weights(const Plan& pl);
 // Threads one launch may have per grid dimension: HIP refuses 2^32 and more.
 constexpr long long kMaxLaunch = (1LL << 32) - 1;
+// Parts of `threads` threads each that one launch takes, at least one.
+inline long long launch_groups(long long threads) {
+  return threads < kMaxLaunch ? kMaxLaunch / threads : 1;
+}
 // Workgroup numbering of a plan's launches (see xcd_logical_block).
 int default_xcd_map(const Plan& pl);
 

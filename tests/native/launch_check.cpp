@@ -54,6 +54,16 @@ void check_csr_many() {
   require(csr_threads(20, 8000.0, 1) == kCsrBlock, "20 outputs of 8 000 entries");
 }
 
+// A launch of launch_groups(t) parts of t threads is below 2^32, and one more
+// part would not be.
+void check_groups() {
+  for (long long t = 64; t < (1LL << 32); t = t * 3 / 2 + 64) {
+    const long long n = launch_groups(t);
+    require(n >= 1 && n * t < (1LL << 32) && (n + 1) * t >= (1LL << 32),
+            "parts of " + std::to_string(t) + " threads");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -62,6 +72,8 @@ int main(int argc, char** argv) {
     check_csr_limit();
   else if (name == "csr_many")
     check_csr_many();
+  else if (name == "groups")
+    check_groups();
   else
     require(false, "no check named '" + name + "'");
   std::printf("launch_check ok %s\n", name.c_str());
