@@ -5,8 +5,9 @@
 // dimension 1 x a chunk of rows of dimension 2 x one sample of dimension 3
 // -- in one queue per XCD.  Grids are assigned whole to the eight queues,
 // largest first onto the least loaded one, so each grid's control points are
-// fetched into one XCD's L2 rather than into all eight; within a queue the
-// grids of costly tiles come first, so that the last tiles to start are short
+// fetched into one XCD's L2 rather than into all eight, and are cut into ranges
+// of tiles only where they would leave the queues uneven; within a queue the
+// costly tiles come first, so that the last to start are short
 // (256 uneven grids: 215 -> 206 us).  One kernel covers every queue, a
 // workgroup per tile (workgroups are dispatched to XCDs round-robin, so
 // workgroup b runs on XCD b mod 8).  Degrees, channel counts, NURBS weights
@@ -666,10 +667,8 @@ int build_mma_tiles(sg_batch* b) {
 // Tiles of every grid the kernel takes in one queue per XCD.  Each grid takes the
 // batch's rows per wave, halved until its tiles fit in the LDS share of one
 // of `blocks_per_cu` workgroups; a grid whose tiles never fit is evaluated
-// with its own launch instead.  Grids go whole to the least loaded queue,
-// largest first (by outputs plus window work); a queue holds its grids in
-// that order, each grid's tiles row by row, so neighbouring tiles share
-// control-point planes in L2.
+// with its own launch instead.  Tiles are listed row by row, so neighbours share
+// control-point planes in L2, and go to the queues by their cost (pack_queues).
 int build_tiles(sg_batch* b, int rows_per_wave, int blocks_per_cu) {
   // the kernel's row tables hold the rows of a wave for at most this many
   if (rows_per_wave < 1 || rows_per_wave > kMaxBatchRows)
@@ -705,7 +704,7 @@ int build_tiles(sg_batch* b, int rows_per_wave, int blocks_per_cu) {
           const long long lanes = std::min(t.tw, d1.m - x * t.tw);
           const long long nrows = std::min(chunk, d2.m - y * chunk);
           const long long planes = pl.nin == 3 ? std::min(kWaves, m3 - z * kWaves) : 1;
-          cost += lanes * nrows * planes * pl.nout + 64LL * planes * t.w1 * t.w2;
+          cost += batch_tile_cost(pl, t, lanes * nrows * planes, planes);
         }
     grid_tiles.push_back(std::move(tiles));
     grid_cost.push_back(cost);

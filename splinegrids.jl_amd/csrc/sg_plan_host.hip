@@ -595,28 +595,47 @@ void pack_queues(const std::vector<std::vector<BTile>>& grid_tiles,
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(),
                    [&](size_t a, size_t c) { return grid_cost[a] > grid_cost[c]; });
-  std::vector<std::vector<size_t>> queue_grids(kXcds);
-  long long load[kXcds] = {};
-  for (size_t g : order) {
-    const int q = static_cast<int>(std::min_element(load, load + kXcds) - load);
-    load[q] += grid_cost[g];
-    queue_grids[q].push_back(g);
-  }
-  // a queue hands out its grids of costly tiles first, so that the last tiles
-  // to start are short
+  struct Piece {  // tiles [first, last) of a grid
+    size_t grid, first, last;
+  };
   const auto tile_cost = [&](size_t g) {
     return static_cast<double>(grid_cost[g]) / std::max<size_t>(1, grid_tiles[g].size());
   };
-  for (std::vector<size_t>& q : queue_grids)
-    std::stable_sort(q.begin(), q.end(),
-                     [&](size_t a, size_t c) { return tile_cost(a) > tile_cost(c); });
+  // What a queue should hold.  A grid that would take the least loaded queue
+  // 1/20 past it is cut into ranges of neighbouring tiles over several.
+  double mean = 0.0;
+  for (size_t g : order) mean += static_cast<double>(grid_cost[g]) / kXcds;
+  std::vector<std::vector<Piece>> queue(kXcds);
+  double load[kXcds] = {};
+  for (size_t g : order) {
+    const size_t n = grid_tiles[g].size();
+    const double each = tile_cost(g);
+    for (size_t first = 0; first < n;) {
+      const int q = static_cast<int>(std::min_element(load, load + kXcds) - load);
+      const double room = mean - load[q];
+      size_t last = n;
+      if (each * static_cast<double>(n - first) > room + 0.05 * mean)
+        last = first + std::min(std::max<size_t>(static_cast<size_t>(std::max(room, 0.0) / each), 1),
+                                n - first);
+      queue[q].push_back(Piece{g, first, last});
+      load[q] += each * static_cast<double>(last - first);
+      first = last;
+    }
+  }
+  // a queue hands out its costly tiles first, so that the last to start are
+  // short
+  for (std::vector<Piece>& q : queue)
+    std::stable_sort(q.begin(), q.end(), [&](const Piece& a, const Piece& c) {
+      return tile_cost(a.grid) > tile_cost(c.grid);
+    });
   sorted.clear();
   std::fill(host_q, host_q + kQueueInts, 0);
   int* start = host_q + kXcds * kQueueStride;
   for (int q = 0; q < kXcds; ++q) {
     start[q] = static_cast<int>(sorted.size());
-    for (size_t g : queue_grids[q])
-      sorted.insert(sorted.end(), grid_tiles[g].begin(), grid_tiles[g].end());
+    for (const Piece& piece : queue[q])
+      sorted.insert(sorted.end(), grid_tiles[piece.grid].begin() + piece.first,
+                    grid_tiles[piece.grid].begin() + piece.last);
   }
   start[kXcds] = static_cast<int>(sorted.size());
 }

@@ -3,9 +3,13 @@
 // address and undefined-behaviour sanitizers: what a launch may ask of the
 // runtime, at sizes no test allocates.  The argument names the check; prints
 // "launch_check ok <name>" and exits 0, or names the first failure.
+#include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <random>
 #include <string>
+#include <vector>
 
 #include "sg_plan_host.hpp"
 
@@ -64,6 +68,119 @@ void check_groups() {
   }
 }
 
+// A plan's host part for clamped uniform knots and uniform samples: the spans.
+Plan make_plan(const std::vector<int>& n, const std::vector<int>& p, const std::vector<int>& m,
+               int nout, bool nurbs) {
+  Plan pl;
+  pl.nin = static_cast<int>(n.size());
+  pl.nout = nout;
+  pl.nurbs = nurbs ? 1 : 0;
+  pl.dims.resize(n.size());
+  for (size_t d = 0; d < n.size(); ++d) {
+    DimDev& D = pl.dims[d];
+    D.n = n[d];
+    D.p = p[d];
+    D.m = m[d];
+    D.h_span.resize(m[d]);
+    const int cells = n[d] - p[d];
+    for (int j = 0; j < m[d]; ++j) {
+      const double t = m[d] > 1 ? static_cast<double>(j) / (m[d] - 1) : 0.0;
+      D.h_span[j] = p[d] + std::min(static_cast<int>(t * cells), cells - 1);
+    }
+  }
+  return pl;
+}
+
+struct Packed {
+  std::vector<BTile> tiles;
+  std::vector<int> q;
+  double longest = 0.0, mean = 0.0;  // queue costs
+  const int* start() const { return q.data() + kXcds * kQueueStride; }
+};
+
+// The queues of a batch at 16 rows; checks that they hold each grid's tiles
+// once, and in each queue as ranges of neighbours.
+Packed pack(const std::vector<Plan>& plans, const std::string& what) {
+  std::vector<std::vector<BTile>> grid_tiles;
+  std::vector<long long> cost;
+  for (size_t g = 0; g < plans.size(); ++g) {
+    const Plan& pl = plans[g];
+    const GridTiling t = batch_grid_tiling(pl, 16, lds_cap(kBatchPerCu));
+    const int nz = pl.nin == 3 ? (pl.dims[2].m + kWaves - 1) / kWaves : 1;
+    std::vector<BTile> tiles;
+    long long sum = 0;
+    for (int z = 0; z < nz; ++z)
+      for (int y = 0; y < t.nty; ++y)
+        for (int x = 0; x < t.ntx; ++x) {
+          tiles.push_back(BTile{static_cast<int>(g), x, y, z});
+          sum += batch_tile_cost(pl, t, 64LL * 64 * (pl.nin == 3 ? kWaves : 1), pl.nin == 3 ? kWaves : 1);
+        }
+    grid_tiles.push_back(tiles);
+    cost.push_back(sum);
+  }
+  Packed out;
+  out.q.assign(kQueueInts, -1);
+  pack_queues(grid_tiles, cost, out.tiles, out.q.data());
+  std::vector<size_t> held(plans.size(), 0);
+  for (int q = 0; q < kXcds; ++q) {
+    double load = 0.0;
+    std::vector<char> seen(plans.size(), 0);
+    for (int i = out.start()[q]; i < out.start()[q + 1]; ++i) {
+      const BTile& t = out.tiles[i];
+      const std::vector<BTile>& of = grid_tiles[t.grid];
+      load += static_cast<double>(cost[t.grid]) / of.size();
+      ++held[t.grid];
+      if (i > out.start()[q] && out.tiles[i - 1].grid == t.grid) {
+        const Plan& pl = plans[t.grid];
+        const GridTiling gt = batch_grid_tiling(pl, 16, lds_cap(kBatchPerCu));
+        const auto at = [&](const BTile& b) { return (static_cast<long long>(b.bz) * gt.nty + b.by) * gt.ntx + b.bx; };
+        require(at(t) > at(out.tiles[i - 1]), what + ": tiles in order");
+      } else {
+        require(!seen[t.grid], what + ": a queue holds one range of a grid");
+        seen[t.grid] = 1;
+      }
+    }
+    out.longest = std::max(out.longest, load);
+    out.mean += load / kXcds;
+  }
+  for (size_t g = 0; g < plans.size(); ++g)
+    require(held[g] == grid_tiles[g].size(), what + ": every tile once");
+  return out;
+}
+
+// No workgroup takes a tile of another XCD's queue, so the queues themselves
+// have to be even: single grids, a large one among small ones, uneven ones.
+void check_queues() {
+  std::mt19937_64 rng(0x0DD);
+  const auto pick = [&](int a, int b) { return std::uniform_int_distribution<int>(a, b)(rng); };
+  const auto even = [&](const std::vector<Plan>& plans, const std::string& what) {
+    const Packed q = pack(plans, what);
+    if (q.tiles.size() < 32 * kXcds) return;  // a tile is more than 1/32 of a queue
+    require(q.longest <= 1.1 * q.mean, what + ": longest queue " + std::to_string(q.longest / q.mean) +
+                                           " of the mean");
+  };
+  even({make_plan({40, 40, 20}, {3, 3, 2}, {256, 255, 200}, 3, false)}, "one volume");
+  even({make_plan({64, 64}, {3, 3}, {2000, 1500}, 3, true)}, "one surface");
+  for (int count : {1, 2, 3, 4, 8, 9, 16, 32, 64, 256})
+    for (int rep = 0; rep < 20; ++rep) {
+      std::vector<Plan> plans;
+      for (int i = 0; i < count; ++i) {
+        const int nin = i < count / 2 ? 2 : 3;
+        std::vector<int> n, p, m;
+        for (int d = 0; d < nin; ++d) {
+          n.push_back(pick(8, 64));
+          p.push_back(pick(1, 4));
+          m.push_back(nin == 2 ? pick(32, 512) : pick(16, 128));
+        }
+        plans.push_back(make_plan(n, p, m, i % 2 ? 3 : 1, i % 4 == 0));
+      }
+      const std::string what = std::to_string(count) + " grids";
+      even(plans, what);
+      plans.push_back(make_plan({40, 40, 20}, {3, 3, 2}, {256, 255, 200}, 3, false));
+      even(plans, what + " and a large one");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -74,6 +191,8 @@ int main(int argc, char** argv) {
     check_csr_many();
   else if (name == "groups")
     check_groups();
+  else if (name == "queues")
+    check_queues();
   else
     require(false, "no check named '" + name + "'");
   std::printf("launch_check ok %s\n", name.c_str());
