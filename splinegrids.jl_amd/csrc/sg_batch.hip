@@ -475,12 +475,12 @@ __device__ __attribute__((always_inline)) void batch_tile_p2(const BGrid& g, con
 // which outweighs the residency of six workgroups per CU.
 __global__ __launch_bounds__(kThreads, 4) void batch_tiles(const BGrid* __restrict__ grids,
                                                         const BTile* __restrict__ tiles,
-                                                        const int* __restrict__ queues) {
+                                                        const int* __restrict__ queues, int first) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   float* smem = reinterpret_cast<float*>(smem_raw);
   const int lane = threadIdx.x & (kLanes - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
-  const int ti = queue_tile(queues);
+  const int ti = queue_tile(queues, first);
   if (ti < 0) return;
   const BTile t = tiles[ti];
   const BGrid g = grids[t.grid];
@@ -739,9 +739,15 @@ int build_tiles(sg_batch* b, int rows_per_wave, int blocks_per_cu) {
 
 hipError_t launch_batch(sg_batch* b, hipStream_t s) {
   if (b->n_tiles == 0 || !b->counters) return hipSuccess;  // no tile to run
-  hipLaunchKernelGGL(batch_tiles, dim3(kXcds * b->queue_len), dim3(kThreads), b->lds, s, b->dgrids,
-                     b->dtiles, b->counters);
-  return hipGetLastError();
+  // queues of more tiles than a launch has workgroups for go out in parts
+  const int most = static_cast<int>(launch_groups(kXcds * kThreads));
+  for (int first = 0; first < b->queue_len; first += most) {
+    hipLaunchKernelGGL(batch_tiles, dim3(kXcds * std::min(most, b->queue_len - first)),
+                       dim3(kThreads), b->lds, s, b->dgrids, b->dtiles, b->counters, first);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace

@@ -24,15 +24,16 @@ struct BTile {
 constexpr int kQueueStride = 64;
 constexpr int kQueueInts = kXcds * kQueueStride + kXcds + 1;
 
-// The tile of this workgroup, or -1 past the end of its queue.
-__device__ inline int queue_tile(const int* __restrict__ queues) {
+// The tile of this workgroup in a launch from the queues' tiles `first` on, or
+// -1 past the end of its queue.
+__device__ inline int queue_tile(const int* __restrict__ queues, int first) {
   const int* start = queues + kXcds * kQueueStride;
   const int q = static_cast<int>(blockIdx.x) % kXcds;
-  const int i = start[q] + static_cast<int>(blockIdx.x) / kXcds;
+  const int i = start[q] + first + static_cast<int>(blockIdx.x) / kXcds;
   return i < start[q + 1] ? i : -1;
 }
 
-// Tiles of the longest queue: queue_tile's launch takes kXcds times as many
+// Tiles of the longest queue: queue_tile's launches take kXcds times as many
 // workgroups.
 inline int longest_queue(const int* host_q) {
   const int* start = host_q + kXcds * kQueueStride;
