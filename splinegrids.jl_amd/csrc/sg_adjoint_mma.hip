@@ -121,6 +121,166 @@ constexpr int unit_buffers() {
   return NC == 1 ? 2 : NC;
 }
 
+__device__ inline bool finite(float x) { return __builtin_isfinite(x); }
+__device__ inline bool finite(double x) { return __builtin_isfinite(x); }
+
+// The kernel's arguments, read again: what the cold path below takes from here
+// the hot one need not hold (held, they spilled 50 scalars and cost 1.2 us of 33
+// on 200 x 201 x 99 x 3 FP64).
+template <typename T>
+using Global = __attribute__((address_space(1))) T;
+template <typename T>
+using AdjArgsAgain = Constant<const AdjMmaArgs<T>>;
+template <typename T>
+__device__ inline AdjArgsAgain<T>* kernel_args() {
+  auto at = reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(at));
+  return reinterpret_cast<AdjArgsAgain<T>*>(at);
+}
+
+// The workgroup's tile, chunk, run and first channel.
+struct AdjBlock {
+  int bx, by, bz, c0;
+};
+template <typename Args>
+__device__ inline AdjBlock adj_block(const Args& a, int nc) {
+  int rest = xcd_logical_block(a.xcd_map, a.ntx);
+  AdjBlock b;
+  b.bx = rest % a.ntx;
+  rest /= a.ntx;
+  b.by = rest % a.nty;
+  rest /= a.nty;
+  b.bz = rest % a.nz;
+  b.c0 = (a.group0 + rest / a.nz) * nc;
+  return b;
+}
+
+// A workgroup's run of one channel (c), every value over its own bands alone:
+// what adj_mma takes back to where Inf or NaN entered its products, whose zeros
+// off the bands make NaN of the whole window.  Same partial windows, plain sums
+// through LDS (banded_lds elements).  Slow, and seldom: 200 x 201 x 99 x 3 FP64
+// with one Inf 185 us, all NaN 222 (clean 33); 400 x 400 x 200 x 3 743 and 1367
+// (88); NURBS 512 x 512 x 256 x 3 3.8 and 5.3 ms (0.18).  What it costs a clean
+// call: 0.2 to 0.4 us.  (A check of each unit in the loop: 0.6 us.)
+template <typename T, int NIN, int P3, int NQ, bool NURBS>
+__device__ __attribute__((always_inline)) void banded_run(AdjArgsAgain<T>& a, T* lds, int bx, int by, int bz, int c) {
+  constexpr int TW = 16 * NQ;
+  // (the compiler knows no address space of a pointer that it reads from memory)
+  const auto span1 = (Global<const int32_t>*)a.span1;
+  const auto span2 = (Global<const int32_t>*)a.span2;
+  const auto span3 = (Global<const int32_t>*)a.span3;
+  const auto tab1 = (Global<const T>*)a.tab1;
+  const auto tab2 = (Global<const T>*)a.tab2;
+  const auto tab3 = (Global<const T>*)a.tab3;
+  const auto part = (Global<T>*)a.part;
+  const int tid = static_cast<int>(threadIdx.x), threads = static_cast<int>(blockDim.x);
+  const int rows = threads / 4;           // rows j2 at a time
+  T* T1 = lds;                            // [rows][kWin]
+  T* G = T1 + 4 * threads;                // NURBS: [kWin][kWin] weights at j3
+  T* winv = G + kSlab;                    // NURBS: [rows][TW] 1 / w
+  const int p1 = a.p1, p2 = a.p2;
+  const int j1_0 = bx * TW, x1 = min(j1_0 + TW, a.m1);
+  const int r0 = by * a.chunk, r1 = min(r0 + a.chunk, a.m2);
+  const int lo1 = span1[j1_0] - p1, lo2 = span2[r0] - p2;
+  const int W1 = span1[x1 - 1] - lo1 + 1, W2 = span2[r1 - 1] - lo2 + 1;
+  const int j3a = NIN == 3 ? bz * a.j3_per_block : 0;
+  const int j3e = NIN == 3 ? min(j3a + a.j3_per_block, a.m3) : 1;
+  const int lo3 = NIN == 3 ? span3[j3a] - P3 : 0;
+  const size_t block = (static_cast<size_t>(bz) * a.nty + by) * a.ntx + bx;
+  // the samples whose bands hold a control point are one range
+  const auto range = [](Global<const int32_t>* span, int p, int from, int to, int k, int& first, int& last) {
+    first = last = from;
+    for (int j = from; j < to; ++j) {
+      first += span[j] < k ? 1 : 0;
+      last += span[j] - p <= k ? 1 : 0;
+    }
+  };
+  const int q1 = tid % kWin;
+  int ja, jb;
+  range(span1, p1, j1_0, x1, lo1 + q1, ja, jb);
+  for (int t0 = 0; t0 < kSlab; t0 += threads) {  // the thread's window entry
+    const int q2 = (t0 + tid) / kWin;
+    int ra, rb;
+    range(span2, p2, r0, r1, lo2 + q2, ra, rb);
+    const auto store = [&](T v, int k3) {
+      if (q2 < W2 && q1 < W1)
+        part[((block * a.w3max + (k3 - lo3)) * a.nout + c) *
+                   (static_cast<size_t>(a.w1max) * a.w2max) + q2 * a.w1max + q1] = v;
+    };
+    T R[P3 + 1];
+#pragma unroll
+    for (int d = 0; d <= P3; ++d) R[d] = T(0);
+    int cur3 = lo3 + P3;
+    for (int j3 = j3a; j3 < j3e; ++j3) {
+      const int s3 = NIN == 3 ? span3[j3] : 0;
+      T b3[P3 + 1];
+#pragma unroll
+      for (int d = 0; d <= P3; ++d)
+        b3[d] = NIN == 3 ? tab3[static_cast<size_t>(j3) * (P3 + 1) + d] : T(1);
+      for (; NIN == 3 && cur3 < s3; ++cur3) {
+        store(R[0], cur3 - P3);
+#pragma unroll
+        for (int d = 0; d < P3; ++d) R[d] = R[d + 1];
+        R[P3] = T(0);
+      }
+      if constexpr (NURBS) {
+        for (int x = tid; x < kSlab; x += threads) {
+          const auto W = (Global<const T>*)a.W + (static_cast<long long>(NIN == 3 ? s3 - P3 : 0) * a.n2 +
+                              lo2 + x / kWin) * a.n1 + lo1 + x % kWin;
+          T v = T(0);
+          if (x / kWin < W2 && x % kWin < W1)
+#pragma unroll
+            for (int d = 0; d <= P3; ++d) v += b3[d] * W[static_cast<long long>(d) * a.n2 * a.n1];
+          G[x] = v;
+        }
+        __syncthreads();
+      }
+      const auto E = (Global<const T>*)a.E + a.m12 * j3 + a.nsamp * c;
+      T t2 = T(0);
+      for (int row0 = r0; row0 < r1; row0 += rows) {
+        const int n = min(rows, r1 - row0);
+        if constexpr (NURBS) {
+          for (int x = tid; x < n * TW; x += threads) {
+            const int j1 = j1_0 + x % TW, j2 = row0 + x / TW;
+            if (j1 >= x1) continue;
+            const T* g = G + (span2[j2] - p2 - lo2) * kWin + span1[j1] - p1 - lo1;
+            T w = T(0);
+            for (int d = 0; d <= p2; ++d, g += kWin) {
+              T u = T(0);
+              for (int q = 0; q <= p1; ++q) u += tab1[static_cast<size_t>(j1) * (p1 + 1) + q] * g[q];
+              w += tab2[static_cast<size_t>(j2) * (p2 + 1) + d] * u;
+            }
+            winv[x] = T(1) / w;
+          }
+          __syncthreads();
+        }
+        for (int x = tid; x < n * kWin; x += threads) {
+          const int r = x / kWin;
+          const auto row = E + static_cast<long long>(row0 + r) * a.m1;
+          T s = T(0);
+#pragma unroll 4
+          for (int j1 = ja; j1 < jb; ++j1)
+            s += tab1[static_cast<size_t>(j1) * (p1 + 1) + lo1 + q1 + p1 - span1[j1]] *
+                 (NURBS ? row[j1] * winv[r * TW + j1 - j1_0] : row[j1]);
+          T1[x] = s;
+        }
+        __syncthreads();
+        for (int j2 = max(ra, row0); j2 < min(rb, row0 + n); ++j2)
+          t2 += tab2[static_cast<size_t>(j2) * (p2 + 1) + lo2 + q2 + p2 - span2[j2]] *
+                T1[(j2 - row0) * kWin + q1];
+        __syncthreads();
+      }
+#pragma unroll
+      for (int d = 0; d <= P3; ++d) R[d] += b3[d] * t2;
+    }
+#pragma unroll
+    for (int d = 0; d <= P3; ++d) store(R[d], cur3 - P3 + d);
+  }
+}
+constexpr size_t banded_lds(int nw, int nq, bool nurbs) {
+  return static_cast<size_t>(nw) * kSlab * (nurbs ? 1 + nq : 1) + (nurbs ? kSlab : 0);
+}
+
 // NURBS: ebar is multiplied by 1 / w(x) as its units arrive.  The weight
 // field of a unit is two more small products with the same operand trick,
 //   V[k2][j1] = sum_k1 Gw[k2][k1] B1[j1][k1],  w^T[j1][j2] = sum_k2 V[k2][j1] B2[j2][k2],
@@ -148,13 +308,8 @@ __global__ __launch_bounds__(kThreads, NURBS && sizeof(T) == 8 ? 1 : 2) void adj
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
   const int nw = static_cast<int>(blockDim.x) / kLanes;
   const int g = lane >> 4, i = lane & 15;
-  int rest = xcd_logical_block(a.xcd_map, a.ntx);
-  const int bx = rest % a.ntx;
-  rest /= a.ntx;
-  const int by = rest % a.nty;
-  rest /= a.nty;
-  const int bz = rest % a.nz;
-  const int c0 = (a.group0 + rest / a.nz) * NC;
+  const AdjBlock at = adj_block(a, NC);
+  const int bx = at.bx, by = at.by, bz = at.bz, c0 = at.c0;
   const int nc = NC == 1 ? 1 : min(NC, a.nout - c0);
   const int j1_0 = bx * 16 * NQ;
   const int r0 = by * a.chunk, r1 = min(r0 + a.chunk, a.m2);
@@ -347,10 +502,12 @@ __global__ __launch_bounds__(kThreads, NURBS && sizeof(T) == 8 ? 1 : 2) void adj
   // next use of a slot only past the barrier that follows every wave's reads
   // of it.
   int par = 0;
+  T seen = T(0);  // not finite once a slab was not (all its entries then are)
   const size_t block = (static_cast<size_t>(bz) * a.nty + by) * a.ntx + bx;
   auto flush = [&](const D& slab, int ch, int k3) {
     T* dst = a.part + ((block * a.w3max + (k3 - lo3)) * a.nout + c0 + ch) *
                           (static_cast<size_t>(a.w1max) * a.w2max);
+    seen += slab[0];
     if (nw == 1) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -481,12 +638,33 @@ __global__ __launch_bounds__(kThreads, NURBS && sizeof(T) == 8 ? 1 : 2) void adj
       }
     }
   }
-  // the run's last band is final
+  // the run's last band is final; the waves tell each other what they have seen
+  // before its last barrier
+  T* flags = red + 2 * static_cast<size_t>(nw) * kSlab;  // [nw]
 #pragma unroll
   for (int d = 0; d <= P3; ++d)
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc)
-      if (cc < nc) flush(R[cc][d], cc, cur3 - P3 + d);
+      if (cc < nc) {
+        if (!MT && d == P3 && cc == nc - 1 && lane == 0) {
+          T all = seen;
+#pragma unroll
+          for (int c = 0; c < NC; ++c) all += R[c][P3][0];
+          flags[wave] = all;
+        }
+        flush(R[cc][d], cc, cur3 - P3 + d);
+      }
+  if constexpr (!MT) {
+    T all = flags[0];
+    for (int w = 1; w < nw; ++w) all += flags[w];
+    if (__builtin_expect(!finite(wave_uniform(all)), 0)) {
+      __syncthreads();
+      AdjArgsAgain<T>& again = *kernel_args<T>();
+      const AdjBlock here = adj_block(again, NC);
+      for (int c = here.c0; c < min(here.c0 + NC, again.nout); ++c)
+        banded_run<T, NIN, P3, NQ, NURBS>(again, red, here.bx, here.by, here.bz, c);
+    }
+  }
 }
 
 template <typename T>
@@ -590,7 +768,9 @@ hipError_t launch_mma(const Plan& pl, int tier, const int32_t* orders, const T* 
   if (!k) return hipErrorInvalidValue;
   const int nw = tl.chunk_rows() / tl.rows_per_wave;
   const long long blocks = static_cast<long long>(tl.n_tiles1) * tl.n_chunks2 * tl.n_z;
-  const size_t lds = nw > 1 ? 2 * static_cast<size_t>(nw) * kSlab * sizeof(T) : 0;
+  // the waves' sums and flags, or what banded_run keeps there
+  const size_t lds = std::max(2 * static_cast<size_t>(nw) * kSlab + nw,
+                              banded_lds(nw, tl.tile_width() / 16, W != nullptr)) * sizeof(T);
   // a plane's tiles are below 2^32 threads by its size (adjoint_mma_shape_ok),
   // those of every channel need not be
   const int groups = (pl.nout + per - 1) / per;
