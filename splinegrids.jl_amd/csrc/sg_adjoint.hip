@@ -307,14 +307,8 @@ struct AdjGatherArgs {
 // sums with a fixed butterfly, so every result is the same sum in the same
 // order on every run.  A workgroup lies in one (k3, channel) plane.
 //
-// Bound: latency -- a table row per dimension, then the windows.  One lane
-// per control point where the points alone fill the chip (64 x 64 x 32 points
-// x 3: 18 us with four lanes, 10 with one) or have few windows; four lanes
-// below kGatherFill points (20^3 x 3 points of up to 75 windows: 14 us with
-// one lane, 7 with four; 40 x 40 x 20 x 3: 6.3 and 6.7 us).
-constexpr int kGatherBatch = 4;
-constexpr long long kGatherFill = 1 << 16;
-
+// Bound: latency -- a table row per dimension, then the windows (gather_lanes
+// chooses LANES).
 template <typename T, int LANES>
 __global__ __launch_bounds__(256) void adj_gather(AdjGatherArgs<T> a) {
   const int q = static_cast<int>(blockIdx.x) / a.blocks, plane = a.plane0 + q;
@@ -642,15 +636,14 @@ hipError_t gather(const Plan& pl, const Tiling& tl, const T* part, T* Pbar, int 
   const long long n12 = static_cast<long long>(g.n1) * g.n2;
   g.ncp = n12 * g.n3;
   const long long planes = static_cast<long long>(g.n3) * pl.nout;
-  const bool wide = tl.gwindows > kGatherBatch && g.ncp * pl.nout <= kGatherFill;
-  const int lanes = wide ? 4 : 1;
+  const int lanes = gather_lanes(tl.gwindows, g.ncp * pl.nout);
   g.blocks = static_cast<int>((n12 * lanes + 255) / 256);
   // small planes are mostly idle threads: many of them take several launches
   const long long per = launch_groups(256LL * g.blocks);
   for (long long p0 = 0; p0 < planes; p0 += per) {
     g.plane0 = static_cast<int>(p0);
     const long long blocks = std::min(per, planes - p0) * g.blocks;
-    hipLaunchKernelGGL((wide ? adj_gather<T, 4> : adj_gather<T, 1>),
+    hipLaunchKernelGGL((lanes == 4 ? adj_gather<T, 4> : adj_gather<T, 1>),
                        dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, g);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -6,6 +6,7 @@
 // sanitizers and driven on the CPU by tests/native/plan_check.cpp.
 #pragma once
 
+#include <algorithm>
 #include <functional>
 #include <vector>
 
@@ -68,6 +69,18 @@ GatherLists gather_lists(const Plan& pl, const Tiling& t, int w1, int w2);
 // come from one cache line; a longer list follows the rows, from the index in
 // the row's second entry.  most: the longest list.
 std::vector<long long> gather_table(const GatherLists& g, int d, int& most);
+
+// Lanes per control point of the gather (1 or 4), for control points of up to
+// `windows` windows and `outputs` control points times channels.  A lane alone
+// where its windows are one batch of loads, or where the points fill the chip
+// before their windows count: one window in 16 384 points (64 x 64 x 32 x 3: 18
+// us with four lanes, 10 with one; 100^3, 12 windows: a whole call 70 and 52).
+// Else four (20^3 x 3, up to 75 windows: 14 us with one lane, 7 with four; 73 x 9
+// x 26 x 4, 94 windows: a whole call 96 and 72; 30 x 30 x 40 x 2, 152: 122, 78).
+constexpr int kGatherBatch = 4;  // loads of windows in flight per lane
+inline int gather_lanes(long long windows, long long outputs) {
+  return windows > std::max<long long>(kGatherBatch, outputs >> 14) ? 4 : 1;
+}
 
 // Transposed band lists of a dimension: the (sample, term) pairs whose band
 // holds control point k, j * (p + 1) + a, in sample order, at

@@ -68,6 +68,18 @@ void check_groups() {
   }
 }
 
+// Four lanes of the gather share a point's windows where there are many, also
+// past 65 536 control points.
+void check_gather_lanes() {
+  require(gather_lanes(94, 68328) == 4, "73 x 9 x 26 x 4 control points of 94 windows");
+  require(gather_lanes(152, 72000) == 4, "30 x 30 x 40 x 2 of 152 windows");
+  require(gather_lanes(88, 128000) == 4, "40 x 40 x 40 x 2 of 88 windows");
+  require(gather_lanes(75, 24000) == 4, "20^3 x 3 of 75 windows");
+  require(gather_lanes(4, 8148) == 1, "four windows are one batch");
+  require(gather_lanes(12, 393216) == 1, "64 x 64 x 32 x 3 control points");
+  require(gather_lanes(12, 1000000) == 1, "100^3 control points");
+}
+
 // A plan's host part for clamped uniform knots and uniform samples: the spans.
 Plan make_plan(const std::vector<int>& n, const std::vector<int>& p, const std::vector<int>& m,
                int nout, bool nurbs) {
@@ -193,6 +205,8 @@ int main(int argc, char** argv) {
     check_groups();
   else if (name == "queues")
     check_queues();
+  else if (name == "gather_lanes")
+    check_gather_lanes();
   else
     require(false, "no check named '" + name + "'");
   std::printf("launch_check ok %s\n", name.c_str());
