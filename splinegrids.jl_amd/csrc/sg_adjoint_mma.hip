@@ -696,7 +696,7 @@ AdjMmaKernel<T> pick_nq(int tile_width, int tier, int nurbs_nc) {
 
 template <typename T>
 AdjMmaKernel<T> pick_adj_mma(const Plan& pl, int tier, int nurbs_nc) {
-  const int tw = pl.adjm.tile_width();
+  const int tw = pl.adjoint(sizeof(T)).tile_width();
   if (pl.nin == 2) return pick_nq<T, 2, 0>(tw, tier, nurbs_nc);
   switch (pl.dims[2].p) {
     case 0: return pick_nq<T, 3, 0>(tw, tier, nurbs_nc);
@@ -713,10 +713,30 @@ long long plane_samples(const Plan& pl) {
   return static_cast<long long>(pl.dims[0].m) * pl.dims[1].m;
 }
 
+// Channels that share a workgroup and its weight field (NURBS).
+template <typename T>
+int weight_channels(const Plan& pl) {
+  return sizeof(T) == 4 && adjoint_shares_weights(pl) ? 3 : 1;
+}
+
+template <typename T>
+int resident_waves(const Plan& pl) {
+  AdjMmaKernel<T> k = pick_adj_mma<T>(pl, SG_TIER_NATIVE, pl.nurbs ? weight_channels<T>(pl) : 0);
+  if (!k) return 0;
+  int blocks = 0, cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(k),
+                                                   kThreads, 0) != hipSuccess)
+    return 0;
+  return blocks * kWaves * cus;
+}
+
 template <typename T>
 hipError_t launch_mma(const Plan& pl, int tier, const int32_t* orders, const T* E, const T* W,
                       T* Pbar, int accumulate, hipStream_t s) {
-  const Tiling& tl = pl.adjm;
+  const Tiling& tl = pl.adjoint(sizeof(T));
   const DimDev& d1 = pl.dims[0];
   const DimDev& d2 = pl.dims[1];
   const auto table = [](const DimDev& d, int order) {
@@ -762,7 +782,7 @@ hipError_t launch_mma(const Plan& pl, int tier, const int32_t* orders, const T* 
   a.w3max = tl.w3max;
   a.m12 = plane_samples(pl);
   a.nsamp = a.m12 * a.m3;
-  const int nurbs_nc = !W ? 0 : sizeof(T) == 4 && adjoint_shares_weights(pl) ? 3 : 1;
+  const int nurbs_nc = W ? weight_channels<T>(pl) : 0;
   const int per = std::max(nurbs_nc, 1);
   AdjMmaKernel<T> k = pick_adj_mma<T>(pl, tier, nurbs_nc);
   if (!k) return hipErrorInvalidValue;
@@ -795,24 +815,18 @@ bool adjoint_mma_shape_ok(const Plan& pl, int dtype) {
          plane_samples(pl) * (dtype == SG_F32 ? 4 : 8) < static_cast<long long>(kOff) - 64;
 }
 
-int adjoint_mma_resident_waves(const Plan& pl) {
-  AdjMmaKernel<float> k = pick_adj_mma<float>(pl, SG_TIER_NATIVE, 0);
-  if (!k) return 0;
-  int blocks = 0, cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(k),
-                                                   kThreads, 0) != hipSuccess)
-    return 0;
-  return blocks * kWaves * cus;
-}
+int adjoint_mma_resident_waves(const Plan& pl) { return resident_waves<float>(pl); }
+int adjoint_mma_resident_waves64(const Plan& pl) { return resident_waves<double>(pl); }
 
 size_t adjoint_mma_work_bytes(const Plan& pl) {
-  const Tiling& t = pl.adjm;
-  if (t.n_tiles1 == 0) return 0;
-  const size_t units = static_cast<size_t>(t.n_tiles1) * t.n_chunks2 * t.n_z;
-  return units * t.w3max * pl.nout * t.w1max * t.w2max * sizeof(double);
+  size_t most = 0;
+  for (size_t elem : {sizeof(float), sizeof(double)}) {
+    const Tiling& t = pl.adjoint(elem);
+    if (t.n_tiles1 == 0) continue;
+    const size_t units = static_cast<size_t>(t.n_tiles1) * t.n_chunks2 * t.n_z;
+    most = std::max(most, units * t.w3max * pl.nout * t.w1max * t.w2max * elem);
+  }
+  return most;
 }
 
 hipError_t launch_adjoint_mma(const Plan& pl, int tier, const int32_t* orders, const void* E,

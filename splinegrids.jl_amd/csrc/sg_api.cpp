@@ -275,13 +275,14 @@ int build_plan(const sg_grid_desc* desc, hipStream_t s, bool want_adjoint, Plan*
   }
   if (rc != SG_OK) return rc;
 
-  plan_tilings(*pl, want_adjoint, adjoint_mma_shape_ok(*pl, SG_F32), adjoint_mma_resident_waves);
+  plan_tilings(*pl, want_adjoint, adjoint_mma_shape_ok(*pl, SG_F32), adjoint_mma_resident_waves,
+               adjoint_mma_resident_waves64);
   // adj_stream is reached only where the matrix-core adjoint is not: without
   // its tiling, or (FP64) with planes past its buffer loads
   if (pl->adjm.n_tiles1 > 0 && adjoint_mma_shape_ok(*pl, SG_F64)) pl->adj = Tiling();
   if (pl->stream_ok && (pl->adj.n_tiles1 > 0 || pl->adjm.n_tiles1 > 0)) {
     hipError_t e = hipSuccess;
-    for (Tiling* t : {&pl->adj, &pl->adjm})
+    for (Tiling* t : {&pl->adj, &pl->adjm, &pl->adjm64})
       if (e == hipSuccess && t->n_tiles1 > 0) e = upload_gather_lists(*pl, *t, t->w1max, t->w2max);
     pl->work_bytes = std::max(adjoint_work_bytes(*pl), adjoint_mma_work_bytes(*pl));
     unsigned char* w = nullptr;
@@ -387,6 +388,7 @@ int sg_plan_describe(const sg_plan* plan, char* text, int32_t capacity) {
   os << " ";
   tiling("adj", pl.adj);
   tiling("adjm", pl.adjm);
+  tiling("adjm_f64", pl.adjm64);
   os << "work_bytes=" << pl.work_bytes;
   const std::string s = os.str();
   const size_t n = std::min(s.size(), static_cast<size_t>(capacity - 1));

@@ -150,12 +150,13 @@ struct Plan {
   Tiling fields, fields64;    //   and launches of several
   Tiling adj, mma;
   Sweep sweep[2];             // FP32, FP64
-  Tiling adjm;                // matrix-core adjoint (n_tiles1 == 0: not used)
+  Tiling adjm, adjm64;        // matrix-core adjoint, FP32 and FP64 (n_tiles1 == 0: not used)
   int nt_stores = 0;          // non-temporal stores of eval
   void* work = nullptr;       // adjoint partial slabs (either adjoint path)
   size_t work_bytes = 0;
   size_t device_bytes = 0;
   std::vector<void*> allocations;
+  const Tiling& adjoint(size_t elem) const { return elem == sizeof(double) ? adjm64 : adjm; }
   const Tiling& forward(size_t elem, int nf = 1) const {
     if (nf > 1) return elem == sizeof(double) ? fields64 : fields;
     return elem == sizeof(double) ? fwd64 : fwd;
@@ -269,7 +270,10 @@ hipError_t launch_adjoint_gather(const Plan& plan, const Tiling& tl,
 
 // ---- sg_adjoint_mma.hip ----
 bool adjoint_mma_shape_ok(const Plan& plan, int dtype);
-int adjoint_mma_resident_waves(const Plan& plan);  // on the current device
+// Waves of the plan's FP32 / FP64 kernel (NURBS plans: with weights) that the
+// current device holds at once.
+int adjoint_mma_resident_waves(const Plan& plan);
+int adjoint_mma_resident_waves64(const Plan& plan);
 size_t adjoint_mma_work_bytes(const Plan& plan);
 // The adjoint on matrix cores (plan.adjm not empty, shape ok for dtype).
 // Tiers other than native take FP32 arrays.  W not null: the adjoint of the

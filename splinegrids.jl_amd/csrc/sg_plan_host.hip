@@ -135,13 +135,14 @@ void balanced_rows(const Plan& pl, Tiling& t, int most, int waves) {
 
 // Matrix-core adjoint: tiles of 64 (or 32) samples j1 and workgroups of 4, 2
 // or 1 waves of up to 16 rows j2 (2-D: up to 128) whose band windows fit one
-// 16 x 16 MFMA tile, and runs of samples j3 (see below).  Leaves pl.adjm
-// empty when the bands do not fit.
-void plan_adjoint_mma(Plan& pl, const std::function<int(const Plan&)>& resident_waves) {
-  Tiling& t = pl.adjm;
-  // workgroups per tile, chunk and run: the channels, or with NURBS weights
-  // the groups of three that share a weight field
-  const long long groups = adjoint_shares_weights(pl) ? (pl.nout + 2) / 3 : pl.nout;
+// 16 x 16 MFMA tile, and runs of samples j3 (see below).  Leaves the tiling t
+// (pl.adjm or pl.adjm64) empty when the bands do not fit.
+void plan_adjoint_mma(Plan& pl, Tiling& t, size_t elem,
+                      const std::function<int(const Plan&)>& resident_waves) {
+  // workgroups per tile, chunk and run: the channels, or with NURBS weights in
+  // FP32 the groups of three that share a weight field
+  const long long groups =
+      elem == sizeof(float) && adjoint_shares_weights(pl) ? (pl.nout + 2) / 3 : pl.nout;
   const auto fit = [&](int tile, int most) {  // most waves per workgroup that fit
     t = Tiling();
     t.tile_w = tile;
@@ -183,17 +184,23 @@ void plan_adjoint_mma(Plan& pl, const std::function<int(const Plan&)>& resident_
     // few partial windows; what costs is a last round of workgroups that
     // leaves CUs idle (400 x 400 x 200 samples: 88 us with 735 workgroups,
     // 100 us with 588), and less than 32 KB of ebar in flight per CU (one
-    // unit per wave).  A run is never cut so short that not all workgroups
-    // are resident at once.
+    // unit per wave).  Runs shorter than 16 samples are never cut so short that
+    // not all workgroups are resident at once: their prologues would not overlap
+    // (FP64 NURBS, one wave per SIMD, 51 x 11 x 286 samples x 4: 40 us in 384
+    // workgroups of 3 samples, 27 in 192 of 6).  Longer ones may take what four
+    // waves per SIMD hold, in several rounds (FP64 NURBS 300 x 301 x 150 x 4: 191
+    // us in 500 workgroups, 254 in 200).
     const long long xy = groups * t.n_tiles1 * t.n_chunks2;
     const int m3 = pl.dims[2].m;
     const int waves = t.chunk_rows() / t.rows_per_wave;
     const long long most = std::max<long long>(resident_waves(pl) / waves, 1);
+    const long long rounds = std::max<long long>(most, 16 * kCus / waves);
     const double unit = 16.0 * t.tile_w * 4 * waves, window = t.w1max * t.w2max;
     const double samples = 1.0 * pl.dims[0].m * pl.dims[1].m * m3;
     double best = 0.0;
-    for (int runs = 1, last = 0; runs <= m3 && (runs == 1 || xy * runs <= most); ++runs) {
+    for (int runs = 1, last = 0; runs <= m3; ++runs) {
       const int len = (m3 + runs - 1) / runs, n = (m3 + len - 1) / len;
+      if (runs > 1 && xy * runs > (len < 16 ? most : rounds)) break;
       if (len == last) continue;
       last = len;
       compute_ztiling(pl, t, len);
@@ -340,7 +347,8 @@ void plan_sweep(const Plan& pl, size_t elem, Sweep& t) {
 }  // namespace
 
 void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
-                  const std::function<int(const Plan&)>& resident_waves) {
+                  const std::function<int(const Plan&)>& resident_waves,
+                  const std::function<int(const Plan&)>& resident_waves64) {
   // streaming kernels: Nin 2-3, monotone spans, p1, p2 <= 5, non-empty grid
   bool ok = (pl.nin == 2 || pl.nin == 3);
   for (int d = 0; ok && d < pl.nin; ++d) ok = pl.dims[d].monotone && pl.dims[d].m > 0;
@@ -408,8 +416,10 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
   const char* adj_mma_env = std::getenv("SG_ADJ_MMA");  // "0": streaming kernel only
   if (ok && want_adjoint && !(adj_mma_env && std::strcmp(adj_mma_env, "0") == 0) &&
       adjm_shape_ok) {
-    plan_adjoint_mma(pl, resident_waves);
-    pl.adjm.xcd_map = pl.adj.xcd_map;
+    plan_adjoint_mma(pl, pl.adjm, sizeof(float), resident_waves);
+    plan_adjoint_mma(pl, pl.adjm64, sizeof(double),
+                     resident_waves64 ? resident_waves64 : resident_waves);
+    pl.adjm.xcd_map = pl.adjm64.xcd_map = pl.adj.xcd_map;
   }
 }
 

@@ -48,11 +48,12 @@ int default_xcd_map(const Plan& pl);
 
 // Every tiling of a plan whose dimensions carry their host spans and
 // monotone flags: stream_ok, fwd, mma, and with want_adjoint adj and (when
-// adjm_shape_ok) adjm, whose task count uses resident_waves(plan) -- the
-// waves of the matrix-core adjoint the device holds at once for the
-// plan's adjm tiling as chosen so far.
+// adjm_shape_ok) adjm and adjm64, whose runs use resident_waves(plan) -- the
+// waves of the matrix-core adjoint the device holds at once for the plan's
+// tiling of that type as chosen so far (resident_waves64: FP64, if it differs).
 void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
-                  const std::function<int(const Plan&)>& resident_waves);
+                  const std::function<int(const Plan&)>& resident_waves,
+                  const std::function<int(const Plan&)>& resident_waves64 = nullptr);
 
 // For dimension d and control point k, the element offsets (in the partial
 // windows of tiling t, w1 x w2 x t.w3max per channel) of the windows that
