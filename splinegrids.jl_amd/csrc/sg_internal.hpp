@@ -148,6 +148,7 @@ struct Plan {
   bool stream_ok = false;     // streaming (sum-factorised) kernels apply
   Tiling fwd, fwd64;          // forward streaming kernels, FP32 and FP64: one field
   Tiling fields, fields64;    //   and launches of several
+  Tiling grad, grad64;        // NURBS value and first derivatives
   Tiling adj, mma;
   Sweep sweep[2];             // FP32, FP64
   Tiling adjm, adjm64;        // matrix-core adjoint, FP32 and FP64 (n_tiles1 == 0: not used)
@@ -156,6 +157,7 @@ struct Plan {
   size_t work_bytes = 0;
   size_t device_bytes = 0;
   std::vector<void*> allocations;
+  const Tiling& gradient(size_t elem) const { return elem == sizeof(double) ? grad64 : grad; }
   const Tiling& adjoint(size_t elem) const { return elem == sizeof(double) ? adjm64 : adjm; }
   const Tiling& forward(size_t elem, int nf = 1) const {
     if (nf > 1) return elem == sizeof(double) ? fields64 : fields;

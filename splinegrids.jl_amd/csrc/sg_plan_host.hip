@@ -11,6 +11,8 @@
 
 namespace sg {
 
+constexpr size_t kLdsPerCu = 160 * 1024;
+
 int env_int(const char* name, int fallback) {
   const char* v = std::getenv(name);
   if (!v || !*v) return fallback;
@@ -245,11 +247,17 @@ void plan_adjoint_mma(Plan& pl, Tiling& t, size_t elem,
 //     14.6 us (16 rows 14.9), 251x250x251 22 (16 rows 26).
 // Small grids take fewer rows, to two workgroups per CU: 1027x773, 3 channels
 // 7.4 us at 8 rows, 7.8 at 16.  (Earlier figures in brackets.)
+// The NURBS gradient takes the tiles of one field (three fields of 333x301x157,
+// 3 channels: 144 us, with those of several 175; 300x300x300, 4 channels 358,
+// 431), but FP64 kernels of three channels, which fill a CU with two workgroups,
+// take no fewer rows for a second round of them (167x264x31: 465 workgroups of
+// 16 rows 26 us, 837 of 8 rows 32), and no 32 rows where the windows, twice the
+// channels', crowd the LDS (99x270x159 of 60x103x66, scalar: 39 us, 16 rows 29).
 struct ForwardShape {
   int rows = 16, wx = 1, xcd_map = 0;
 };
 
-ForwardShape forward_shape(const Plan& pl, size_t elem, bool several) {
+ForwardShape forward_shape(const Plan& pl, size_t elem, bool several, bool gradient = false) {
   const DimDev& d1 = pl.dims[0];
   const int m1 = d1.m, m2 = pl.dims[1].m;
   const long long m3 = pl.nin == 3 ? pl.dims[2].m : 1;
@@ -273,7 +281,11 @@ ForwardShape forward_shape(const Plan& pl, size_t elem, bool several) {
     s.rows = 8;
   }
   auto groups = [&](int rows) { return m3 * tiles(s.wx) * chunks(rows); };
-  while (s.rows > 8 && groups(s.rows) < 2 * kCus) s.rows /= 2;
+  // (two per CU is all that the FP64 gradient's kernels of three channels hold)
+  const bool full = gradient && elem == sizeof(double) && pl.nin == 3 && pl.nout >= 3;
+  while (s.rows > 8 && groups(s.rows) < 2 * kCus &&
+         !(full && groups(s.rows / 2) > 2 * kCus))
+    s.rows /= 2;
   while (s.rows < 32 && groups(s.rows) > (1 << 23)) s.rows *= 2;  // grid limit: 2^24
   s.wx = env_int("SG_FWD_WX", s.wx);
   if (s.wx != 1 && s.wx != 2 && s.wx != 4) s.wx = 1;
@@ -357,9 +369,12 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
   if (ok) {
     const char* xm = std::getenv("SG_XCD_MAP");
     const int xcd = (xm && *xm) ? std::atoi(xm) : default_xcd_map(pl);
-    Tiling* const tilings[4] = {&pl.fwd, &pl.fields, &pl.fwd64, &pl.fields64};
-    for (int k = 0; k < 4; ++k) {
-      ForwardShape f = forward_shape(pl, k / 2 ? sizeof(double) : sizeof(float), k % 2 != 0);
+    Tiling* const tilings[6] = {&pl.fwd, &pl.fields, &pl.grad, &pl.fwd64, &pl.fields64, &pl.grad64};
+    for (int k = 0; k < 6; ++k) {
+      const size_t elem = k / 3 ? sizeof(double) : sizeof(float);
+      const bool gradient = k % 3 == 2;
+      if (gradient && !pl.nurbs) continue;
+      ForwardShape f = forward_shape(pl, elem, k % 3 == 1, gradient);
       Tiling& fwd = *tilings[k];
       compute_tiling(pl, fwd, f.rows, f.wx);
       // four windows of one channel: the NURBS gradient's least (two fields of
@@ -376,6 +391,9 @@ void plan_tilings(Plan& pl, bool want_adjoint, bool adjm_shape_ok,
           f.rows /= 2;
         compute_tiling(pl, fwd, f.rows, f.wx);
       }
+      // the gradient's windows, twice the channels', leave eight workgroups per CU
+      if (gradient && f.rows > 16 && 4 * elem * fwd.w1max * fwd.w2max > kLdsPerCu / 8)
+        compute_tiling(pl, fwd, 16, f.wx);
       fwd.xcd_map = f.xcd_map;
       ok = ok && forward_lds_worst(pl, fwd) <= static_cast<size_t>(kMaxLds);
     }
@@ -513,9 +531,8 @@ int csr_threads(long long outputs, double entries, int nin) {
              : kLanes;
 }
 
-// LDS of one CU; a launch meant to keep `bpc` workgroups per CU gives each
-// at most a bpc-th of it, or fewer workgroups than asked are resident.
-constexpr size_t kLdsPerCu = 160 * 1024;
+// A launch meant to keep `bpc` workgroups per CU gives each at most a bpc-th of
+// its LDS, or fewer workgroups than asked are resident.
 
 size_t lds_cap(int blocks_per_cu) {
   const size_t share = kLdsPerCu / static_cast<size_t>(std::max(1, blocks_per_cu));

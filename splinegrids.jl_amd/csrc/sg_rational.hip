@@ -255,7 +255,7 @@ int rat_grad_channels(const Plan& pl, int nf, const int32_t* orders, size_t elem
     if (total > 1 || seen[kind]++) return 0;
     d3 = d3 || kind == 3;
   }
-  const Tiling& t = pl.forward(elem);
+  const Tiling& t = pl.gradient(elem);
   for (int nc = std::min(kRatGradMaxNC, pl.nout); nc >= 1; --nc) {
     const size_t lds = static_cast<size_t>(d3 ? 2 : 1) * (nc + 1) * t.w1max * t.w2max * elem;
     if (lds <= static_cast<size_t>(kMaxLds)) return nc;
@@ -268,7 +268,7 @@ hipError_t rational_first_order(const Plan& pl, int nf, const int32_t* orders, c
                                 const T* W, T* const* outs, int nc_max, hipStream_t s) {
   const DimDev& d1 = pl.dims[0];
   const DimDev& d2 = pl.dims[1];
-  const Tiling& t = pl.forward(sizeof(T));
+  const Tiling& t = pl.gradient(sizeof(T));
   RatGradArgs<T> a{};
   T* out[4] = {nullptr, nullptr, nullptr, nullptr};
   for (int f = 0; f < nf; ++f) {

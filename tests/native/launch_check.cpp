@@ -103,6 +103,27 @@ Plan make_plan(const std::vector<int>& n, const std::vector<int>& p, const std::
   return pl;
 }
 
+Plan tiled(const std::vector<int>& n, const std::vector<int>& p, const std::vector<int>& m,
+           int nout, bool nurbs) {
+  Plan pl = make_plan(n, p, m, nout, nurbs);
+  plan_tilings(pl, true, true, [](const Plan&) { return 2048; });
+  require(pl.stream_ok, "streaming plan");
+  return pl;
+}
+
+// The NURBS gradient's rows where they differ from the evaluation's, and where not.
+void check_gradient() {
+  const Plan dense = tiled({60, 103, 66}, {1, 2, 3}, {99, 270, 159}, 1, true);
+  require(dense.fwd.rows_per_wave == 32 && dense.grad.rows_per_wave == 16, "windows crowd the LDS");
+  require(tiled({40, 40, 20}, {3, 3, 2}, {333, 301, 157}, 1, true).grad.rows_per_wave == 32,
+          "windows that do not");
+  const Plan full = tiled({124, 19, 4}, {3, 3, 2}, {167, 264, 31}, 3, true);
+  require(full.grad64.rows_per_wave == 16 && full.grad.rows_per_wave == 8, "two workgroups per CU");
+  require(tiled({60, 60, 30}, {2, 2, 2}, {300, 300, 300}, 4, true).grad.rows_per_wave == 8,
+          "a large volume");
+  require(tiled({40, 40, 20}, {3, 3, 2}, {333, 301, 157}, 1, false).grad.n_tiles1 == 0, "no weights");
+}
+
 struct Packed {
   std::vector<BTile> tiles;
   std::vector<int> q;
@@ -207,6 +228,8 @@ int main(int argc, char** argv) {
     check_queues();
   else if (name == "gather_lanes")
     check_gather_lanes();
+  else if (name == "gradient")
+    check_gradient();
   else
     require(false, "no check named '" + name + "'");
   std::printf("launch_check ok %s\n", name.c_str());

@@ -30,7 +30,7 @@ def launch_check(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", ["csr_limit", "csr_many", "groups", "queues",
-                                  "gather_lanes"])
+                                  "gather_lanes", "gradient"])
 def test_launch_shapes(launch_check, name):
     # the HIP runtime library keeps allocations to the end of the process
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0", UBSAN_OPTIONS="print_stacktrace=1")
