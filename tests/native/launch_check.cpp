@@ -124,6 +124,156 @@ void check_gradient() {
   require(tiled({40, 40, 20}, {3, 3, 2}, {333, 301, 157}, 1, false).grad.n_tiles1 == 0, "no weights");
 }
 
+std::string name_of(const Plan& pl) {
+  std::string s;
+  for (const DimDev& D : pl.dims)
+    s += "n" + std::to_string(D.n) + " p" + std::to_string(D.p) + " m" + std::to_string(D.m) + ", ";
+  return s + std::to_string(pl.nout) + (pl.nurbs ? " nurbs" : "");
+}
+
+// Every block of `len` samples: its window inside the control points, and
+// within `widest`.
+void check_windows(const DimDev& D, int blocks, int len, int widest, const std::string& what) {
+  require(blocks == (D.m + len - 1) / len, what + ": blocks");
+  for (int a = 0; a < D.m; a += len) {
+    const int lo = D.h_span[a] - D.p, hi = D.h_span[std::min(a + len, D.m) - 1];
+    require(lo >= 0 && hi < D.n && hi - lo + 1 <= widest, what + ": window");
+  }
+}
+
+// The swept forward's tiles: every sample in one, the windows of every tile
+// within the LDS that the launch takes.
+void check_sweep(const Plan& pl, int k, const std::string& what) {
+  const Sweep& t = pl.sweep[k];
+  if (t.threads_x == 0) return;
+  const DimDev &d1 = pl.dims[0], &d2 = pl.dims[1], &d3 = pl.dims[2];
+  const size_t elem = k ? sizeof(double) : sizeof(float);
+  const int tw = t.threads_x * (16 / static_cast<int>(elem));
+  require(t.threads_x * t.rows <= kThreads, what + ": threads");
+  require(t.ntx == (d1.m + tw - 1) / tw && t.nty == (d2.m + t.rows - 1) / t.rows &&
+              t.nz == (d3.m + t.run - 1) / t.run,
+          what + ": tiles");
+  require(t.lds_elements * elem <= static_cast<size_t>(kMaxLds), what + ": LDS");
+  require(static_cast<long long>(t.ntx) * t.nty * t.nz * kThreads < (1LL << 32), what + ": grid");
+  for (int a = 0; a < d1.m; a += tw)
+    for (int z = 0; z < d3.m; z += t.run) {
+      const int w1 = d1.h_span[std::min(a + tw, d1.m) - 1] - d1.h_span[a] + d1.p + 1;
+      const int planes = d3.h_span[std::min(z + t.run, d3.m) - 1] - d3.h_span[z] + d3.p + 1;
+      require(static_cast<size_t>(planes) * t.rows * w1 <= t.lds_elements, what + ": windows");
+    }
+}
+
+// The gather of a matrix-core tiling as the library lays it out: for every
+// control point the tables list the windows that hold it, whose element is the
+// one that the workgroup of that window writes.
+void check_gather(const Plan& pl, const Tiling& t, const std::string& what) {
+  const GatherLists g = gather_lists(pl, t, t.w1max, t.w2max);
+  const int nb[3] = {t.n_tiles1, t.n_chunks2, pl.nin == 3 ? t.n_z : 1};
+  const int len[3] = {t.tile_width(), t.chunk_rows(), t.j3_per_block};
+  const long long plane = static_cast<long long>(t.w1max) * t.w2max;
+  const long long block = plane * t.w3max * pl.nout;
+  const long long per_block[3] = {block, block * nb[0], block * nb[0] * nb[1]};
+  const long long per_point[3] = {1, t.w1max, plane * pl.nout};
+  require(g.gchan == plane, what + ": channels");
+  for (int d = 0; d < 3; ++d) {
+    int most = 0;
+    const std::vector<long long> table = gather_table(g, d, most);
+    const int n = d < pl.nin ? pl.dims[d].n : 1;
+    require(table.size() >= static_cast<size_t>(n) * kGatherRow, what + ": rows");
+    for (int k = 0; k < n; ++k) {
+      std::vector<long long> want;
+      for (int b = 0; b < nb[d]; ++b) {
+        if (d >= pl.nin) {
+          want.push_back(0);
+          continue;
+        }
+        const DimDev& D = pl.dims[d];
+        const int a = b * len[d], lo = D.h_span[a] - D.p, hi = D.h_span[std::min(a + len[d], D.m) - 1];
+        if (lo <= k && k <= hi) want.push_back(b * per_block[d] + (k - lo) * per_point[d]);
+      }
+      const long long* row = table.data() + static_cast<size_t>(k) * kGatherRow;
+      require(row[0] == static_cast<long long>(want.size()) && row[0] <= most, what + ": count");
+      size_t at = static_cast<size_t>(row - table.data()) + 2;
+      if (row[0] > kGatherRow - 2) at = static_cast<size_t>(row[1]);
+      require(at + want.size() <= table.size(), what + ": list");
+      require(std::equal(want.begin(), want.end(), table.begin() + at), what + ": offsets");
+    }
+  }
+}
+
+// Every tiling of plans over degrees, sizes and densities: the four forward
+// tilings, the gradient's, the swept forward's, both adjoints' and the batch's.
+void check_tilings() {
+  std::mt19937_64 rng(0x711E5);
+  const auto pick = [&](int a, int b) { return std::uniform_int_distribution<int>(a, b)(rng); };
+  std::vector<Plan> plans;
+  const auto add = [&](const std::vector<int>& n, const std::vector<int>& p, const std::vector<int>& m,
+                       int nout, bool nurbs) {
+    Plan pl = make_plan(n, p, m, nout, nurbs);
+    plan_tilings(pl, true, pl.nin == 2 || pl.dims[2].p <= kMaxStreamDegree,
+                 [](const Plan&) { return 4096; }, [](const Plan&) { return 1024; });
+    plans.push_back(pl);
+  };
+  add({64, 64, 32}, {3, 3, 2}, {512, 512, 256}, 3, true);
+  add({64, 64, 32}, {3, 3, 2}, {512, 512, 256}, 1, false);
+  add({40, 40, 20}, {3, 3, 3}, {400, 400, 200}, 3, false);
+  add({40, 40, 20}, {3, 3, 3}, {400, 401, 203}, 1, false);
+  add({128, 128}, {3, 3}, {4096, 4096}, 1, false);
+  add({200, 150}, {5, 5}, {210, 160}, 4, true);
+  add({9, 8, 30}, {2, 1, 1}, {700, 9, 901}, 1, false);
+  for (int i = 0; i < 400; ++i) {
+    const int nin = 2 + i % 2;
+    std::vector<int> n, p, m;
+    for (int d = 0; d < nin; ++d) {
+      const int limit = nin == 2 ? 2500 : i % 5 ? 90 : 260;
+      m.push_back(static_cast<int>(std::exp(std::uniform_real_distribution<double>(0.0, std::log(limit))(rng))));
+      p.push_back(pick(0, 5));
+      n.push_back(p[d] + 1 + pick(0, std::max(1, m[d])));
+    }
+    add(n, p, m, pick(1, 5), i % 3 == 0);
+  }
+  for (const Plan& pl : plans) {
+    const std::string nm = name_of(pl);
+    if (!pl.stream_ok) continue;
+    const long long m3 = pl.nin == 3 ? pl.dims[2].m : 1;
+    const Tiling* forward[] = {&pl.fwd, &pl.fwd64, &pl.fields, &pl.fields64, &pl.grad, &pl.grad64};
+    for (int k = 0; k < 6; ++k) {
+      const Tiling& t = *forward[k];
+      const std::string what = nm + " forward tiling " + std::to_string(k);
+      if (k >= 4 && !pl.nurbs) continue;
+      check_windows(pl.dims[0], t.n_tiles1, t.tile_width(), t.w1max, what);
+      check_windows(pl.dims[1], t.n_chunks2, t.chunk_rows(), t.w2max, what);
+      require(forward_lds_worst(pl, t) <= static_cast<size_t>(kMaxLds), what + ": LDS");
+      require(m3 * t.n_tiles1 * t.n_chunks2 * kThreads < (1LL << 32), what + ": grid");
+    }
+    for (int k = 0; k < 2; ++k) check_sweep(pl, k, nm + " sweep " + std::to_string(k));
+    for (const Tiling* t : {&pl.adjm, &pl.adjm64}) {
+      if (t->n_tiles1 == 0) continue;
+      const std::string what = nm + (t == &pl.adjm ? " adjm" : " adjm64");
+      require(t->w1max <= kAdjMmaWin && t->w2max <= kAdjMmaWin, what + ": window edge");
+      const int waves = t->chunk_rows() / t->rows_per_wave;
+      require((waves == 1 || waves == 2 || waves == 4) && waves * t->rows_per_wave == t->chunk_rows(),
+              what + ": waves");
+      check_windows(pl.dims[0], t->n_tiles1, t->tile_width(), t->w1max, what);
+      check_windows(pl.dims[1], t->n_chunks2, t->chunk_rows(), t->w2max, what);
+      if (pl.nin == 3) check_windows(pl.dims[2], t->n_z, t->j3_per_block, t->w3max, what);
+      check_gather(pl, *t, what);
+    }
+    require((pl.adjm.n_tiles1 > 0) == (pl.adjm64.n_tiles1 > 0), nm + ": both types or none");
+  }
+  // the batch's rows, and its longest queue
+  for (size_t count : {size_t(1), size_t(5), plans.size()}) {
+    std::vector<const Plan*> some;
+    for (size_t i = 0; i < count; ++i)
+      if (plans[i].stream_ok) some.push_back(&plans[i]);
+    const int rows = batch_default_rows(some, 256);
+    require(rows == 8 || rows == 16 || rows == 32, "batch rows");
+  }
+  std::vector<int> q(kQueueInts, 0);
+  for (int i = 0; i <= kXcds; ++i) q[kXcds * kQueueStride + i] = i < 3 ? 0 : 7 * i - 5;
+  require(longest_queue(q.data()) == 16, "longest queue");
+}
+
 struct Packed {
   std::vector<BTile> tiles;
   std::vector<int> q;
@@ -230,6 +380,8 @@ int main(int argc, char** argv) {
     check_gather_lanes();
   else if (name == "gradient")
     check_gradient();
+  else if (name == "tilings")
+    check_tilings();
   else
     require(false, "no check named '" + name + "'");
   std::printf("launch_check ok %s\n", name.c_str());

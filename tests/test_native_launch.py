@@ -1,5 +1,6 @@
-"""The launch shapes of the host plan code on the CPU (no GPU), built like
-the plan check of test_native_sanitize.py: tests/native/launch_check.cpp."""
+"""The launch shapes and tilings of the host plan code on the CPU (no GPU),
+built like the plan check of test_native_sanitize.py:
+tests/native/launch_check.cpp."""
 from __future__ import annotations
 
 import os
@@ -30,7 +31,7 @@ def launch_check(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", ["csr_limit", "csr_many", "groups", "queues",
-                                  "gather_lanes", "gradient"])
+                                  "gather_lanes", "gradient", "tilings"])
 def test_launch_shapes(launch_check, name):
     # the HIP runtime library keeps allocations to the end of the process
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0", UBSAN_OPTIONS="print_stacktrace=1")
