@@ -101,7 +101,7 @@ def workload(name: str):
                     knots=None, fields=[(0,)], P=None, W=None, copy=name)
     if name == "c5":
         return dict(name="c5: 1024 uneven grids (half 2-D, half 3-D, 25 % NURBS, Nout 1|3), "
-                         "one persistent launch, hipGraph, FP32",
+                         "one launch, hipGraph, FP32",
                     batch=True, dtype=np.float32, fields=[None], W=None)
     if name in ("c4", "c4a"):
         rng = np.random.default_rng(SEED0 + 4)
@@ -443,7 +443,7 @@ def timed_steps(step, steps: int, warmup: int):
 
 
 def bench_batch(args, sg, wl):
-    """The 1024-grid batch: the per-grid launch loop, the batched persistent launch, and the
+    """The 1024-grid batch: the per-grid launch loop, the batched launch, and the
     batched launch captured in a hipGraph; value is the graph replay."""
     import torch
 

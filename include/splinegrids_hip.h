@@ -187,8 +187,9 @@ int sg_evaluate_rational_adjoint(sg_plan* plan, const void* weights, const void*
  * accumulate = 0 overwrites control_points (the reference zeroes it first,
  * src/adjoint.jl:61); accumulate = 1 adds to it (reverse-mode AD).
  * Inf and NaN in eval reach the control points whose basis functions hold
- * their sample, and no others (split-FP16 and BF16: all of the 16 x 16 control
- * points of a tile).
+ * their sample, and no others on matrix cores and in the general adjoint; the
+ * streaming adjoint adds those of up to three samples beside it in dimension 1,
+ * the split-FP16 and BF16 tiers all of the 16 x 16 control points of a tile.
  * B-spline plans only (src/adjoint.jl:57).  The split-FP16 and BF16 tiers
  * run on the matrix-core adjoint (FP32 plans whose band windows fit 16 x 16
  * control points per tile); other plans return SG_ERR_UNSUPPORTED for them. */

@@ -295,14 +295,14 @@ function SplineGrids.spline_eval(grid::HIPGrid{Nin, Nout, Tv}, control_points::R
 end
 
 # ---------------------------------------------------------------------------
-# many grids in one persistent launch (no counterpart in the reference)
+# many grids in one launch (no counterpart in the reference)
 # ---------------------------------------------------------------------------
 
 """
     Batch(grids)
 
 Every grid (Float32, on the current AMD GPU) evaluated with derivative order 0
-by one persistent launch: `evaluate!(batch)`.  `autotune!(batch)` picks the
+by one launch: `evaluate!(batch)`.  `autotune!(batch)` picks the
 tiling on the current arrays; do it before capturing the launch in a graph.
 """
 mutable struct Batch

@@ -33,10 +33,10 @@
 //
 // Bound: HBM reads of ebar (a kernel that only reads ebar in this tile pattern
 // takes 76 us of the 82 here on 400 x 400 x 200 samples x 3, 147 of 154 on
-// 512 x 512 x 256 x 3).  With the gather: FP32 400 x 400 x 200 x 3 88 us (91
+// 512 x 512 x 256 x 3).  With the gather: FP32 400 x 400 x 200 x 3 87 us (91
 // with the channels and 64 rows in one wave); FP32 251 x 197 x 123 x 3 24 us
-// (50: rows of odd length took 4-byte loads); FP64 200 x 201 x 99 x 3 33 us
-// (154 with a sliding window of FMAs and LDS); NURBS 512 x 512 x 256 x 3 181 us
+// (50: rows of odd length took 4-byte loads); FP64 200 x 201 x 99 x 3 32 us
+// (154 with a sliding window of FMAs and LDS); NURBS 512 x 512 x 256 x 3 179 us
 // (327 with 1 / w(x) written by a pass of its own and read back).  What the
 // layout is for:
 //  - a wave holds one unit (16 rows x 16 NQ samples, 4 KB in FP32, 8 in FP64 at

@@ -380,6 +380,13 @@ int sg_plan_describe(const sg_plan* plan, char* text, int32_t capacity) {
   tiling("fwd", pl.fwd);
   tiling("fwd_f64", pl.fwd64);
   tiling("fields", pl.fields);
+  tiling("fields_f64", pl.fields64);
+  tiling("grad", pl.grad);
+  tiling("grad_f64", pl.grad64);
+  for (int k = 0; k < 2; ++k)
+    if (const Sweep& t = pl.sweep[k]; t.threads_x > 0)
+      os << (k ? "sweep_f64=" : "sweep=") << t.threads_x << "x" << t.rows << "x" << t.run
+         << ",tiles=" << t.ntx << "x" << t.nty << "x" << t.nz << " ";
   tiling("mma", pl.mma);
   const char* slow = (pl.stream_ok && pl.adj.n_tiles1 > 0) ? "stream" : "csr";
   const bool mma = pl.adjm.n_tiles1 > 0;
@@ -594,8 +601,8 @@ int sg_evaluate_adjoint(sg_plan* plan, const int32_t* derivative_order, const vo
   if (tier != SG_TIER_NATIVE && pl.adjm.n_tiles1 == 0)
     return fail(SG_ERR_UNSUPPORTED,
                 "the split-FP16 and BF16 adjoint tiers run on the matrix-core adjoint, which "
-                "needs band windows of at most 16 control points per 64 samples of dimension 1 "
-                "and per 16..64 samples of dimension 2 (and SG_ADJ_MMA not 0)");
+                "needs band windows of at most 16 control points per 32 samples of dimension 1 "
+                "and per 16 samples of dimension 2 (and SG_ADJ_MMA not 0)");
   if ((rc = check_orders(pl, 1, derivative_order)) != SG_OK) return rc;
   if (n_control(pl) == 0) return SG_OK;
   if (!control_points || (!eval && n_samples(pl) > 0))

@@ -8,7 +8,7 @@
 // fetched into one XCD's L2 rather than into all eight, and are cut into ranges
 // of tiles only where they would leave the queues uneven; within a queue the
 // costly tiles come first, so that the last to start are short
-// (256 uneven grids: 215 -> 206 us).  One kernel covers every queue, a
+// (256 uneven grids: 193 us in another order, 173 in this).  One kernel covers every queue, a
 // workgroup per tile (workgroups are dispatched to XCDs round-robin, so
 // workgroup b runs on XCD b mod 8).  Degrees, channel counts, NURBS weights
 // and sizes are per tile at run time; the p2+1 register window is selected by
@@ -466,9 +466,10 @@ __device__ __attribute__((always_inline)) void batch_tile_p2(const BGrid& g, con
 // One tile per workgroup: a workgroup that goes on to another tile waits, at
 // that tile's first load, for every store of the one before it (loads and
 // stores share a counter), while one that ends leaves its stores to drain.
-// 256 uneven grids, 500 MB: 198 us with four workgroups per CU taking tiles
-// from the queues in turn, 183 like this; 100 grids 99 and 84 us; 16 grids 41
-// and 23 us.  Bound: latency and VALU of the tiles (window staging alone 66
+// 256 uneven grids, 500 MB: 213 us with three workgroups per CU taking tiles
+// from the queues in turn, 170 like this; 128 grids 106 and 72 us; 16 grids 39
+// and 18 us; one volume of 256 x 255 x 200 x 3 58 and 32 us.  Bound: latency
+// and VALU of the tiles (of 198 us, in the other form: window staging alone 66
 // us, rows without their stores 60 us, the stores 73 us).
 // At most 128 VGPRs (four waves per SIMD): the row loop keeps a window
 // column's LDS reads in flight together and the row tables in registers,

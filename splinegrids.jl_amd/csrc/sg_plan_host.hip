@@ -181,8 +181,9 @@ void plan_adjoint_mma(Plan& pl, Tiling& t, size_t elem,
   int j3 = env_int("SG_ADJM_J3", 0);
   if (j3 <= 0) {
     // Runs of j3: the number that minimises a fit to measured times (14
-    // grids of 2 to 805 MB, FP32 and FP64, every run length; the fit picks
-    // within 2 % of the best on average, 7 % at worst).  Few long runs leave
+    // grids of 2 to 805 MB, FP32 and FP64, every run length; furthest from the
+    // best since: NURBS 230 x 281 x 132, 47 us in its 12 runs, 42 in 22).  Few
+    // long runs leave
     // few partial windows; what costs is a last round of workgroups that
     // leaves CUs idle (400 x 400 x 200 samples: 88 us with 735 workgroups,
     // 100 us with 588), and less than 32 KB of ebar in flight per CU (one
@@ -225,7 +226,7 @@ void plan_adjoint_mma(Plan& pl, Tiling& t, size_t elem,
 // that is set by how close together in time the pieces of one line and of one
 // DRAM page are written; so the waves of a workgroup stand side by side along
 // dimension 1 (unless that leaves over 11 % more of their lanes past the row's
-// end: 439x111x60, 3 channels, four fields 61 us with four, 55 with one), few
+// end: 439x111x60, 3 channels, four fields 56.5 us with four, 55 with one), few
 // rows deep:
 //   - rows of whole 64-byte sectors: no sector is shared; the launch order is
 //     kept, or by rows where a 128-byte line is shared.  16 rows: 512x512x256,
@@ -240,8 +241,8 @@ void plan_adjoint_mma(Plan& pl, Tiling& t, size_t elem,
 //     again weigh more (362x32x240, 4 channels: 16.7 us in 8 rows, 14.8);
 //     2-D grids have 16 (8001x6001, 3 channels 114 us, 8 rows 129; 171).
 //   - several fields in a launch are several streams of stores at one sample
-//     each: 16 rows (4096x4096, four fields 48 us, 52 with the tiles of one
-//     scalar; 203x311x160, 2 channels, four fields 91 us, 8 rows 105; 119).
+//     each: 16 rows (4096x4096, four fields 45 us, 57 with 32 rows; 203x311x160,
+//     2 channels, four fields 83 us, 8 rows 100).
 //   - one FP32 channel: a wave writes so little per row that its first columns
 //     (stage 1, first band) weigh more than the stores: 32 rows.  3001x3001
 //     14.6 us (16 rows 14.9), 251x250x251 22 (16 rows 26).

@@ -148,10 +148,11 @@ GridTiling batch_grid_tiling(const Plan& pl, int rows_per_wave, size_t cap);
 // Workgroups per CU a batch is tiled for (its LDS share; the kernel's 128
 // registers allow four waves per SIMD), and its rows per wave by the number of
 // tiles that 16 rows give: 8 below one tile per resident workgroup (16 grids,
-// 256 tiles: 26.4 us with 16 rows, 23.1 with 8), 32 from six on, where the
-// window staging weighs more than the last tiles (256 grids, 7 681 tiles:
-// 214 and 194 us; 1024 grids: 745 and 697 us), else 16 (64 grids, 1 878 tiles:
-// 55.3, 51.5, 54.7 us with 8, 16, 32; 180 grids, 5 207 tiles: 151, 143, 142).
+// 444 tiles: 19.5 us with 16 rows, 18.3 with 8), 32 from six on, where the
+// window staging weighs more than the last tiles (1024 grids, 30 785 tiles: 701
+// and 649 us; 256 grids, 7 171 tiles, near the line: 167 and 172), else 16 (100
+// grids, 3 024 tiles: 57.1, 55.8, 56.7 us with 8, 16, 32; 64 grids, 1 523 tiles:
+// 37.7, 41.4, 40.4).
 constexpr int kBatchPerCu = 4;
 int batch_default_rows(const std::vector<const Plan*>& plans, int cus);
 

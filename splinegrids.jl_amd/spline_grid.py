@@ -98,7 +98,7 @@ class Plan:
 
     def describe(self) -> str:
         """The kernels and tile shapes this plan uses, as one line of text."""
-        buf = ctypes.create_string_buffer(1024)
+        buf = ctypes.create_string_buffer(2048)
         _lib.check(self._lib.sg_plan_describe(self.handle, buf, len(buf)))
         return buf.value.decode()
 
