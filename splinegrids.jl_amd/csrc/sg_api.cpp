@@ -172,6 +172,13 @@ int validate_desc(const sg_grid_desc* desc) {
   return SG_OK;
 }
 
+// Two tilings of one plan whose workgroups hold the same windows.
+static bool same_windows(const Tiling& a, const Tiling& b) {
+  return a.tile_width() == b.tile_width() && a.chunk_rows() == b.chunk_rows() &&
+         a.rows_per_wave == b.rows_per_wave && a.j3_per_block == b.j3_per_block &&
+         a.n_tiles1 == b.n_tiles1;
+}
+
 // Uploads the gather lists of tiling tl (partial windows w1 x w2 x w3max per
 // channel) as the tables adj_gather reads.
 static hipError_t upload_gather_lists(Plan& pl, Tiling& tl, int w1, int w2) {
@@ -282,8 +289,12 @@ int build_plan(const sg_grid_desc* desc, hipStream_t s, bool want_adjoint, Plan*
   if (pl->adjm.n_tiles1 > 0 && adjoint_mma_shape_ok(*pl, SG_F64)) pl->adj = Tiling();
   if (pl->stream_ok && (pl->adj.n_tiles1 > 0 || pl->adjm.n_tiles1 > 0)) {
     hipError_t e = hipSuccess;
-    for (Tiling* t : {&pl->adj, &pl->adjm, &pl->adjm64})
+    for (Tiling* t : {&pl->adj, &pl->adjm})
       if (e == hipSuccess && t->n_tiles1 > 0) e = upload_gather_lists(*pl, *t, t->w1max, t->w2max);
+    if (same_windows(pl->adjm, pl->adjm64))
+      pl->adjm64 = pl->adjm;  // gather tables included
+    else if (e == hipSuccess && pl->adjm64.n_tiles1 > 0)
+      e = upload_gather_lists(*pl, pl->adjm64, pl->adjm64.w1max, pl->adjm64.w2max);
     pl->work_bytes = std::max(adjoint_work_bytes(*pl), adjoint_mma_work_bytes(*pl));
     unsigned char* w = nullptr;
     if (e == hipSuccess) e = dalloc(*pl, &w, pl->work_bytes);
